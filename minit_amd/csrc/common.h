@@ -51,6 +51,8 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef int int4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int uint4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int uint2_t __attribute__((ext_vector_type(2)));
+// 16 bytes on any 2-byte boundary: one 16-byte global access all the same
+typedef unsigned int uint4_any_t __attribute__((ext_vector_type(4), aligned(2)));
 typedef int int16_t_v __attribute__((ext_vector_type(16)));
 
 constexpr int kWave = 64;

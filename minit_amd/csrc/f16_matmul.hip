@@ -241,7 +241,7 @@ __global__ __launch_bounds__(512) void f16_gemv_nk_kernel(const half_t* __restri
     }
 }
 
-// Any K (no divisibility or alignment assumptions): one thread per output.
+// K below 8, which the vector loads of the other kernels do not fit: one thread per output.
 __global__ void f16_matmul_nk_generic_kernel(const half_t* __restrict__ a, const half_t* __restrict__ b,
                                              half_t* __restrict__ out, int M, int N, int K) {
     a += (size_t)blockIdx.y * M * K;  // blockIdx.y: the matrix of a batch
@@ -277,14 +277,19 @@ namespace mh {
 // f16_matmul_lds.hip
 bool f16_matmul_lds_supported(int M, int N, int K);
 int f16_matmul_lds_launch(hipStream_t stream, const void* a, const void* b, void* out, int batch, int M, int N, int K);
+// f16_matmul_tiled.hip
+bool f16_matmul_tiled_supported(int M, int N, int K);
+bool f16_matmul_tiled_preferred(int M, int N, int K);
+int f16_matmul_tiled_launch(hipStream_t stream, const void* a, const void* b, void* out, int batch, int M, int N, int K);
 }  // namespace mh
 
 using namespace mh;
 
-// The MFMA kernels for `batch` matrices (K a multiple of 32, every matrix on a 16-byte boundary): the weight
-// streamed through LDS in whole lines where that kernel serves the shape, operands straight from global
-// memory otherwise.  Kernel and tiling depend on M, N and K only.
+// The MFMA kernels for `batch` matrices (K a multiple of 32, every matrix on a 16-byte boundary): tiles of both
+// operands in LDS for many rows, the weight streamed through LDS in whole lines where that kernel serves the
+// shape, operands straight from global memory otherwise.  Kernel and tiling depend on M, N and K only.
 static int launch_dense_mfma(hipStream_t st, const void* a, const void* b, void* out, int batch, int M, int N, int K) {
+    if (f16_matmul_tiled_preferred(M, N, K)) return f16_matmul_tiled_launch(st, a, b, out, batch, M, N, K);
     if (f16_matmul_lds_supported(M, N, K) && (M + 63) / 64 <= 65535) return f16_matmul_lds_launch(st, a, b, out, batch, M, N, K);
     const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
     const int nt = mt == 1 ? 1 : 2;  // columns per wave: 16 or 32
@@ -316,6 +321,7 @@ extern "C" int mh_f16_matmul_nk(mh_stream_t stream, const void* a, const void* b
     MH_REQUIRE(a && b && out, "mh_f16_matmul_nk: null pointer");
     hipStream_t st = as_stream(stream);
     const bool fast = K > 0 && K % 32 == 0 && ((uintptr_t)a | (uintptr_t)b) % 16 == 0;
+    if (!fast && f16_matmul_tiled_supported(M, N, K)) return f16_matmul_tiled_launch(st, a, b, out, 1, M, N, K);
     if (!fast) {
         size_t blocks = ((size_t)M * N + 255) / 256;
         const size_t cap = (size_t)compute_units() * 16;
@@ -368,6 +374,7 @@ extern "C" int mh_f16_matmul_nk_batched(mh_stream_t stream, const void* a, const
     // every matrix of the batch must start on a 16-byte boundary for the vector loads
     const bool fast = K > 0 && K % 32 == 0 && ((uintptr_t)a | (uintptr_t)b) % 16 == 0 &&
                       ((size_t)M * K * 2) % 16 == 0 && ((size_t)N * K * 2) % 16 == 0;
+    if (!fast && f16_matmul_tiled_supported(M, N, K)) return f16_matmul_tiled_launch(st, a, b, out, batch, M, N, K);
     if (!fast) {
         size_t blocks = ((size_t)M * N + 255) / 256;
         const size_t cap = (size_t)compute_units() * 16;

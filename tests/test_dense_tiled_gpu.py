@@ -1,0 +1,32 @@
+"""The tiled dense fp16 product (csrc/f16_matmul_tiled.hip) where it can go wrong: lengths of K around its rounds of
+64 and its 16-byte pieces, rows that start on odd 2-byte boundaries, ragged tiles of every height, batches whose
+matrices lie back to back (what follows a row must not leak into it), against the float64 product."""
+import numpy as np
+import pytest
+
+from helpers import assert_fp16_close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("batch,m,n,k", [
+    (1, 1, 1, 8), (2, 5, 7, 9), (3, 33, 129, 63),          # shorter than a round: the remainder alone
+    (2, 32, 128, 65), (2, 31, 130, 71), (1, 64, 127, 127),  # one round and 1, 7, 63 elements
+    (2, 65, 129, 128), (3, 128, 256, 192), (1, 129, 5, 193),  # 128-row tiles, two and three rounds, odd rows
+    (2, 200, 300, 1001), (4, 257, 128, 1500), (2, 130, 128, 4096),  # the p v of a prompt
+    (1, 2100, 4200, 256), (1, 100, 24600, 512)])            # two tiles per CU; one block of rows
+def test_tiled_dense_product(hip, batch, m, n, k):
+    from minit_amd.hip.tensor import HIPTensor
+    rng = np.random.default_rng(m * 7 + k)
+    a = rng.normal(0, 1, size=(batch, m, k)).astype(np.float16)
+    b = rng.normal(0, 0.1, size=(batch, n, k)).astype(np.float16)
+    if batch > 1:   # a neighbour's infinities stay in its own rows
+        a[1, 0, 0] = np.inf
+    out = HIPTensor.allocate((batch, m, n), "float16")
+    da, db = HIPTensor.from_numpy(a), HIPTensor.from_numpy(b)
+    hip.call("mh_f16_matmul_nk_batched", None, da.data_ptr, db.data_ptr, out.data_ptr, batch, m, n, k)
+    got = out.numpy()
+    for i in range(batch):
+        rows = slice(1, None) if i == 1 else slice(None)
+        ref = a[i, rows].astype(np.float64) @ b[i].astype(np.float64).T
+        assert_fp16_close(got[i, rows], ref, what=f"matrix {i}")
