@@ -851,10 +851,10 @@ int gptq_gemm_wide_launch(hipStream_t stream, const void* x, const int32_t* qwei
 
 // gptq_gemm_tall.hip: blocks of 128 rows, weights dequantised in registers, K sliced over the waves
 bool gemm_tall_preferred(int M, int N, int K, int group_size, int bits, int epilogue);
-size_t gemm_tall_workspace_bytes(int M, int N, int K);
+size_t gemm_tall_workspace_bytes(int M, int N, int K, int bits);
 bool gemm_tall_silu_pairs_supported(int M, int N, int K, int group_size, int bits);
 int gptq_gemm_tall_launch(hipStream_t stream, const void* x, const int32_t* qweight, const int32_t* qzeros,
-                          const void* scales, void* out, int M, int N, int K, int group_size, void* workspace,
+                          const void* scales, void* out, int M, int N, int K, int group_size, int bits, void* workspace,
                           size_t workspace_bytes, const half_t* bias, int epilogue);
 
 struct GemmPlan {
@@ -1063,7 +1063,7 @@ static bool row_blocked(int M, int group_size) { return M > kSmallMaxM && use_sm
 size_t gemm_workspace_bytes(int M, int N, int K, int group_size, int bits) {
     // Up to kSmallMaxM rows a launch with an epilogue or the norm prologue takes the small-M or the
     // column-owner kernel where the plain product takes the 128-row-block kernel: the size covers all three.
-    const size_t tall = gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone) ? gemm_tall_workspace_bytes(M, N, K) : 0;
+    const size_t tall = gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone) ? gemm_tall_workspace_bytes(M, N, K, bits) : 0;
     if (M > kSmallMaxM && gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone)) return tall;
     if (gemm_wide_preferred(M, N, K, group_size, bits, kEpilogueNone)) return gemm_wide_workspace_bytes(M, N, K);
     if (row_blocked(M, group_size)) {
@@ -1190,10 +1190,10 @@ int gptq_gemm_launch(hipStream_t stream, const void* x, const int32_t* qweight, 
                     "(mh_gptq_matmul serves them with the per-element kernel)");
     // more than 64 rows: blocks of 128 rows, a packed word dequantised once per block
     if (fuse.ssq_in == nullptr && gemm_tall_preferred(M, N, K, group_size, bits, epilogue))
-        return gptq_gemm_tall_launch(stream, x, qweight, qzeros, scales, out, M, N, K, group_size, workspace,
+        return gptq_gemm_tall_launch(stream, x, qweight, qzeros, scales, out, M, N, K, group_size, bits, workspace,
                                      workspace_bytes, fuse.bias, kEpilogueNone);
     if (fuse.ssq_in == nullptr && epilogue == kEpilogueSiluPairs && gemm_tall_silu_pairs_supported(M, N, K, group_size, bits))
-        return gptq_gemm_tall_launch(stream, x, qweight, qzeros, scales, out, M, N, K, group_size, workspace,
+        return gptq_gemm_tall_launch(stream, x, qweight, qzeros, scales, out, M, N, K, group_size, bits, workspace,
                                      workspace_bytes, nullptr, kEpilogueSiluPairs);
     // many rows: the kernel that dequantises a weight tile once for 128 rows
     if (fuse.ssq_in == nullptr && gemm_wide_preferred(M, N, K, group_size, bits, epilogue))

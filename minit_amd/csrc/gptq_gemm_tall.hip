@@ -1,4 +1,4 @@
-// GPTQ w4a16 product for blocks of 128 (or 256) rows: weights dequantised in registers, straight into
+// GPTQ product (4 and 8 bit) for blocks of 128 (or 256) rows: weights dequantised in registers, straight into
 // the B operand of v_mfma_f32_16x16x32_f16, activations fetched by LDS-destination loads.
 //
 // Replaces the same reference pair as the other product kernels
@@ -13,11 +13,12 @@
 // of 64 k, 16 x 4 tiles and 256 accumulators per wave, 64 MFMAs per step.)  Lane (j, o) of a
 // wave holds columns 4j..4j+3 of the wave's 64 -- MFMA tile c takes column 4j + c -- and the
 // o-th eight k of the step: its four packed words are one 16-byte load, its four scales one
-// 8-byte load, its four zero points sit in one word.
+// 8-byte load, its four zero points sit in one word.  (8 bit: two 16-byte loads, the words of the octet's two
+// rows.)
 //
 // Per round every wave advances one step:
 //   * all global loads are issued from inline assembly and waited for by hand; one
-//     s_waitcnt vmcnt(14) per round covers everything the round consumes: the packed words and
+//     s_waitcnt vmcnt (14 outstanding at 4 bit and 128 rows) per round covers everything the round consumes: the packed words and
 //     constants of step r + 1 (requested four rounds ahead into a ring of four) and the
 //     activation stage of round r (requested three rounds ahead into one of four 32 KiB LDS
 //     buffers by buffer_load_dwordx4 ... lds: 128 rows x 256 bytes as two halves of 128-byte
@@ -28,15 +29,19 @@
 //     16-byte chunk per quarter wave) free of bank conflicts is applied to the global address);
 //   * one barrier;
 //   * the 32 MFMAs of step r, with the round's seven loads and the dequantisation of step r + 1
-//     (13 instructions per word = the bit-exact W of Dequantize, 4 to put the pairs back into k order, 4
-//     for the column's constants) placed between them one or two instructions at a time
-//     (kTallSchedule): two vector instructions per MFMA issue in its shadow, more cost 4.6 cycles each,
+//     (4 bit: 13 instructions per word = the bit-exact W of Dequantize, 4 to put the pairs back into k order, 4
+//     for the column's constants; 8 bit: 12 per two words, which come out in k order, and 3) placed between them one or two instructions at a time
+//     (TallSchedule): two vector instructions per MFMA issue in its shadow, more cost 4.6 cycles each,
 //     and one block of 17 behind every eighth MFMA left the matrix pipe idle.
 // At the end the waves' shares of K are added through LDS in a fixed order (the waves that meet exchange
 // halves of their accumulators, so that each ends up with its own share of the row tiles), the tile is
 // turned into row-major order in LDS and leaves as 16-byte row pieces: fp16 results (plus bias), with
 // kEpilogueSiluPairs silu(gate) * up of a tile made of 64 gate and the 64 matching up columns, or,
 // with K split over blockIdx.y, fp32 partial sums for splitk_finalize_kernel.
+//
+// 8-bit weights against the small-M kernel's 64-row blocks that served them before (us, now / before): 2048 x 4096 x
+// 28672 447 / 646, 2048 x 14336 x 4096 197 / 269, 1000 x 5120 x 15360 146 / 216, 128 x 4096 x 28672 36.9 / 57.0, 64 x
+// 5120 x 15360 25.0 / 33.7; 1.02-1.22 PFLOP/s at 2048 rows, as the 4-bit form.
 #include "gptq_common.h"
 
 #include <type_traits>
@@ -97,8 +102,12 @@ __device__ __forceinline__ void tall_load_to_lds_pair(uint32_t lds_addr, int vof
 // Everything but the newest NEWEST loads has arrived; the registers read next pass through the
 // wait, so that no use can be scheduled above it.
 template <int NEWEST>
-__device__ __forceinline__ void tall_wait(uint4_t& q, uint2_t& s, uint32_t& z) {
-    asm volatile("s_waitcnt vmcnt(%3)" : "+v"(q), "+v"(s), "+v"(z) : "n"(NEWEST) : "memory");
+__device__ __forceinline__ void tall_wait(uint4_t (&q)[1], uint2_t& s, uint32_t& z) {
+    asm volatile("s_waitcnt vmcnt(%3)" : "+v"(q[0]), "+v"(s), "+v"(z) : "n"(NEWEST) : "memory");
+}
+template <int NEWEST>
+__device__ __forceinline__ void tall_wait(uint4_t (&q)[2], uint2_t& s, uint32_t& z) {
+    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(q[0]), "+v"(q[1]), "+v"(s), "+v"(z) : "n"(NEWEST) : "memory");
 }
 
 // The 84 vector instructions that dequantise a step (21 per packed word: code = word * 21 + u, u as in
@@ -108,14 +117,34 @@ __device__ __forceinline__ void tall_wait(uint4_t& q, uint2_t& s, uint32_t& z) {
 // followed by an instruction of the next word that does not depend on it (its constants 0..3, shift 4 and
 // extractions 5..8; words alternate between two sets of temporaries); the re-ordering (17..20) of word 2 is
 // held back to pair with the subtractions of word 3, whose first two multiplications stay alone.
-constexpr int kTallUnits = 54;
-constexpr signed char kTallSchedule[kTallUnits][2] = {
-    {0, -1}, {1, -1}, {2, -1}, {3, -1}, {4, -1}, {5, -1}, {6, -1}, {7, -1}, {8, -1},
-    {9, 21}, {10, 22}, {11, 23}, {12, 24}, {13, 25}, {14, 26}, {15, 27}, {16, 28}, {29, -1},
-    {17, -1}, {18, -1}, {19, -1}, {20, -1}, {30, 42}, {31, 43}, {32, 44}, {33, 45}, {34, 46},
-    {35, 47}, {36, 48}, {37, 49}, {50, -1}, {38, -1}, {39, -1}, {40, -1}, {41, -1}, {51, 63},
-    {52, 64}, {53, 65}, {54, 66}, {55, 67}, {56, 68}, {57, 69}, {58, 70}, {71, -1}, {72, 59},
-    {73, 60}, {74, 61}, {75, 62}, {76, -1}, {77, -1}, {78, 80}, {79, 81}, {82, -1}, {83, -1},
+template <int BITS> struct TallSchedule;
+template <> struct TallSchedule<4> {
+    static constexpr int kPerColumn = 21;
+    static constexpr int kUnits = 54;
+    static constexpr signed char kUnit[kUnits][2] = {
+        {0, -1}, {1, -1}, {2, -1}, {3, -1}, {4, -1}, {5, -1}, {6, -1}, {7, -1}, {8, -1},
+        {9, 21}, {10, 22}, {11, 23}, {12, 24}, {13, 25}, {14, 26}, {15, 27}, {16, 28}, {29, -1},
+        {17, -1}, {18, -1}, {19, -1}, {20, -1}, {30, 42}, {31, 43}, {32, 44}, {33, 45}, {34, 46},
+        {35, 47}, {36, 48}, {37, 49}, {50, -1}, {38, -1}, {39, -1}, {40, -1}, {41, -1}, {51, 63},
+        {52, 64}, {53, 65}, {54, 66}, {55, 67}, {56, 68}, {57, 69}, {58, 70}, {71, -1}, {72, 59},
+        {73, 60}, {74, 61}, {75, 62}, {76, -1}, {77, -1}, {78, 80}, {79, 81}, {82, -1}, {83, -1},
+    };
+};
+// 8 bit: 15 instructions per column (code = column * 15 + u): a byte permutation builds two fp16 values 1024 + q in
+// k order straight from a word, so there is neither a shift nor a re-ordering and the two words of a column's eight k
+// cost what a 4-bit word costs less six.  u = 0..2 the column's constants, 3..6 the permutations, 7..10 the
+// subtractions, 11..14 the multiplications, which write the operand; the packed-fp16 ones (7..14) of a column are
+// followed by the others (0..6) of the next.
+template <> struct TallSchedule<8> {
+    static constexpr int kPerColumn = 15;
+    static constexpr int kUnits = 39;
+    static constexpr signed char kUnit[kUnits][2] = {
+        {0, -1}, {1, -1}, {2, -1}, {3, -1}, {4, -1}, {5, -1}, {6, -1},
+        {7, 15}, {8, 16}, {9, 17}, {10, 18}, {11, 19}, {12, 20}, {13, 21}, {14, -1},
+        {22, 30}, {23, 31}, {24, 32}, {25, 33}, {26, 34}, {27, 35}, {28, 36}, {29, -1},
+        {37, 45}, {38, 46}, {39, 47}, {40, 48}, {41, 49}, {42, 50}, {43, 51}, {44, -1},
+        {52, -1}, {53, -1}, {54, -1}, {55, -1}, {56, -1}, {57, -1}, {58, -1}, {59, -1},
+    };
 };
 
 // The A operands are read from LDS by hand as well: the compiler waits before the first use of every one
@@ -139,7 +168,7 @@ __device__ __forceinline__ void tall_lds_wait(half8_t* a) {
 // LDS allows them below eight row tiles) measured slower, 32 x 8192 x 57344 90.3 against 77.8 us and 64 x 8192 x
 // 10240 30.3 against 29.0 -- what holds the kernel back at few rows is its ~105 vector instructions per
 // round, not latency.
-template <int MT, int NS>
+template <int BITS, int MT, int NS>
 __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel(
     const half_t* __restrict__ x, const uint32_t* __restrict__ qweight, const uint32_t* __restrict__ qzeros,
     const half_t* __restrict__ scales, half_t* __restrict__ out, float* __restrict__ partial, int M, int N, int K,
@@ -151,7 +180,9 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
     constexpr int kHalfBytes = BM * 128;           // [row][64 k], chunks swizzled
     constexpr int kStageBytes = (RK / 64) * kHalfBytes;  // the halves of a round's k
     constexpr int PW = MT / 2;                     // 1 KiB pieces of a stage per wave
-    constexpr int LR = 3 + PW;                     // loads per wave and round
+    constexpr int WR = BITS / 4;                   // rows of packed words behind a lane's eight k
+    constexpr int LR = 2 + WR + PW;                // loads per wave and round
+    using Schedule = TallSchedule<BITS>;
     constexpr int kRegion = MT * 4096;             // a wave's accumulators in LDS
     static_assert(MT == 2 || MT == 4 || MT == 8 || MT == 16, "two, four, eight or sixteen row tiles");
     __shared__ __attribute__((aligned(1024))) int8_t smem[NS * kStageBytes];
@@ -176,9 +207,9 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
     // the descriptors live in fixed scalar registers; past the workgroup's last round their record count is
     // set to zero (one scalar instruction), and a load moves nothing and returns zeros
     int4_t x_rsrc = tall_rsrc(x, (uint32_t)((size_t)M * K * 2));
-    int4_t w_rsrc = tall_rsrc(qweight, (uint32_t)((size_t)(K / 8) * N * 4));
+    int4_t w_rsrc = tall_rsrc(qweight, (uint32_t)((size_t)(K / 8 * WR) * N * 4));
     int4_t s_rsrc = tall_rsrc(scales, (uint32_t)((size_t)(K / group_size) * N * 2));
-    int4_t z_rsrc = tall_rsrc(qzeros, (uint32_t)((size_t)(K / group_size) * (N / 8) * 4));
+    int4_t z_rsrc = tall_rsrc(qzeros, (uint32_t)((size_t)(K / group_size) * (N / 8 * WR) * 4));
     const int x_bytes = x_rsrc[2], w_bytes = w_rsrc[2], s_bytes = s_rsrc[2], z_bytes = z_rsrc[2];
 
     // ---- what a lane fetches per round
@@ -197,67 +228,69 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
     }
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(size_t)smem);
     const uint32_t lds_wave = lds0 + (uint32_t)(wave >> 2) * kHalfBytes + (uint32_t)((wave & 3) * PW) * 1024u;
-    const int w_off = ((k_wave / 8 + o) * N + col) * 4;
-    const int s_off = col * 2, z_off = (col >> 3) * 4;
-    const int z_shift = (j & 1) * 16;  // the lane's four zero points: nibbles 4 (j & 1) .. + 3 of the word
+    const int w_off = ((k_wave / 8 + o) * WR * N + col) * 4;
+    const int s_off = col * 2, z_off = (BITS == 4 ? col >> 3 : col >> 2) * 4;
+    // the lane's four zero points: nibbles 4 (j & 1) .. + 3 of the word, or its four bytes
+    const int z_shift = BITS == 4 ? (j & 1) * 16 : 0;
 
-    uint4_t rq[NS];   // packed words of steps r .. r + NS - 1
-    uint2_t rs[NS];   // their scales
-    uint32_t rz[NS];  // their zero-point words
+    uint4_t rq[NS][WR];  // packed words of steps r .. r + NS - 1
+    uint2_t rs[NS];      // their scales
+    uint32_t rz[NS];     // their zero-point words
     // group of the step whose loads are issued next / whose constants are built next
     int load_group = __builtin_amdgcn_readfirstlane(k_wave / group_size);
     int load_in_group = __builtin_amdgcn_readfirstlane(k_wave % group_size);
-    // The LR loads that go with step `step`, in their fixed order: piece 0 the packed words, 1 the scales,
-    // 2 the zero points (all into ring slot S), 3.. the wave's 1 KiB pieces of the activation stage of round
+    // The LR loads that go with step `step`, in their fixed order: pieces 0 .. WR - 1 the packed words, then the
+    // scales, the zero points (all into ring slot S) and the wave's 1 KiB pieces of the activation stage of round
     // step - 1 (into buffer (step - 1) % NS).  The main loop spreads the pieces over the round's MFMAs: issued
     // back to back by all eight waves right after the barrier they fill the vector memory queue, and the
     // waves stall in issue with the matrix pipes idle.
     auto issue_piece = [&](auto slot, auto piece, int step) {
         constexpr int S = decltype(slot)::value, I = decltype(piece)::value;
         const bool live = step < n_rounds;
-        if constexpr (I == 0) {
-            w_rsrc[2] = live ? w_bytes : 0;
-            tall_load_b128_stream(rq[S], w_off, w_rsrc, step * (RK / 2) * N);
+        if constexpr (I < WR) {
+            if constexpr (I == 0) w_rsrc[2] = live ? w_bytes : 0;
+            tall_load_b128_stream(rq[S][I], w_off, w_rsrc, (step * (RK / 8) * WR + I) * N * 4);
         }
-        if constexpr (I == 1) {
+        if constexpr (I == WR) {
             s_rsrc[2] = live ? s_bytes : 0;
             tall_load_b64(rs[S], s_off, s_rsrc, __builtin_amdgcn_readfirstlane(load_group * N * 2));
         }
-        if constexpr (I == 2) {
+        if constexpr (I == WR + 1) {
             z_rsrc[2] = live ? z_bytes : 0;
-            tall_load_b32(rz[S], z_off, z_rsrc, __builtin_amdgcn_readfirstlane(load_group * (N / 8) * 4));
+            tall_load_b32(rz[S], z_off, z_rsrc, __builtin_amdgcn_readfirstlane(load_group * (N / 8 * WR) * 4));
             load_in_group += RK;
             while (load_in_group >= group_size) {
                 load_in_group -= group_size;
                 ++load_group;
             }
         }
-        if constexpr (I >= 3) {
+        if constexpr (I >= WR + 2) {
+            constexpr int X = I - WR - 2;
             const int stage = step - 1;
             const uint32_t base = lds_wave + (uint32_t)((S + NS - 1) % NS) * kStageBytes;
-            if constexpr (I == 3) x_rsrc[2] = stage < n_rounds ? x_bytes : 0;
+            if constexpr (X == 0) x_rsrc[2] = stage < n_rounds ? x_bytes : 0;
             if constexpr (PW == 1)
                 tall_load_to_lds(base, x_off[0], x_rsrc, stage * (RK * 2));
-            else if constexpr ((I - 3) % 2 == 0)
-                tall_load_to_lds_pair(base + (uint32_t)(I - 3) * 1024u, x_off[I - 3], x_off[I - 2], x_rsrc, stage * (RK * 2));
+            else if constexpr (X % 2 == 0)
+                tall_load_to_lds_pair(base + (uint32_t)X * 1024u, x_off[X], x_off[X + 1], x_rsrc, stage * (RK * 2));
         }
     };
     auto issue = [&](auto slot, int step, bool with_stage) {
-        issue_piece(slot, std::integral_constant<int, 0>{}, step);
-        issue_piece(slot, std::integral_constant<int, 1>{}, step);
-        issue_piece(slot, std::integral_constant<int, 2>{}, step);
-        if (with_stage) tall_static_for<3, LR>([&](auto piece) { issue_piece(slot, piece, step); });
+        tall_static_for<0, WR + 2>([&](auto piece) { issue_piece(slot, piece, step); });
+        if (with_stage) tall_static_for<WR + 2, LR>([&](auto piece) { issue_piece(slot, piece, step); });
     };
 
     DequantRegs regs;
-    regs.init(4);
+    regs.init(BITS);
+    uint32_t high_bytes = 0x64646464u;  // the high bytes of fp16 1024 + q
+    if (BITS == 8) asm volatile("" : "+v"(high_bytes));
     ColumnConst cc[4];
     // The constants of make_column_const() without conversions, four instructions per column: for a zero
     // point z <= 15 the fp16 values 1024 + (z + 1) and 64 + (z + 1) are 0x6400 + (z + 1) and 0x5400 +
     // 16 (z + 1) as bit patterns (one unit, one sixteenth per mantissa step), so both pairs are one
     // 24-bit multiply-add of z each.
     auto make_const = [&](int c, const uint2_t& s, uint32_t z) {
-        const uint32_t zc = (z >> (z_shift + 4 * c)) & 0xFu;
+        const uint32_t zc = (z >> (z_shift + BITS * c)) & Packing<BITS>::kMask;
         const uint32_t sw = s[c >> 1];
         cc[c].scale = as_half2((c & 1) ? __builtin_amdgcn_perm(sw, sw, 0x07060706u) : __builtin_amdgcn_perm(sw, sw, 0x05040504u));
         cc[c].zero_lo = as_half2(zc * 0x00010001u + 0x64016401u);
@@ -267,14 +300,20 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
 #pragma unroll
         for (int c = 0; c < 4; ++c) make_const(c, s, z);
     };
-    // one packed word -> the B operand of MFMA tile c: k0 .. k7 of column 4j + c
-    auto dequant_piece = [&](half8_t& b, uint32_t word, int c) {
+    // the packed words of column 4j + c -> the B operand of MFMA tile c: k0 .. k7
+    auto dequant_piece = [&](half8_t& b, const uint4_t (&q)[WR], int c) {
         half2_t w[4];
-        dequant_word<4>(word, cc[c], regs, w);
-        b = half8_t{w[0][0], w[1][0], w[2][0], w[3][0], w[0][1], w[1][1], w[2][1], w[3][1]};
+        if constexpr (BITS == 4) {
+            dequant_word<4>(q[0][c], cc[c], regs, w);
+            b = half8_t{w[0][0], w[1][0], w[2][0], w[3][0], w[0][1], w[1][1], w[2][1], w[3][1]};
+        } else {
+            dequant_word<8>(q[0][c], cc[c], regs, w);
+            dequant_word<8>(q[WR - 1][c], cc[c], regs, w + 2);
+            b = half8_t{w[0][0], w[1][0], w[0][1], w[1][1], w[2][0], w[3][0], w[2][1], w[3][1]};
+        }
     };
-    // The same arithmetic (dequant_word<4>, the constants above) one instruction at a time, 21 per packed
-    // word: a wave issues one instruction of any kind in about five cycles, so whatever stands between two
+    // The same arithmetic (dequant_word, the constants above) one instruction at a time, 21 per packed
+    // 4-bit word (15 per two 8-bit words): a wave issues one instruction of any kind in about five cycles, so whatever stands between two
     // of its MFMAs beyond two or three instructions leaves the matrix pipe waiting.  Instruction u of word c
     // reads packed word `word` and the step's scales and zero points; the last four write the B operand
     // registers.  Dependent instructions are at least three apart (next to each other they cost a wait
@@ -283,17 +322,31 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
     ColumnConst kc[2];
     uint32_t zc[2], q8[2];
     half2_t wq[2][4];
-    auto dequant_op = [&](auto op_c, uint4_t& bw, const uint4_t& q4, int c, const uint2_t& sc, uint32_t z) {
-        constexpr int u = decltype(op_c)::value % 21, e = (decltype(op_c)::value / 21) & 1;
+    auto dequant_op = [&](auto op_c, uint4_t& bw, const uint4_t (&q4)[WR], int c, const uint2_t& sc, uint32_t z) {
+        constexpr int u = decltype(op_c)::value % Schedule::kPerColumn, e = (decltype(op_c)::value / Schedule::kPerColumn) & 1;
         const half2_t sixteenth = half2_t{(half_t)0.0625f, (half_t)0.0625f};
-        const uint32_t sw = sc[c >> 1], word = q4[c];
+        const uint32_t sw = sc[c >> 1], word = q4[0][c];
         auto pin = [&](auto& out) { asm volatile("" : "+v"(out)); };
-        if constexpr (u == 0) { zc[e] = (z >> (z_shift + 4 * c)) & 0xFu; pin(zc[e]); }
+        if constexpr (u == 0) { zc[e] = (z >> (z_shift + BITS * c)) & Packing<BITS>::kMask; pin(zc[e]); }
         if constexpr (u == 1) {
             kc[e].scale = as_half2((c & 1) ? __builtin_amdgcn_perm(sw, sw, 0x07060706u) : __builtin_amdgcn_perm(sw, sw, 0x05040504u));
             pin(kc[e].scale);
         }
         if constexpr (u == 2) { kc[e].zero_lo = as_half2(__umul24(zc[e], 0x00010001u) + 0x64016401u); pin(kc[e].zero_lo); }
+        if constexpr (BITS == 8) {
+            if constexpr (u >= 3 && u <= 6) {
+                constexpr int i = u - 3;  // k 2i and 2i + 1: bytes 0, 1 or 2, 3 of the first or second word
+                wq[e][i] = as_half2(__builtin_amdgcn_perm(q4[i >> 1 < WR ? i >> 1 : 0][c], high_bytes, (i & 1) ? 0x00070006u : 0x00050004u));
+                pin(wq[e][i]);
+            }
+            if constexpr (u >= 7 && u <= 10) { wq[e][u - 7] = wq[e][u - 7] - kc[e].zero_lo; pin(wq[e][u - 7]); }
+            if constexpr (u >= 11) {
+                uint32_t r = __builtin_bit_cast(uint32_t, wq[e][u - 11] * kc[e].scale);
+                pin(r);
+                bw[u - 11] = r;
+            }
+            return;
+        }
         if constexpr (u == 3) { kc[e].zero_hi = as_half2(__umul24(zc[e], 0x00100010u) + 0x54105410u); pin(kc[e].zero_hi); }
         if constexpr (u == 4) { q8[e] = word >> 8; pin(q8[e]); }
         if constexpr (u >= 5 && u <= 8) {
@@ -349,7 +402,7 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         half8_t b0;
-        dequant_piece(b0, rq[0][c], c);
+        dequant_piece(b0, rq[0], c);
         bw[0][c] = __builtin_bit_cast(uint4_t, b0);
     }
 
@@ -369,7 +422,7 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
             tall_lds_read<(decltype(rt)::value % kOwn) * 2048>(a[decltype(rt)::value], a_stage + (uint32_t)a_group_off[decltype(rt)::value / kOwn]);
         });
         __builtin_amdgcn_sched_barrier(0);
-        // 4 MT MFMAs; after MFMA m its share of the 54 units that dequantise step r + 1 and, after
+        // 4 MT MFMAs; after MFMA m its share of the units that dequantise step r + 1 and, after
         // every fourth (second at four row tiles, every one at two), one of the round's loads
         tall_static_for<0, 4 * MT>([&](auto mfma) {
             constexpr int m = decltype(mfma)::value;
@@ -380,11 +433,12 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
             __builtin_amdgcn_sched_barrier(0);
             constexpr int load = MT >= 8 ? (m % 4 == 3 ? m / 4 : -1) : MT == 4 ? (m % 2 == 1 ? m / 2 : -1) : m;
             if constexpr (load >= 0 && load < LR) issue_piece(slot, std::integral_constant<int, load>{}, r + NS);
-            tall_static_for<m * kTallUnits / (4 * MT), (m + 1) * kTallUnits / (4 * MT)>([&](auto unit) {
-                constexpr int first = kTallSchedule[decltype(unit)::value][0], second = kTallSchedule[decltype(unit)::value][1];
-                dequant_op(std::integral_constant<int, first>{}, bw[P ^ 1][first / 21], rq[S1], first / 21, rs[S1], rz[S1]);
+            tall_static_for<m * Schedule::kUnits / (4 * MT), (m + 1) * Schedule::kUnits / (4 * MT)>([&](auto unit) {
+                constexpr int first = Schedule::kUnit[decltype(unit)::value][0], second = Schedule::kUnit[decltype(unit)::value][1];
+                constexpr int kPer = Schedule::kPerColumn;
+                dequant_op(std::integral_constant<int, first>{}, bw[P ^ 1][first / kPer], rq[S1], first / kPer, rs[S1], rz[S1]);
                 if constexpr (second >= 0)
-                    dequant_op(std::integral_constant<int, second>{}, bw[P ^ 1][second / 21], rq[S1], second / 21, rs[S1], rz[S1]);
+                    dequant_op(std::integral_constant<int, second>{}, bw[P ^ 1][second / kPer], rq[S1], second / kPer, rs[S1], rz[S1]);
             });
             __builtin_amdgcn_sched_barrier(0);
         });
@@ -523,7 +577,7 @@ static int tall_mt16_mode() {
     return v;
 }
 
-static TallPlan plan_tall(int M, int N, int K) {
+static TallPlan plan_tall(int M, int N, int K, int bits) {
     TallPlan p;
     p.mt = M <= 32 ? 2 : M <= 64 ? 4 : 8;
     p.tiles_n = (N + kTallBN - 1) / kTallBN;
@@ -557,8 +611,8 @@ static TallPlan plan_tall(int M, int N, int K) {
         if (split > most) split = most;
         return split < 1 ? 1L : split;
     };
-    long split = capped(16);
-    const long relaxed = capped(8);
+    long split = capped(64 / bits);
+    const long relaxed = capped(32 / bits);
     if (((rounds + relaxed - 1) / relaxed) * 4 <= ((rounds + split - 1) / split) * 3) split = relaxed;
     p.rounds_per_block = (int)((rounds + split - 1) / split);
     p.split_k = (rounds + p.rounds_per_block - 1) / p.rounds_per_block;
@@ -584,8 +638,21 @@ static int tall_min_m_env() {
 // nearly everywhere (8192 x 8192 12.3 against 15.7).
 static bool tall_two_row_tiles_preferred(int M, int N, int K) {
     if (M < 17 || M > 32) return false;
-    const TallPlan p = plan_tall(M, N, K);
+    const TallPlan p = plan_tall(M, N, K, 4);
     return (long)p.tiles_n * p.split_k * 8 >= (long)compute_units() * 5 && p.rounds_per_block <= 40;
+}
+
+// 8-bit weights of 9 to 32 rows: a packed word costs 7.5 vector instructions per eight k and column here against 13 in
+// the small-M kernel, and at these rows the weight stream dominates both.  Measured against the small-M and
+// column-owner kernels (us, this kernel / before): at 16 rows 5120 x 15360 18.9 / 21.5, 5120 x 27392 27.3 / 28.6,
+// 13696 x 5120 18.3 / 19.6, 14336 x 4096 15.7 / 23.0, 28672 x 8192 41.2 / 43.9, 8192 x 8192 17.5 / 17.7; at 32 rows
+// 20.5 / 27.5, 29.4 / 33.1, 19.6 / 22.3, 16.9 / 24.3, 43.6 / 51.2, 18.2 / 21.6, 4096 x 4096 11.8 / 12.3.  It loses where a
+// launch is all fixed costs (4096 x 4096 at 16 rows 10.5 / 9.5, 2048 x 1024 at 32 rows 8.7 / 7.3) and where there are
+// more column tiles than CUs (8192 x 57344 at 16 / 32 rows 79.8 / 73.1, 86.5 / 78.7).  Up to eight rows the gain is
+// within a few per cent either way and the other kernels' epilogues stay in one launch.
+static bool tall_8bit_preferred(int M, int N, int K) {
+    if (M < 9 || M > 32 || (N + kTallBN - 1) / kTallBN > compute_units()) return false;
+    return (size_t)N * K >= (M <= 16 ? (size_t)24 << 20 : (size_t)16 << 20);
 }
 
 // Measured on one box against what served these shapes before (the small-M kernel's 64-row blocks up to
@@ -606,41 +673,46 @@ static bool tall_two_row_tiles_preferred(int M, int N, int K) {
 bool gemm_tall_preferred(int M, int N, int K, int group_size, int bits, int epilogue) {
     static const char* off = getenv("MH_GEMM_NO_TALL");
     if (off && *off && atoi(off)) return false;
-    if (!(bits == 4 && epilogue == kEpilogueNone && K % kTallRoundK == 0 && K >= 4 * kTallRoundK &&
+    if (!(epilogue == kEpilogueNone && K % kTallRoundK == 0 && K >= 4 * kTallRoundK &&
           group_size % 32 == 0 && K % group_size == 0 && N % 8 == 0 && (size_t)M * K * 2 < ((size_t)1 << 31) &&
-          (size_t)K * N / 2 < ((size_t)1 << 31)))
+          (size_t)K * N * bits / 8 < ((size_t)1 << 31)))
         return false;
     if (tall_min_m_env() > 0) return M >= tall_min_m_env();
-    return M >= 33 || tall_two_row_tiles_preferred(M, N, K);
+    return M >= 33 || (bits == 4 ? tall_two_row_tiles_preferred(M, N, K) : tall_8bit_preferred(M, N, K));
 }
 
-size_t gemm_tall_workspace_bytes(int M, int N, int K) {
-    const TallPlan p = plan_tall(M, N, K);
+size_t gemm_tall_workspace_bytes(int M, int N, int K, int bits) {
+    const TallPlan p = plan_tall(M, N, K, bits);
     return p.split_k > 1 ? kTileCounterBytes + (size_t)p.split_k * M * N * sizeof(float) : 0;
 }
 
 // kEpilogueSiluPairs in the kernel's own store: an unsplit plan, whole blocks of 128 + 128 columns.
 bool gemm_tall_silu_pairs_supported(int M, int N, int K, int group_size, int bits) {
-    return gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone) && N % 256 == 0 && plan_tall(M, N, K).split_k == 1;
+    return gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone) && N % 256 == 0 && plan_tall(M, N, K, bits).split_k == 1;
 }
 
 int gptq_gemm_tall_launch(hipStream_t stream, const void* x, const int32_t* qweight, const int32_t* qzeros,
-                          const void* scales, void* out, int M, int N, int K, int group_size, void* workspace,
+                          const void* scales, void* out, int M, int N, int K, int group_size, int bits, void* workspace,
                           size_t workspace_bytes, const half_t* bias, int epilogue) {
-    const TallPlan p = plan_tall(M, N, K);
+    const TallPlan p = plan_tall(M, N, K, bits);
     if (epilogue != kEpilogueNone && (epilogue != kEpilogueSiluPairs || p.split_k != 1 || N % 256 != 0 || bias))
         return fail(MH_ERR_INVALID, "gptq gemm (128-row blocks): epilogue %d is not served for M=%d N=%d K=%d", epilogue, M, N, K);
-    const size_t need = gemm_tall_workspace_bytes(M, N, K);
+    const size_t need = gemm_tall_workspace_bytes(M, N, K, bits);
     if (need != 0 && (workspace == nullptr || workspace_bytes < need))
         return fail(MH_ERR_WORKSPACE, "mh_gptq_gemm: workspace of %zu bytes required, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
     float* partial = need ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kTileCounterBytes) : nullptr;
-#define MH_LAUNCH_TALL(MT)                                                                                            \
-    hipLaunchKernelGGL((gptq_gemm_tall_kernel<MT, 4>), dim3(p.tiles_n, p.split_k, p.row_blocks),                     \
+#define MH_LAUNCH_TALL_BITS(BITS, MT)                                                                                 \
+    hipLaunchKernelGGL((gptq_gemm_tall_kernel<BITS, MT, 4>), dim3(p.tiles_n, p.split_k, p.row_blocks),               \
                        dim3(tall_k_shares(MT) * 128), 0,                                                              \
                        stream, (const half_t*)x, (const uint32_t*)qweight, (const uint32_t*)qzeros,                  \
                        (const half_t*)scales, (half_t*)out, partial, M, N, K, group_size, p.rounds_per_block,        \
                        p.split_k, bias, epilogue)
+#define MH_LAUNCH_TALL(MT)                                                                                            \
+    if (bits == 4)                                                                                                    \
+        MH_LAUNCH_TALL_BITS(4, MT);                                                                                   \
+    else                                                                                                              \
+        MH_LAUNCH_TALL_BITS(8, MT)
     switch (p.mt) {
         case 2: MH_LAUNCH_TALL(2); break;
         case 4: MH_LAUNCH_TALL(4); break;
@@ -648,6 +720,7 @@ int gptq_gemm_tall_launch(hipStream_t stream, const void* x, const int32_t* qwei
         default: MH_LAUNCH_TALL(8); break;
     }
 #undef MH_LAUNCH_TALL
+#undef MH_LAUNCH_TALL_BITS
     MH_CHECK_LAUNCH();
     if (p.split_k > 1) {
         SmallFuse fuse;
