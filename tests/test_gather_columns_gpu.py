@@ -1,0 +1,19 @@
+"""mh_gather_columns on its kernels: four columns per thread (16-bit, whole 16-byte pieces, few elements), a row parked
+in LDS (more, up to 64 KiB) and one element per thread; index entries outside the row are clamped into it."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols,dtype", [(1, 8, np.float16), (3, 4104, np.float16), (300, 4112, np.float16), (1100, 952, np.float16), (33, 32768, np.float16),
+                                             (2, 32776, np.float16), (5, 12, np.float16), (4, 2048, np.float32)])
+def test_gather_columns(hip, rows, cols, dtype):
+    from minit_amd.hip.tensor import HIPTensor
+    rng = np.random.default_rng(cols)
+    x = rng.normal(size=(rows, cols)).astype(dtype)
+    index = rng.permutation(cols).astype(np.int32)
+    index[0], index[-1] = -5, cols + 7
+    dx, di, out = HIPTensor.from_numpy(x), HIPTensor.from_numpy(index), HIPTensor.allocate((rows, cols), x.dtype.name)
+    hip.call("mh_gather_columns", None, dx.data_ptr, di.data_ptr, out.data_ptr, rows, cols, 0 if dtype == np.float16 else 2)
+    np.testing.assert_array_equal(out.numpy(), x[:, np.clip(index, 0, cols - 1)])
