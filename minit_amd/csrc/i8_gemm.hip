@@ -511,6 +511,10 @@ __global__ __launch_bounds__(256) void i8_transpose_kernel(const int8_t* __restr
 bool i8_gemm_dma_supported(int M, int N, int K);
 int i8_gemm_dma_launch(hipStream_t stream, const int8_t* a, const int8_t* w, const float* a_scale,
                        const float* w_scale, void* out_f16, int32_t* acc_i32, int M, int N, int K);
+// i8_gemm_rows.hip: small tiles, K split over the waves of a workgroup
+bool i8_gemm_rows_preferred(int M, int N, int K);
+int i8_gemm_rows_launch(hipStream_t stream, const int8_t* a, const int8_t* w, const float* a_scale,
+                        const float* w_scale, void* out_f16, int32_t* acc_i32, int M, int N, int K);
 
 }  // namespace mh
 
@@ -528,6 +532,8 @@ int mh_i8_gemm(mh_stream_t stream, const int8_t* a, const int8_t* w, const float
     MH_REQUIRE(!out_f16 || (a_scale && w_scale), "mh_i8_gemm: scales required for the fp16 output");
     MH_REQUIRE(((uintptr_t)a | (uintptr_t)w | (uintptr_t)acc_i32) % 16 == 0 && (uintptr_t)out_f16 % 16 == 0,
                "mh_i8_gemm: operands and outputs must be 16-byte aligned");
+    if (i8_gemm_rows_preferred(M, N, K))
+        return i8_gemm_rows_launch(as_stream(stream), a, w, a_scale, w_scale, out_f16, acc_i32, M, N, K);
     const int tiles_m = (M + kI8BM - 1) / kI8BM, tiles_n = (N + kI8BN - 1) / kI8BN;
     const int tiles = tiles_m * tiles_n;
     const int group_m = tiles_m < 8 ? tiles_m : 8;
