@@ -230,59 +230,65 @@ __global__ __launch_bounds__(1024) void argmax_advance_kernel(const half_t* __re
 // alternate chunks and are merged through LDS; splits are merged by the last
 // block to arrive.
 
-template <int G, int D, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
-    const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
-    const int32_t* __restrict__ positions, half_t* __restrict__ out, float* partial, unsigned* counters,
-    int kvh, int max_seq, float scale, int splits) {
+constexpr int kAttnPitch = 72;   // halfs per row of the P tile in LDS (64 + padding)
+
+// What one wave holds of the G heads of a (row, KV head) pair, and its walk over 64-position chunks.
+template <int G, int D>
+struct AttnWave {
     static_assert(D == 128 && G <= 16, "head size 128, at most 16 query heads per KV head");
-    constexpr int PP = 72;  // halfs per row of the P tile in LDS (64 + padding)
-    const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int i16 = lane & 15, kq = lane >> 4;
-    // Chunks of 64 positions (one tile of the V cache) are dealt round robin, first over the
-    // blocks of a (row, KV head) pair and then over their waves: chunk c belongs to block
-    // c % splits, wave (c / splits) % WAVES.  The deal does not depend on the length, so a
-    // wave requests its first chunk before the position has arrived, and no wave holds more
-    // than one chunk over the others.
-    const int stride = splits * WAVES * 64;
-    const int c_first = (split + wave * splits) * 64;
-    const int t1 = min(max(positions[b], 0), max_seq - 1) + 1;  // the new token has been appended
-
-    __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * PP];
-    __shared__ float m_s[WAVES][16], l_s[WAVES][16];
-    __shared__ float acc_s[WAVES][G][D];
-
-    // A operand of S = Q K^T: row = head i16, k = dims s*32 + kq*8 .. +8
     uint4 qf[4];
-    {
-        const half_t* qp = q + (((size_t)b * kvh + g) * G + min(i16, G - 1)) * D + kq * 8;
+    uint4 kf[4][4], vf[8][2];
+    // rows of every accumulator tile held by this lane: heads kq*4 + r; acc[dt][r] is dim dt*16 + i16
+    float m_run[4], l_run[4];
+    float4_t acc[8];
+
+    __device__ __forceinline__ void reset() {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            m_run[r] = -INFINITY;
+            l_run[r] = 0.f;
+        }
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) acc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+    }
+
+    // A operand of S = Q K^T: row = head i16, k = dims s*32 + kq*8 .. +8 (q: the pair's G heads)
+    __device__ __forceinline__ void load_q(const half_t* q, int i16, int kq) {
+        const half_t* qp = q + (size_t)min(i16, G - 1) * D + kq * 8;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             qf[s] = *reinterpret_cast<const uint4*>(qp + s * 32);
             if (i16 >= G) qf[s] = make_uint4(0, 0, 0, 0);
         }
     }
-    const half_t* kbase = k_cache + ((size_t)b * kvh + g) * max_seq * D;
-    const half_t* vbase = vt_cache + ((size_t)b * kvh + g) * D * max_seq;
-
-    // rows of every accumulator tile held by this lane: heads kq*4 + r
-    float m_run[4], l_run[4];
-    float4_t acc[8];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        m_run[r] = -INFINITY;
-        l_run[r] = 0.f;
-    }
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) acc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
 
     // all loads of a chunk are issued before the first use (refilling K after Q K^T and V
     // after P V for the wave's next chunk, so that loads stay in flight under the arithmetic,
-    // measured no faster at batch 1 and 32 and slower at 8).  Rows and tiles are clamped to
-    // the cache, not to the length: what lies past the end is masked below.
-    uint4 kf[4][4], vf[8][2];
-    auto load_chunk = [&](int c0) {
+    // measured no faster at batch 1 and 32 and slower at 8).  k, v: the chunk's 64 rows of K and
+    // its tile of V, the same address for the whole wave; what lies past a row's end is masked in
+    // step().
+    __device__ __forceinline__ void load_chunk(const half_t* k, const half_t* v, int i16, int kq) {
+        const unsigned lane_k = (i16 * D + kq * 8) * sizeof(half_t), lane_v = (i16 * kVTile + kq * 8) * sizeof(half_t);
+        auto at = [](const half_t* base, int halfs, unsigned lane) {
+            return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base + halfs) + lane);
+        };
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) kf[pt][s] = at(k, pt * 16 * D + s * 32, lane_k);
+        __builtin_amdgcn_sched_barrier(0);   // K first: Q K^T starts while V is on its way
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) vf[dt][ks] = at(v, dt * 16 * kVTile + ks * 32, lane_v);
+    }
+
+    // The same with an address per lane, which the compiler mixes into the chunk's arithmetic: K as soon as its
+    // registers are free, V behind Q K^T.  Four waves of a block (one per SIMD) are 3 to 7 % faster with it
+    // (8 rows x 8 heads x 2112 16.6 us against 17.8 with the form above), eight waves 4 % slower
+    // (32 x 8 x 2048 40.7 against 39.0).  Rows and tiles are clamped to the cache.
+    __device__ __forceinline__ void load_chunk_by_lane(const half_t* kbase, const half_t* vbase, int c0, int max_seq,
+                                                       int i16, int kq) {
 #pragma unroll
         for (int pt = 0; pt < 4; ++pt) {
             const int row = min(c0 + pt * 16 + i16, max_seq - 1);
@@ -297,17 +303,11 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
             for (int dt = 0; dt < 8; ++dt)
                 vf[dt][ks] = *reinterpret_cast<const uint4*>(vbase + vt_offset(dt * 16 + i16, p0));
         }
-    };
-    load_chunk(c_first);
-    // Two waves share a SIMD when a block has eight, and the older one wins every arbitration: the
-    // priority of a wave falls with the share of its chunks it has behind it, so that the four
-    // younger waves are not left to walk their last chunks alone.
-    const int n_chunks = t1 > c_first ? (t1 - c_first + stride - 1) / stride : 0;
-    int chunk_no = 0;
-    for (int c0 = c_first; c0 < t1;) {
-        if constexpr (WAVES > 4) {
-            set_priority_by_progress(chunk_no++, n_chunks);
-        }
+    }
+
+    // The loaded chunk of positions c0 .. c0 + 63, of which those below t1 (at least one) count;
+    // p_s: the wave's own P tile in LDS.
+    __device__ __forceinline__ void step(half_t* p_s, int c0, int t1, float scale, int i16, int kq) {
         // S tile pt: rows = heads kq*4 + r, column = position c0 + pt*16 + i16
         float4_t sc[4];
 #pragma unroll
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
             for (int pt = 0; pt < 4; ++pt) {
                 const float pv = expf(sc[pt][r] - m_new);  // exp(-inf) = 0 for masked positions
                 sum += pv;
-                p_s[wave][(kq * 4 + r) * PP + pt * 16 + i16] = (half_t)pv;
+                p_s[(kq * 4 + r) * kAttnPitch + pt * 16 + i16] = (half_t)pv;
             }
 #pragma unroll
             for (int off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off, 64);
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
         uint4 pa[2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
-            pa[ks] = *reinterpret_cast<const uint4*>(&p_s[wave][i16 * PP + ks * 32 + kq * 8]);
+            pa[ks] = *reinterpret_cast<const uint4*>(&p_s[i16 * kAttnPitch + ks * 32 + kq * 8]);
         if (c0 + 64 > t1) {
             // positions past the end carry weight 0 but whatever the cache holds there
             // (possibly not finite): clear them
@@ -380,47 +380,149 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();  // p_s is rewritten by the next chunk
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        c0 += stride;
-        if (c0 < t1) load_chunk(c0);
     }
+};
 
-    // acc[dt][r] is head kq*4 + r, dim dt*16 + i16
+constexpr int kAttnRecord = 128 + 4;   // floats of one head's record in the workspace: acc[D], m, l, two unused
+
+// The waves of a block meet: their sums (zero chunks: maximum -inf) added into one, per head and four dims.
+template <int G, int D, int WAVES>
+struct AttnMerge {
+    static constexpr int kItems = G * D / 4;   // threads that merge: (head, four dims) each
+    float m[WAVES][16], l[WAVES][16];
+    float acc[WAVES][G][D];
+
+    __device__ __forceinline__ void put(const AttnWave<G, D>& w, int wave, int i16, int kq) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int h = kq * 4 + r;
-        if (h < G) {
+        for (int r = 0; r < 4; ++r) {
+            const int h = kq * 4 + r;
+            if (h < G) {
 #pragma unroll
-            for (int dt = 0; dt < 8; ++dt) acc_s[wave][h][dt * 16 + i16] = acc[dt][r];
-            if (i16 == 0) {
-                m_s[wave][h] = m_run[r];
-                l_s[wave][h] = l_run[r];
+                for (int dt = 0; dt < 8; ++dt) acc[wave][h][dt * 16 + i16] = w.acc[dt][r];
+                if (i16 == 0) {
+                    m[wave][h] = w.m_run[r];
+                    l[wave][h] = w.l_run[r];
+                }
             }
         }
     }
-    __syncthreads();
-
-    // merge the waves: thread -> (head, four dims)
-    constexpr int REC = D + 4;        // floats per (head, split) record: acc[D], m, l, two unused
-    constexpr int ITEMS = G * D / 4;  // <= 256
-    const size_t head0 = ((size_t)b * kvh + g) * G;
-    const int h = tid / (D / 4), d = tid % (D / 4) * 4;
-    if (tid < ITEMS) {
-        float mm = m_s[0][h];
+    __device__ __forceinline__ float4_t fold(int h, int d, float& mm, float& ll) const {
+        mm = m[0][h];
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) mm = fmaxf(mm, m_s[w][h]);
-        float ll = 0.f;
+        for (int w = 1; w < WAVES; ++w) mm = fmaxf(mm, m[w][h]);
+        ll = 0.f;
         float4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-            const float f = (m_s[w][h] == -INFINITY) ? 0.f : expf(m_s[w][h] - mm);
-            ll += l_s[w][h] * f;
-            a += *reinterpret_cast<const float4_t*>(&acc_s[w][h][d]) * f;
+            const float f = (m[w][h] == -INFINITY) ? 0.f : expf(m[w][h] - mm);
+            ll += l[w][h] * f;
+            a += *reinterpret_cast<const float4_t*>(&acc[w][h][d]) * f;
         }
-        if (splits == 1) {
-            const half4_t o = {(half_t)(a[0] / ll), (half_t)(a[1] / ll), (half_t)(a[2] / ll), (half_t)(a[3] / ll)};
-            *reinterpret_cast<half4_t*>(out + (head0 + h) * D + d) = o;
+        return a;
+    }
+};
+
+__device__ __forceinline__ void attn_store(half_t* out, float4_t a, float ll) {
+    const half4_t o = {(half_t)(a[0] / ll), (half_t)(a[1] / ll), (half_t)(a[2] / ll), (half_t)(a[3] / ll)};
+    *reinterpret_cast<half4_t*>(out) = o;
+}
+
+// Last block of a pair: every thread folds the records of its four output elements with the
+// running-maximum recurrence, reading each record's maximum, sum and partial values itself: the loads
+// of up to BATCH records are independent and in flight together, so the merge costs one memory round
+// trip.  record(i) is the address of record i of `count`.
+template <int BATCH, typename Record>
+__device__ __forceinline__ void attn_fold_records(half_t* out, int d, int count, Record record) {
+    float mm = -INFINITY, ll = 0.f;
+    float4_t a = {0.f, 0.f, 0.f, 0.f};
+    for (int sp0 = 0; sp0 < count; sp0 += BATCH) {
+        float ms[BATCH], ls[BATCH];
+        float4_t as[BATCH];
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const float* ps = record(min(sp0 + u, count - 1));
+            as[u] = load_agent4(ps + d);
+            ms[u] = load_agent(ps + 128);
+            ls[u] = load_agent(ps + 128 + 1);
+        }
+        wait_agent_loads(as);
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            if (sp0 + u < count && ms[u] != -INFINITY) {
+                const float m_new = fmaxf(mm, ms[u]);
+                const float f_old = expf(mm - m_new);  // exp(-inf) = 0 for the first record folded in
+                const float f = expf(ms[u] - m_new);
+                ll = ll * f_old + ls[u] * f;
+                a = a * f_old + as[u] * f;
+                mm = m_new;
+            }
+        }
+    }
+    attn_store(out, a, ll);
+}
+
+template <int G, int D, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
+    const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
+    const int32_t* __restrict__ positions, half_t* __restrict__ out, float* partial, unsigned* counters,
+    int kvh, int max_seq, float scale, int splits) {
+    const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = WAVES > 4 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+    const int i16 = lane & 15, kq = lane >> 4;
+    // Chunks of 64 positions (one tile of the V cache) are dealt round robin, first over the
+    // blocks of a (row, KV head) pair and then over their waves: chunk c belongs to block
+    // c % splits, wave (c / splits) % WAVES.  The deal does not depend on the length, so a
+    // wave requests its first chunk before the position has arrived, and no wave holds more
+    // than one chunk over the others.
+    const int stride = splits * WAVES * 64;
+    const int c_first = (split + wave * splits) * 64;
+    const int t1 = min(max(positions[b], 0), max_seq - 1) + 1;  // the new token has been appended
+
+    __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * kAttnPitch];
+    __shared__ __attribute__((aligned(16))) AttnMerge<G, D, WAVES> merge;
+
+    const size_t pair = (size_t)b * kvh + g;
+    const half_t* kbase = k_cache + pair * max_seq * D;
+    const half_t* vbase = vt_cache + pair * D * max_seq;
+    AttnWave<G, D> w;
+    w.load_q(q + pair * G * D, i16, kq);
+    w.reset();
+    auto load = [&](int c0) {
+        if constexpr (WAVES > 4) {
+            const size_t at = (size_t)min(c0, max_seq - 64) * D;   // a chunk past the cache is not used: any will do
+            w.load_chunk(kbase + at, vbase + at, i16, kq);
         } else {
-            float* pp = partial + ((head0 + h) * splits + split) * REC;
+            w.load_chunk_by_lane(kbase, vbase, c0, max_seq, i16, kq);
+        }
+    };
+    load(c_first);
+    // Two waves share a SIMD when a block has eight, and the older one wins every arbitration: the
+    // priority of a wave falls with the share of its chunks it has behind it, so that the four
+    // younger waves are not left to walk their last chunks alone.
+    const int n_chunks = t1 > c_first ? (t1 - c_first + stride - 1) / stride : 0;
+    int chunk_no = 0;
+    for (int c0 = c_first; c0 < t1;) {
+        if constexpr (WAVES > 4) {
+            set_priority_by_progress(chunk_no++, n_chunks);
+        }
+        w.step(p_s[wave], c0, t1, scale, i16, kq);
+        c0 += stride;
+        if (c0 < t1) load(c0);
+    }
+    merge.put(w, wave, i16, kq);
+    __syncthreads();
+
+    // merge the waves: thread -> (head, four dims)
+    const size_t head0 = pair * G;
+    const int h = tid / (D / 4), d = tid % (D / 4) * 4;
+    if (tid < merge.kItems) {
+        float mm, ll;
+        const float4_t a = merge.fold(h, d, mm, ll);
+        if (splits == 1) {
+            attn_store(out + (head0 + h) * D + d, a, ll);
+        } else {
+            float* pp = partial + ((head0 + h) * splits + split) * kAttnRecord;
             store_agent4(pp + d, a);
             if (d == 0) store_agent4(pp + D, float4_t{mm, ll, 0.f, 0.f});
         }
@@ -428,42 +530,123 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
     if (splits == 1) return;
 
     __shared__ int is_last;
-    if (!arrive_and_check_last(counters + (size_t)b * kvh + g, (unsigned)splits, &is_last)) return;
-    // Last block: merge the splits.  Every thread folds the splits of its four
-    // output elements with the running-maximum recurrence, reading each split's
-    // maximum, sum and partial values itself: the loads of up to 16 splits are
-    // independent and in flight together, so the merge costs one memory round
-    // trip.
-    constexpr int BATCH = 16;
-    if (tid < ITEMS) {
-        const float* pp = partial + (head0 + h) * splits * REC;
-        float mm = -INFINITY, ll = 0.f;
-        float4_t a = {0.f, 0.f, 0.f, 0.f};
-        for (int sp0 = 0; sp0 < splits; sp0 += BATCH) {
-            float ms[BATCH], ls[BATCH];
-            float4_t as[BATCH];
+    if (!arrive_and_check_last(counters + pair, (unsigned)splits, &is_last)) return;
+    if (tid < merge.kItems) {
+        const float* pp = partial + (head0 + h) * splits * kAttnRecord;
+        attn_fold_records<16>(out + (head0 + h) * D + d, d, splits, [&](int i) { return pp + (size_t)i * kAttnRecord; });
+    }
+}
+
+// The same for rows of different lengths: the chunks of all pairs stand in one line (pair after pair),
+// and every block takes an equal piece of it, whatever pairs it holds.
+// Bound by the caches' bytes; a block per (row, KV head) pair leaves the chip to the longest rows at the
+// end.  32 rows of a 8192-entry cache, lengths from an eighth of it to all: 150 -> 131 us (5.2 TB/s; 180 us =
+// 6.0 TB/s with all rows full).  What a block needs to know, it works out from the lengths by itself: every
+// wave holds them one row per lane and adds them up across the lanes.  A pair that one block holds whole is
+// finished there; of a pair that several share, each leaves a record and the last to arrive adds them up.
+// At the end of a pair a wave requests its first chunk of the next one before the waves meet.
+template <int G, int D, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 2) void attn_decode_balanced_kernel(
+    const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
+    const int32_t* __restrict__ positions, half_t* __restrict__ out, float* partial, unsigned* counters, int batch,
+    int kvh, int max_seq, float scale) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15, kq = lane >> 4;
+    __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * kAttnPitch];
+    __shared__ __attribute__((aligned(16))) AttnMerge<G, D, WAVES> merge;
+    __shared__ int is_last;
+
+    // lane r: row r (batch <= 64): its length, and where its chunks end in the line
+    const int len = lane < batch ? min(max(positions[lane], 0), max_seq - 1) + 1 : 0;
+    const int mine = (len + 63) / 64 * kvh;
+    int upto = mine;
 #pragma unroll
-            for (int u = 0; u < BATCH; ++u) {
-                const float* ps = pp + (size_t)min(sp0 + u, splits - 1) * REC;
-                as[u] = load_agent4(ps + d);
-                ms[u] = load_agent(ps + D);
-                ls[u] = load_agent(ps + D + 1);
-            }
-            wait_agent_loads(as);
-#pragma unroll
-            for (int u = 0; u < BATCH; ++u) {
-                if (sp0 + u < splits && ms[u] != -INFINITY) {
-                    const float m_new = fmaxf(mm, ms[u]);
-                    const float f_old = expf(mm - m_new);  // exp(-inf) = 0 for the first split folded in
-                    const float f = expf(ms[u] - m_new);
-                    ll = ll * f_old + ls[u] * f;
-                    a = a * f_old + as[u] * f;
-                    mm = m_new;
-                }
+    for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(upto, off, 64);
+        if (lane >= off) upto += v;
+    }
+    const int total = __builtin_amdgcn_readlane(upto, 63);
+    // a block takes one chunk per wave or more: where the rows are short, blocks are left without work
+    const int blocks = min((int)gridDim.x, (total + WAVES - 1) / WAVES);
+    if ((int)blockIdx.x >= blocks) return;
+    auto first_of = [&](int block) { return (int)((long long)total * block / blocks); };
+    auto block_of = [&](int chunk) { return (int)((((long long)chunk + 1) * blocks - 1) / total); };
+    const int begin = first_of(blockIdx.x), end = first_of(blockIdx.x + 1);
+
+    // piece of a pair in the block's part of the line
+    struct Piece {
+        int pair, start, stop, t1;   // pair, the line's chunks start .. stop of it, its length
+    };
+    auto piece_at = [&](int chunk) {
+        Piece p;
+        const int b = __popcll(__ballot(upto <= chunk));
+        const int n = __builtin_amdgcn_readlane(mine, b) / kvh;
+        const int row0 = __builtin_amdgcn_readlane(upto, b) - n * kvh;
+        const int g = (chunk - row0) / n;
+        p.pair = b * kvh + g;
+        p.start = row0 + g * n;
+        p.stop = p.start + n;
+        p.t1 = __builtin_amdgcn_readlane(len, b);
+        return p;
+    };
+    AttnWave<G, D> w;
+    // chunk c of the line belongs to wave (c - begin) % WAVES: over the whole block no wave holds more
+    // than one chunk over the others
+    int c = begin + wave;
+    Piece p = piece_at(begin);
+    auto request = [&] {   // the wave's next chunk, if it lies in piece p
+        if (c >= min(end, p.stop)) return;
+        const size_t at = ((size_t)p.pair * max_seq + (size_t)(c - p.start) * 64) * D;
+        w.load_chunk(k_cache + at, vt_cache + at, i16, kq);
+    };
+    w.load_q(q + (size_t)p.pair * G * D, i16, kq);
+    request();
+    w.reset();
+    const int h = tid / (D / 4), d = tid % (D / 4) * 4;
+    const int n_chunks = (end - begin - wave + WAVES - 1) / WAVES;
+    int chunk_no = 0;
+    for (;;) {
+        const int stop = min(end, p.stop);
+        if (c < stop) {
+            if constexpr (WAVES > 4) set_priority_by_progress(chunk_no++, n_chunks);
+            w.step(p_s[wave], (c - p.start) * 64, p.t1, scale, i16, kq);
+            c += WAVES;
+        }
+        const Piece now = p;
+        if (c >= stop && stop < end) {
+            // what the next pair needs is requested before this one's sums meet
+            p = piece_at(stop);
+            w.load_q(q + (size_t)p.pair * G * D, i16, kq);
+        }
+        request();
+        if (c < stop) continue;
+        merge.put(w, wave, i16, kq);
+        w.reset();
+        __syncthreads();
+        const int first = block_of(now.start), last = block_of(now.stop - 1);
+        half_t* op = out + ((size_t)now.pair * G + h) * D + d;
+        if (tid < G * D / 4) {
+            float mm, ll;
+            const float4_t a = merge.fold(h, d, mm, ll);
+            if (first == last) {
+                attn_store(op, a, ll);
+            } else {
+                // two records per block: of the pair it begins with, and of the one it ends in
+                float* pp = partial + (((size_t)blockIdx.x * 2 + (now.start > begin)) * G + h) * kAttnRecord;
+                store_agent4(pp + d, a);
+                if (d == 0) store_agent4(pp + D, float4_t{mm, ll, 0.f, 0.f});
             }
         }
-        const half4_t o = {(half_t)(a[0] / ll), (half_t)(a[1] / ll), (half_t)(a[2] / ll), (half_t)(a[3] / ll)};
-        *reinterpret_cast<half4_t*>(out + (head0 + h) * D + d) = o;
+        if (first != last && arrive_and_check_last(counters + now.pair, (unsigned)(last - first + 1), &is_last) &&
+            tid < G * D / 4) {
+            const int slot = now.start > first_of(first);
+            // (four records at a time: the next pair's chunk is in registers already)
+            attn_fold_records<4>(op, d, last - first + 1, [&](int i) {
+                return partial + (((size_t)(first + i) * 2 + (i == 0 ? slot : 0)) * G + h) * kAttnRecord;
+            });
+        }
+        if (stop >= end) break;
+        __syncthreads();   // the sums' LDS is written again
     }
 }
 
@@ -524,25 +707,55 @@ static int attn_splits(int n_kv_heads, int max_seq, int batch) {
 }
 static int attn_splits(const Llama& m, int batch) { return attn_splits(m.cfg.n_kv_heads, m.cfg.max_seq, batch); }
 
+// Whether the blocks share the chunks of all rows evenly (attn_decode_balanced_kernel) instead of taking one
+// row's each.  The lengths are on the device, so the line is drawn by what the cache could hold, in chunks
+// per block.  The walk costs 3 to 6 us more than a block of its own (lengths read first, sums meeting
+// across blocks), and wins back what the longest row keeps the other blocks waiting.  Measured with lengths
+// from an eighth of the cache to all of it / from half / all equal, this kernel against the even deal, us:
+// 48 rows x 4 heads x 4096 (48 chunks) 52 / 60 / 76 against 67 / 69 / 75; 32 x 8 x 8192 (128) 131 / 147 / 181
+// against 150 / 162 / 180; below it 32 x 8 x 2048 (32) 38 / 48 / 51 against 39 / 44 / 49.  Where the even deal
+// has to meet across blocks as well (splits > 1) the line is lower: 8 x 8 x 8192 (32) 35 / 46 / 53 against
+// 43 / 50 / 55, 16 x 8 x 2048 (16) 21 / 29 / 32 against 25 / 28 / 30; below it 8 x 8 x 2112 (8) 19 / 21 / 20
+// against 19 / 20 / 21, 4 x 8 x 2048 (4) 18 / 18 / 15 against 10 / 12 / 13.
+static bool attn_balanced(int n_kv_heads, int max_seq, int batch) {
+    if (batch < 2 || batch > 64) return false;   // a lane per row holds its length
+    const long long chunks = (long long)batch * n_kv_heads * (max_seq / kVTile);
+    return chunks >= (long long)compute_units() * (attn_splits(n_kv_heads, max_seq, batch) > 1 ? 16 : 48);
+}
+static size_t attn_record_bytes(int batch, int n_q_heads, int n_kv_heads, int max_seq, bool balanced) {
+    const size_t heads = balanced ? (size_t)2 * compute_units() * (n_q_heads / n_kv_heads)
+                                  : (size_t)batch * n_q_heads * attn_splits(n_kv_heads, max_seq, batch);
+    return align_up(heads * kAttnRecord * sizeof(float));
+}
+// Records of whichever kernel the shape runs; never less than the even deal needs.
+static size_t attn_record_bytes(int batch, int n_q_heads, int n_kv_heads, int max_seq) {
+    const size_t even = attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq, false);
+    if (!attn_balanced(n_kv_heads, max_seq, batch)) return even;
+    const size_t balanced = attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq, true);
+    return balanced > even ? balanced : even;
+}
+
 // Workspace of a stand-alone attention call: arrival counters (one per row and KV
 // head, zero between calls), then the per-split records.
 static size_t attn_counter_bytes(int batch, int n_kv_heads) { return align_up((size_t)batch * n_kv_heads * sizeof(unsigned)); }
-static size_t attn_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int head_dim, int max_seq) {
-    return attn_counter_bytes(batch, n_kv_heads) +
-           align_up((size_t)batch * n_q_heads * attn_splits(n_kv_heads, max_seq, batch) * (head_dim + 4) * sizeof(float));
+static size_t attn_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int max_seq) {
+    return attn_counter_bytes(batch, n_kv_heads) + attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq);
 }
 
 template <int G>
 static void launch_attn_raw(hipStream_t st, const half_t* q, const half_t* k_cache, const half_t* vt_cache,
                             const int32_t* positions, half_t* out, float* partial, unsigned* counters, int batch,
-                            int n_kv_heads, int max_seq, int splits) {
-    if (splits == 1)
+                            int n_kv_heads, int max_seq, int splits, bool balanced) {
+    const float scale = 1.0f / sqrtf(128.f);
+    if (balanced)
+        hipLaunchKernelGGL((attn_decode_balanced_kernel<G, 128, 8>), dim3(compute_units()), dim3(512), 0, st, q, k_cache,
+                           vt_cache, positions, out, partial, counters, batch, n_kv_heads, max_seq, scale);
+    else if (splits == 1)
         hipLaunchKernelGGL((attn_decode_kernel<G, 128, 8>), dim3(1, n_kv_heads, batch), dim3(512), 0, st, q, k_cache,
-                           vt_cache, positions, out, partial, counters, n_kv_heads, max_seq, 1.0f / sqrtf(128.f), 1);
+                           vt_cache, positions, out, partial, counters, n_kv_heads, max_seq, scale, 1);
     else
         hipLaunchKernelGGL((attn_decode_kernel<G, 128, 4>), dim3(splits, n_kv_heads, batch), dim3(256), 0, st, q,
-                           k_cache, vt_cache, positions, out, partial, counters, n_kv_heads, max_seq,
-                           1.0f / sqrtf(128.f), splits);
+                           k_cache, vt_cache, positions, out, partial, counters, n_kv_heads, max_seq, scale, splits);
 }
 
 static Scratch carve(const Llama& m, int batch, char* base) {
@@ -582,7 +795,7 @@ static Scratch carve(const Llama& m, int batch, char* base) {
         if ((size_t)c.ffn > widest) widest = (size_t)c.ffn;
         s.gathered = (half_t*)take((size_t)batch * widest * 2);
     }
-    s.attn_partial = (float*)take((size_t)batch * c.n_q_heads * attn_splits(m, batch) * (c.head_dim + 4) * 4);
+    s.attn_partial = (float*)take(attn_record_bytes(batch, c.n_q_heads, c.n_kv_heads, c.max_seq));
     s.ssq_a = (float*)take((size_t)batch * ((c.hidden + 31) / 32) * 4);
     s.ssq_b = (float*)take((size_t)batch * ((c.hidden + 31) / 32) * 4);
     s.pos_base = (int32_t*)take((size_t)batch * sizeof(int32_t));
@@ -595,7 +808,8 @@ static void launch_attn(hipStream_t st, const Llama& m, const Scratch& s, const 
                         const int32_t* positions, int batch, int splits) {
     const mh_llama_config& c = m.cfg;
     launch_attn_raw<G>(st, s.q, (const half_t*)L.k_cache, (const half_t*)L.v_cache, positions, s.attn, s.attn_partial,
-                       s.attn_counters, batch, c.n_kv_heads, c.max_seq, splits);
+                       s.attn_counters, batch, c.n_kv_heads, c.max_seq, splits,
+                       attn_balanced(c.n_kv_heads, c.max_seq, batch));
 }
 
 }  // namespace mh
@@ -606,7 +820,7 @@ extern "C" {
 
 size_t mh_attn_decode_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int head_dim, int max_seq) {
     if (batch <= 0 || n_q_heads <= 0 || n_kv_heads <= 0 || head_dim != 128 || max_seq <= 0) return 0;
-    return attn_workspace_bytes(batch, n_q_heads, n_kv_heads, head_dim, max_seq);
+    return attn_workspace_bytes(batch, n_q_heads, n_kv_heads, max_seq);
 }
 
 int mh_attn_decode(mh_stream_t stream, const void* q, const void* k_cache, const void* vt_cache,
@@ -623,7 +837,10 @@ int mh_attn_decode(mh_stream_t stream, const void* q, const void* k_cache, const
     MH_REQUIRE(max_seq >= kVTile && max_seq % kVTile == 0, "mh_attn_decode: max_seq must be a multiple of 64, got %d", max_seq);
     MH_REQUIRE(((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)vt_cache | (uintptr_t)out) % 16 == 0,
                "mh_attn_decode: operands must be 16-byte aligned");
-    const size_t need = attn_workspace_bytes(batch, n_q_heads, n_kv_heads, head_dim, max_seq);
+    // a workspace that holds the even deal's records alone gets the even deal
+    const size_t need = attn_counter_bytes(batch, n_kv_heads) + attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq, false);
+    const bool balanced = attn_balanced(n_kv_heads, max_seq, batch) &&
+                          workspace_bytes >= attn_workspace_bytes(batch, n_q_heads, n_kv_heads, max_seq);
     if (workspace == nullptr || workspace_bytes < need)
         return fail(MH_ERR_WORKSPACE, "mh_attn_decode: workspace of %zu bytes required, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
@@ -634,7 +851,7 @@ int mh_attn_decode(mh_stream_t stream, const void* q, const void* k_cache, const
     hipStream_t st = as_stream(stream);
 #define MH_ATTN(G)                                                                                                 \
     launch_attn_raw<G>(st, (const half_t*)q, (const half_t*)k_cache, (const half_t*)vt_cache, positions, (half_t*)out, \
-                       partial, counters, batch, n_kv_heads, max_seq, splits)
+                       partial, counters, batch, n_kv_heads, max_seq, splits, balanced)
     switch (g) {
         case 1: MH_ATTN(1); break;
         case 2: MH_ATTN(2); break;
