@@ -29,7 +29,7 @@ def lookup_implementation_from_types(tys: Tuple[Type, ...]) -> Callable:
 
 
 def dispatch(*args: Object):
-    arg_types = tuple(arg.type() for arg in args)
+    arg_types = tuple([arg.type() for arg in args])
     try:
         func = DISPATCH_CACHE[arg_types]
     except KeyError:

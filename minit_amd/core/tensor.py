@@ -18,6 +18,10 @@ class Tensor(Object):
     def device(self) -> str:
         raise NotImplementedError()
 
+    def dims(self) -> Tuple[int, ...]:
+        """The shape as plain ints."""
+        return tuple(dim.item() for dim in self.shape)
+
     def type(self):
         return type(self)
 

@@ -7,28 +7,35 @@ from ..core.tensor import Tensor
 from ..operator import BatchMatrixMultiply, MatrixMultiply
 
 
+def _dims(x) -> tuple:
+    return x.dims() if isinstance(x, Tensor) else tuple(d.item() for d in x.shape)
+
+
 def matrix_multiply(x: Tensor, y: Tensor) -> Tensor:
-    assert len(y.shape) == 2
+    assert len(_dims(y)) == 2
+    dims = _dims(x)
     lead = None
-    if len(x.shape) > 2:
-        lead = tuple(d.item() for d in x.shape[:-1])
+    if len(dims) > 2:
+        lead = dims[:-1]
         m = 1
         for d in lead:
             m *= d
-        x = x.reshape((m, x.shape[-1].item()))
+        x = x.reshape((m, dims[-1]))
     (z,) = dispatch(MatrixMultiply(), x, y)
     if lead is not None:
-        z = z.reshape((*lead, z.shape[-1].item()))
+        z = z.reshape((*lead, _dims(z)[-1]))
     return z
 
 
 def batch_matrix_multiply(x: Tensor, y: Tensor) -> Tensor:
-    assert len(x.shape) > 2 and len(y.shape) > 2
-    lead = tuple(d.item() for d in x.shape[:-2])
+    xd, yd = _dims(x), _dims(y)
+    assert len(xd) > 2 and len(yd) > 2
+    lead = xd[:-2]
     batch = 1
     for d in lead:
         batch *= d
-    x = x.reshape((batch, x.shape[-2].item(), x.shape[-1].item()))
-    y = y.reshape((batch, y.shape[-2].item(), y.shape[-1].item()))
+    x = x.reshape((batch, xd[-2], xd[-1]))
+    y = y.reshape((batch, yd[-2], yd[-1]))
     (z,) = dispatch(BatchMatrixMultiply(), x, y)
-    return z.reshape((*lead, z.shape[-2].item(), z.shape[-1].item()))
+    zd = _dims(z)
+    return z.reshape((*lead, zd[-2], zd[-1]))

@@ -8,52 +8,95 @@ blocks go to a small size-keyed free list so a steady-state loop does not call
 """
 import ctypes
 import threading
-from typing import Dict, List
+from collections import OrderedDict
+from typing import List
 
 from .. import lib
 
-_POOL: Dict[int, List[int]] = {}
+# Free blocks by their size, the sizes used last at the end.  What does not fit under the limit any more
+# makes room by giving back the sizes that have gone unused for longest: a pool that keeps the first 4 GiB it
+# sees sends every later size through hipMalloc and hipFree (attention over 32 heads of 1977 tokens after
+# other lengths: 14.2 ms a pass, of which the kernels take 0.3).
+_POOL: "OrderedDict[int, List[int]]" = OrderedDict()
 _POOL_BYTES = 0
 _POOL_LIMIT = 4 << 30
+# Reentrant: a tensor may die (and release its block) while the lock is held.
+_POOL_LOCK = threading.RLock()
 
 
 def _round(size: int) -> int:
-    return max(256, (size + 255) // 256 * 256)
+    """Block size for ``size`` bytes: multiples of 256, above 1 MiB eighths of a power of two, so that lengths
+    close to each other share blocks (a prompt of another length costs a hipMalloc per block otherwise);
+    exact again above 1 GiB, where an eighth is no longer small change."""
+    if size <= 256:
+        return 256
+    if 1 << 20 < size <= 1 << 30:
+        step = 1 << ((size - 1).bit_length() - 4)
+        return (size + step - 1) // step * step
+    return (size + 255) // 256 * 256
+
+
+def _malloc(size: int) -> int:
+    ptr = ctypes.c_void_p()
+    lib.call("mh_malloc", ctypes.byref(ptr), size)
+    return ptr.value
 
 
 def allocate(size: int) -> int:
+    """A block of at least ``size`` bytes; ``release(ptr, size)`` gives it back."""
     global _POOL_BYTES
     size = _round(size)
-    bucket = _POOL.get(size)
-    if bucket:
-        _POOL_BYTES -= size
-        return bucket.pop()
-    ptr = ctypes.c_void_p()
+    with _POOL_LOCK:
+        bucket = _POOL.get(size)
+        if bucket:
+            ptr = bucket.pop()
+            _POOL_BYTES -= size
+            return ptr
     try:
-        lib.call("mh_malloc", ctypes.byref(ptr), size)
+        return _malloc(size)
     except lib.HipError:
         empty_cache()
-        lib.call("mh_malloc", ctypes.byref(ptr), size)
-    return ptr.value
+        return _malloc(size)
 
 
 def release(ptr: int, size: int) -> None:
     global _POOL_BYTES
     size = _round(size)
-    if _POOL_BYTES + size <= _POOL_LIMIT:
-        _POOL.setdefault(size, []).append(ptr)
+    with _POOL_LOCK:
+        if size > _POOL_LIMIT:
+            lib.call("mh_free", ptr)
+            return
+        if _POOL_BYTES + size > _POOL_LIMIT:
+            _make_room(size)
+        bucket = _POOL.get(size)
+        if bucket is None:
+            bucket = _POOL[size] = []
+        else:
+            _POOL.move_to_end(size)
+        bucket.append(ptr)
         _POOL_BYTES += size
-    else:
+
+
+def _make_room(size: int) -> None:
+    global _POOL_BYTES
+    while _POOL and _POOL_BYTES + size > _POOL_LIMIT:
+        oldest, bucket = next(iter(_POOL.items()))
+        if not bucket:
+            del _POOL[oldest]
+            continue
+        ptr = bucket.pop()
+        _POOL_BYTES -= oldest
         lib.call("mh_free", ptr)
 
 
 def empty_cache() -> None:
     global _POOL_BYTES
-    for bucket in _POOL.values():
-        for ptr in bucket:
-            lib.call("mh_free", ptr)
-    _POOL.clear()
-    _POOL_BYTES = 0
+    with _POOL_LOCK:
+        while _POOL:
+            size, bucket = _POOL.popitem()
+            _POOL_BYTES -= size * len(bucket)
+            for ptr in bucket:
+                lib.call("mh_free", ptr)
 
 
 def synchronize(stream=None) -> None:

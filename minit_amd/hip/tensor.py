@@ -9,7 +9,7 @@ from typing import Optional, Tuple
 
 import numpy
 
-from ..core.dtype import dtype_info
+from ..core.dtype import DATA_TYPES, dtype_info
 from ..core.scalar import ScalarTensor
 from ..core.tensor import Tensor
 from . import memory
@@ -24,9 +24,10 @@ _NUMPY_DTYPES = {
 
 
 def _nbytes(shape: Tuple[int, ...], dtype: str) -> int:
-    size = dtype_info(dtype).size_in_bytes
+    size = DATA_TYPES[dtype].size_in_bytes
     for dim in shape:
-        assert isinstance(dim, int), f"shape entries must be int, got {type(dim)}"
+        if dim.__class__ is not int:
+            assert isinstance(dim, int), f"shape entries must be int, got {type(dim)}"
         size *= dim
     return size
 
@@ -43,6 +44,9 @@ class HIPTensor(Tensor):
     @property
     def shape(self) -> Tuple[Tensor, ...]:
         return tuple(ScalarTensor(dim, (), "int32") for dim in self._shape)
+
+    def dims(self) -> Tuple[int, ...]:
+        return self._shape
 
     @property
     def dtype(self) -> str:
@@ -61,18 +65,19 @@ class HIPTensor(Tensor):
 
     @property
     def data_ptr(self) -> int:
-        return self.memory._pointer
+        memory = self._memory
+        return (memory if memory is not None else self.memory)._pointer
 
     @staticmethod
     def allocate(shape: Tuple[int, ...], dtype: str) -> "HIPTensor":
-        result = HIPTensor(tuple(shape), dtype)
-        result._memory = HIPMemory(_nbytes(tuple(shape), dtype))
+        result = HIPTensor(shape, dtype)
+        result._memory = HIPMemory(_nbytes(result._shape, dtype))
         return result
 
     @staticmethod
     def wrap(shape: Tuple[int, ...], dtype: str, memory: HIPMemory) -> "HIPTensor":
-        assert memory._size == _nbytes(tuple(shape), dtype), "wrap: size mismatch"
-        result = HIPTensor(tuple(shape), dtype)
+        result = HIPTensor(shape, dtype)
+        assert memory._size == _nbytes(result._shape, dtype), "wrap: size mismatch"
         result._memory = memory
         return result
 

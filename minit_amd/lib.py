@@ -120,13 +120,16 @@ def last_error() -> str:
     return cdll().mh_last_error().decode(errors="replace")
 
 
+_functions = {}   # name -> bound function of the loaded library
+
+
 def call(name: str, *args):
     """Calls ``name`` and raises :class:`HipError` on a non-zero status."""
-    fn = getattr(cdll(), name)
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(cdll(), name)
     rc = fn(*args)
-    if name in _NOT_STATUS:
-        return rc
-    if rc != 0:
+    if rc and name not in _NOT_STATUS:
         raise HipError(f"{name} failed ({rc}): {last_error()}")
     return rc
 

@@ -67,6 +67,9 @@ class QuantizedTensor(Tensor):
     def shape(self):
         return (ScalarTensor(self.in_features, (), "int32"), ScalarTensor(self.out_features, (), "int32"))
 
+    def dims(self):
+        return (self.in_features, self.out_features)
+
     @property
     def dtype(self):
         return f"quint{self.bits}"

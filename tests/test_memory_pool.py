@@ -1,0 +1,57 @@
+"""The free list behind the tensors: bounded, the sizes used last kept, close sizes sharing blocks."""
+import pytest
+
+from minit_amd.hip import memory
+
+
+@pytest.fixture
+def device(monkeypatch):
+    """mh_malloc / mh_free on a host that counts: live pointers and their sizes."""
+    live, calls = {}, []
+
+    def call(name, *args):
+        calls.append(name)
+        if name == "mh_malloc":
+            pointer = 0x1000 * len(calls)
+            args[0]._obj.value = pointer
+            live[pointer] = args[1]
+        elif name == "mh_free":
+            del live[args[0]]   # a block given back twice is an error
+        return 0
+
+    monkeypatch.setattr(memory.lib, "call", call)
+    monkeypatch.setattr(memory, "_POOL", type(memory._POOL)())
+    monkeypatch.setattr(memory, "_POOL_BYTES", 0)
+    return live, calls
+
+
+@pytest.mark.parametrize("size", [0, 1, 256, 257, 1 << 20, (1 << 20) + 1, 3 << 20, (1 << 28) - 5, (1 << 28) + 5,
+                                  1 << 30, (1 << 30) + 1])
+def test_block_sizes(size):
+    block = memory._round(size)
+    assert block >= max(size, 256) and block % 256 == 0
+    assert memory._round(block) == block                 # release finds the block allocate gave
+    assert block - size <= max(256, size // 8 if 1 << 20 < size <= 1 << 30 else 0)
+
+
+def test_sizes_used_last_stay(device):
+    live, calls = device
+    block = 256 << 20
+    old = [memory.allocate(block) for _ in range(14)]
+    for p in old:
+        memory.release(p, block)
+    new_size = 500 << 20
+    for _ in range(3):   # the pool is nearly full of another size: the second pass on has its blocks
+        pair = [memory.allocate(new_size) for _ in range(2)]
+        for p in pair:
+            memory.release(p, new_size)
+    assert calls.count("mh_malloc") == 16
+    assert memory._POOL_BYTES == sum(live.values()) <= memory._POOL_LIMIT
+    memory.empty_cache()
+    assert not live and memory._POOL_BYTES == 0
+
+
+def test_blocks_above_the_limit_are_given_back(device):
+    live, calls = device
+    memory.release(memory.allocate(5 << 30), 5 << 30)
+    assert not live and memory._POOL_BYTES == 0
