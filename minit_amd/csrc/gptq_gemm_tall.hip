@@ -44,6 +44,7 @@
 // 5120 x 15360 25.0 / 33.7; 1.02-1.22 PFLOP/s at 2048 rows, as the 4-bit form.
 #include "gptq_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace mh {
@@ -172,7 +173,8 @@ template <int BITS, int MT, int NS>
 __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel(
     const half_t* __restrict__ x, const uint32_t* __restrict__ qweight, const uint32_t* __restrict__ qzeros,
     const half_t* __restrict__ scales, half_t* __restrict__ out, float* __restrict__ partial, int M, int N, int K,
-    int group_size, int rounds_per_block, int split_k, const half_t* __restrict__ bias, int epilogue) {
+    int group_size, int tiles_n, int whole_tiles, int split_tiles, int rounds_per_block, const half_t* __restrict__ bias,
+    int epilogue) {
     constexpr int BM = 16 * MT;
     constexpr int KS = tall_k_shares(MT);          // waves per column group, each with 32 k of every round
     constexpr int RK = 32 * KS;                    // k per round
@@ -192,16 +194,23 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cg = wave & 1, ks = wave >> 1;
     const int j = lane & 15, o = lane >> 4;
-    const int n0 = blockIdx.x * kTallBN, m0 = blockIdx.z * BM;
+    // tiles in (row block, column) order; the first whole_tiles of them walk all of K, the others are split_tiles
+    // workgroups per K range
+    const int behind = (int)blockIdx.x - whole_tiles;
+    const bool whole = behind < 0;
+    const int k_range = whole ? 0 : behind / split_tiles;
+    const int tile = whole ? (int)blockIdx.x : whole_tiles + behind - k_range * split_tiles;
+    const int tile_m = tile / tiles_n, tile_n = tile - tile_m * tiles_n;
+    const int n0 = tile_n * kTallBN, m0 = tile_m * BM;
     const int rounds_total = K / RK;
-    const int r_begin = blockIdx.y * rounds_per_block;
-    const int n_rounds = min(rounds_per_block, rounds_total - r_begin);
+    const int r_begin = k_range * rounds_per_block;
+    const int n_rounds = whole ? rounds_total : min(rounds_per_block, rounds_total - r_begin);
     // this wave's 32 k of the workgroup's first round
     const int k_wave = r_begin * RK + ks * 32;
     // first of the lane's four columns.  kEpilogueSiluPairs (columns in blocks of 128 gate + 128 up): the
-    // tile is 64 gate columns (cg = 0) and the 64 matching up columns (cg = 1) of block blockIdx.x / 2
+    // tile is 64 gate columns (cg = 0) and the 64 matching up columns (cg = 1) of block tile_n / 2
     const bool silu = epilogue == kEpilogueSiluPairs;
-    const int pair_col = (blockIdx.x >> 1) * 256 + cg * 128 + (blockIdx.x & 1) * 64;
+    const int pair_col = (tile_n >> 1) * 256 + cg * 128 + (tile_n & 1) * 64;
     const int col = (silu ? pair_col : n0 + cg * 64) + 4 * j;
 
     // the descriptors live in fixed scalar registers; past the workgroup's last round their record count is
@@ -501,7 +510,7 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
     const bool owner = MT >= 4 || ks == 0;  // holds sums to store
 
     // ---- results: acc[rt][c][e], rt < kOwn, is row (own + rt)*16 + o*4 + e, column cg*64 + 4j + c of the tile
-    if (split_k == 1) {
+    if (whole) {
         constexpr int kRow = 256 + 16;  // bytes per tile row in LDS
         if (owner) {
 #pragma unroll
@@ -514,8 +523,8 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
         }
         __syncthreads();
         if (silu) {
-            // out[m, b*128 + h*64 + c] = silu(gate) * up of the fp16-rounded sums, b = blockIdx.x / 2, h = blockIdx.x % 2
-            half_t* dst = out + (blockIdx.x >> 1) * 128 + (blockIdx.x & 1) * 64;
+            // out[m, b*128 + h*64 + c] = silu(gate) * up of the fp16-rounded sums, b = tile_n / 2, h = tile_n % 2
+            half_t* dst = out + (tile_n >> 1) * 128 + (tile_n & 1) * 64;
 #pragma unroll
             for (int i = 0; i < (BM * 8 + kThreads - 1) / kThreads; ++i) {
                 const int id = i * kThreads + tid, row = id >> 3, ch = id & 7;
@@ -538,72 +547,148 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
             if (bias) h = h + *reinterpret_cast<const half8_t*>(bias + n);
             *reinterpret_cast<half8_t*>(out + (size_t)m * N + n) = h;
         }
-    } else if constexpr (MT <= 8) {  // (sixteen row tiles: the fp32 tile does not fit the LDS; the plan never splits K there)
-        constexpr int kRow = 512 + 16;
-        if (owner) {
+    } else {
+        // up to 128 rows at a time (the fp32 tile of sixteen row tiles does not fit the LDS: first the rows of the
+        // waves with ks = 0, then of those with ks = 1)
+        constexpr int kRow = 512 + 16, kRows = BM < 128 ? BM : 128;
+        // [K range][M][N] where every tile is split, [K range][tile][BM][128] of the tiles behind the whole ones
+        const size_t pitch = whole_tiles ? kTallBN : N;
+        float* dst = whole_tiles ? partial + ((size_t)k_range * split_tiles + (tile - whole_tiles)) * (BM * kTallBN)
+                                 : partial + ((size_t)k_range * M + m0) * N + n0;
 #pragma unroll
-            for (int rt = 0; rt < kOwn; ++rt)
+        for (int part = 0; part < BM / kRows; ++part) {
+            if (part) __syncthreads();
+            if (owner && (BM == kRows || ks == part)) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float4_t v = {acc[rt][0][e], acc[rt][1][e], acc[rt][2][e], acc[rt][3][e]};
-                    *reinterpret_cast<float4_t*>(smem + ((own + rt) * 16 + o * 4 + e) * kRow + (cg * 64 + 4 * j) * 4) = v;
-                }
-        }
-        __syncthreads();
+                for (int rt = 0; rt < kOwn; ++rt)
 #pragma unroll
-        for (int i = 0; i < BM * 32 / kThreads; ++i) {
-            const int id = i * kThreads + tid, row = id >> 5, ch = id & 31;
-            const int m = m0 + row, n = n0 + ch * 4;
-            if (m >= M || n >= N) continue;
-            *reinterpret_cast<float4_t*>(partial + ((size_t)blockIdx.y * M + m) * N + n) =
-                *reinterpret_cast<const float4_t*>(smem + row * kRow + ch * 16);
+                    for (int e = 0; e < 4; ++e) {
+                        const float4_t v = {acc[rt][0][e], acc[rt][1][e], acc[rt][2][e], acc[rt][3][e]};
+                        *reinterpret_cast<float4_t*>(smem + ((own + rt) * 16 + o * 4 + e - part * kRows) * kRow + (cg * 64 + 4 * j) * 4) = v;
+                    }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kRows * 32 / kThreads; ++i) {
+                const int id = i * kThreads + tid, row = part * kRows + (id >> 5), ch = id & 31;
+                const int m = m0 + row, n = n0 + ch * 4;
+                if (m >= M || n >= N) continue;
+                *reinterpret_cast<float4_t*>(dst + row * pitch + ch * 4) =
+                    *reinterpret_cast<const float4_t*>(smem + (row - part * kRows) * kRow + ch * 16);
+            }
         }
     }
+}
+
+// The tiles behind the whole ones: partial sums [K range][tile][BM][128] added in the order of the ranges, bias or
+// SiLU * up as in the product kernel's own store.  A workgroup takes eight rows of a tile, a thread four columns
+// (SiluPairs: four output columns, the upper half of a row's threads idle).
+template <int BM>
+__global__ __launch_bounds__(256) void tall_finish_kernel(const float* __restrict__ partial, half_t* __restrict__ out, int M,
+                                                          int N, int tiles_n, int whole_tiles, int split_tiles, int ranges,
+                                                          const half_t* __restrict__ bias, int epilogue) {
+    const int t = blockIdx.x / (BM / 8), row = blockIdx.x % (BM / 8) * 8 + (threadIdx.x >> 5), c = (threadIdx.x & 31) * 4;
+    const int tile = whole_tiles + t, tile_m = tile / tiles_n, tile_n = tile - tile_m * tiles_n;
+    const int m = tile_m * BM + row, n = tile_n * kTallBN + c;
+    if (m >= M || n >= N) return;
+    const float* src = partial + ((size_t)t * BM + row) * kTallBN + c;
+    const size_t stride = (size_t)split_tiles * BM * kTallBN;
+    auto sum = [&](const float* p) {
+        float4_t s = *reinterpret_cast<const float4_t*>(p);
+        for (int r = 1; r < ranges; ++r) s += *reinterpret_cast<const float4_t*>(p + r * stride);
+        return half4_t{(half_t)s[0], (half_t)s[1], (half_t)s[2], (half_t)s[3]};
+    };
+    if (epilogue == kEpilogueSiluPairs) {
+        if (c >= 64) return;
+        const half4_t g = sum(src), u = sum(src + 64);
+        half4_t h;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) h[e] = silu_pair(g[e], u[e]);
+        *reinterpret_cast<half4_t*>(out + (size_t)m * (N / 2) + (tile_n >> 1) * 128 + (tile_n & 1) * 64 + c) = h;
+        return;
+    }
+    half4_t h = sum(src);
+    if (bias) h = h + *reinterpret_cast<const half4_t*>(bias + n);
+    *reinterpret_cast<half4_t*>(out + (size_t)m * N + n) = h;
 }
 
 // ---- host side ---------------------------------------------------------------------------
 
+// split_k: K ranges of every tile (whole_tiles = 0) or of the tiles behind the first whole_tiles (1: none)
 struct TallPlan {
-    int mt, tiles_n, row_blocks, split_k, rounds_per_block;
+    int mt, tiles_n, row_blocks, split_k, rounds_per_block, whole_tiles;
+    double cost;
+    int tiles() const { return tiles_n * row_blocks; }
+    bool tail() const { return whole_tiles > 0 && split_k > 1; }
+    bool split_all() const { return whole_tiles == 0; }
 };
 
-// MH_GEMM_TALL_MT16: 0 never blocks of 256 rows, 1 (default) where they pad the rows no further than blocks
-// of 128 and fill the CUs without a split of K, 2 wherever K need not be split.
-static int tall_mt16_mode() {
-    static const int v = [] {
+// MH_GEMM_TALL_MT16: 0 never blocks of 256 rows, 1 (default) where they take less time.
+static bool tall_mt16_allowed() {
+    static const bool v = [] {
         const char* e = getenv("MH_GEMM_TALL_MT16");
-        return e && *e ? atoi(e) : 1;
+        return !(e && *e && atoi(e) == 0);
     }();
     return v;
 }
 
-static TallPlan plan_tall(int M, int N, int K, int bits) {
+// Tiles of BM = 16 mt rows in passes over the CUs: whole tiles for as many passes as they fill, and the tiles of the
+// last pass, if they leave CUs idle, in K ranges that fill them (us, before / with the ranges: 1000 x 13696 x 5120
+// 187 / 141, 1000 x 5120 x 5120 78 / 65, 1000 x 5120 x 27392 at 8 bit 302 / 285, 700 x 4096 x 12288 97 / 80).  cost: in
+// rounds of a 128 x 128 tile (about a microsecond).  A tile of 256 rows takes 1.74 times a tile of 128 (2048 x 8192 x
+// 57344 1666 us against 1932), the ranges' sums about eight rounds on their way through memory: with these two the
+// cheapest of the four plans came out fastest or within 3 % of it for each of 25 shapes of 130 to 2048 rows.
+static TallPlan plan_passes(int mt, int M, int N, int K, bool tail_allowed) {
     TallPlan p;
-    p.mt = M <= 32 ? 2 : M <= 64 ? 4 : 8;
+    const int cus = compute_units(), k_per_round = 32 * tall_k_shares(mt), rounds = K / k_per_round;
+    p.mt = mt;
     p.tiles_n = (N + kTallBN - 1) / kTallBN;
-    if (M > 128 && tall_mt16_mode() != 0) {
-        // blocks of 256 rows: one wave per SIMD, a packed word dequantised once per 256 rows; the whole K per
-        // workgroup (its fp32 tile would not fit the LDS for a split)
-        const int blocks = (M + 255) / 256;
-        const bool same_padding = blocks * 256 == (M + 127) / 128 * 128;
-        if ((same_padding || tall_mt16_mode() == 2) && (long)p.tiles_n * blocks * 8 >= (long)compute_units() * 7) {
-            p.mt = 16;
-            p.row_blocks = blocks;
-            p.split_k = 1;
-            p.rounds_per_block = K / (32 * tall_k_shares(16));
-            return p;
+    p.row_blocks = (M + 16 * mt - 1) / (16 * mt);
+    p.split_k = 1;
+    p.rounds_per_block = rounds;
+    p.whole_tiles = p.tiles();
+    const double per_round = mt == 16 ? 1.74 / 2 : 1.0;
+    const int rest = p.tiles() % cus, full = p.tiles() / cus;
+    p.cost = per_round * rounds * (full + (rest ? 1 : 0));
+    if (rest && full && tail_allowed) {
+        const int split = std::min(cus / rest, rounds / 4);
+        if (split > 1) {
+            const int per = (rounds + split - 1) / split;
+            const double cost = per_round * (full * rounds + per) + 8;
+            if (cost < p.cost) {
+                p.whole_tiles = p.tiles() - rest;
+                p.rounds_per_block = per;
+                p.split_k = (rounds + per - 1) / per;
+                p.cost = cost;
+            }
         }
     }
+    return p;
+}
+
+static TallPlan plan_tall(int M, int N, int K, int bits, bool tail_allowed = true) {
+    TallPlan p;
+    const int cus = compute_units();
+    p.mt = M <= 32 ? 2 : M <= 64 ? 4 : 8;
+    p.tiles_n = (N + kTallBN - 1) / kTallBN;
     const int bm = 16 * p.mt;
     p.row_blocks = (M + bm - 1) / bm;
     const int rounds = K / kTallRoundK;
+    if (p.mt == 8 && p.tiles() > cus) {
+        TallPlan best = plan_passes(8, M, N, K, tail_allowed);
+        if (M > 128 && tall_mt16_allowed()) {
+            const TallPlan p16 = plan_passes(16, M, N, K, tail_allowed);
+            if (p16.cost <= best.cost) best = p16;
+        }
+        return best;
+    }
     // one workgroup per CU (eight waves; 128 KiB of LDS at eight row tiles); a workgroup keeps at least four
     // rounds, and the fp32 partial sums (8 M N bytes per split, written and read) stay below the packed
     // weights' bytes -- or below twice those where that shortens a workgroup's walk by a quarter or more
     // (4096 x 4096 at 128 rows 23.0 us with two K ranges against 19.8 with four, 5120 x 5120 26.9 / 22.9,
     // 1024 x 8192 21.5 / 16.9; below four times: 21.4, 23.8, 16.8; 4096 x 14336 at 128 rows measures the
     // same with seven and with eight ranges and keeps seven)
-    long most = (long)compute_units() / ((long)p.tiles_n * p.row_blocks);
+    long most = (long)cus / ((long)p.tiles_n * p.row_blocks);
     if (most > rounds / 4) most = rounds / 4;
     const long rows = M < bm ? M : bm;
     auto capped = [&](long per_rows) {
@@ -616,6 +701,7 @@ static TallPlan plan_tall(int M, int N, int K, int bits) {
     if (((rounds + relaxed - 1) / relaxed) * 4 <= ((rounds + split - 1) / split) * 3) split = relaxed;
     p.rounds_per_block = (int)((rounds + split - 1) / split);
     p.split_k = (rounds + p.rounds_per_block - 1) / p.rounds_per_block;
+    p.whole_tiles = p.split_k == 1 ? p.tiles() : 0;
     return p;
 }
 
@@ -681,33 +767,39 @@ bool gemm_tall_preferred(int M, int N, int K, int group_size, int bits, int epil
     return M >= 33 || (bits == 4 ? tall_two_row_tiles_preferred(M, N, K) : tall_8bit_preferred(M, N, K));
 }
 
-size_t gemm_tall_workspace_bytes(int M, int N, int K, int bits) {
-    const TallPlan p = plan_tall(M, N, K, bits);
-    return p.split_k > 1 ? kTileCounterBytes + (size_t)p.split_k * M * N * sizeof(float) : 0;
+static size_t tall_plan_bytes(const TallPlan& p, int M, int N) {
+    if (p.split_k == 1) return 0;
+    const size_t sums = p.tail() ? (size_t)(p.tiles() - p.whole_tiles) * (16 * p.mt) * kTallBN : (size_t)M * N;
+    return kTileCounterBytes + p.split_k * sums * sizeof(float);
 }
+
+size_t gemm_tall_workspace_bytes(int M, int N, int K, int bits) { return tall_plan_bytes(plan_tall(M, N, K, bits), M, N); }
 
 // kEpilogueSiluPairs in the kernel's own store: an unsplit plan, whole blocks of 128 + 128 columns.
 bool gemm_tall_silu_pairs_supported(int M, int N, int K, int group_size, int bits) {
-    return gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone) && N % 256 == 0 && plan_tall(M, N, K, bits).split_k == 1;
+    return gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone) && N % 256 == 0 && !plan_tall(M, N, K, bits).split_all();
 }
 
 int gptq_gemm_tall_launch(hipStream_t stream, const void* x, const int32_t* qweight, const int32_t* qzeros,
                           const void* scales, void* out, int M, int N, int K, int group_size, int bits, void* workspace,
                           size_t workspace_bytes, const half_t* bias, int epilogue) {
-    const TallPlan p = plan_tall(M, N, K, bits);
-    if (epilogue != kEpilogueNone && (epilogue != kEpilogueSiluPairs || p.split_k != 1 || N % 256 != 0 || bias))
+    TallPlan p = plan_tall(M, N, K, bits);
+    // a workspace without room for the last pass's sums gets whole tiles
+    if (p.tail() && (workspace == nullptr || workspace_bytes < tall_plan_bytes(p, M, N))) p = plan_tall(M, N, K, bits, false);
+    if (epilogue != kEpilogueNone && (epilogue != kEpilogueSiluPairs || p.split_all() || N % 256 != 0 || bias))
         return fail(MH_ERR_INVALID, "gptq gemm (128-row blocks): epilogue %d is not served for M=%d N=%d K=%d", epilogue, M, N, K);
-    const size_t need = gemm_tall_workspace_bytes(M, N, K, bits);
+    const size_t need = tall_plan_bytes(p, M, N);
     if (need != 0 && (workspace == nullptr || workspace_bytes < need))
         return fail(MH_ERR_WORKSPACE, "mh_gptq_gemm: workspace of %zu bytes required, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
+    const int split_tiles = p.tiles() - p.whole_tiles;
     float* partial = need ? reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + kTileCounterBytes) : nullptr;
 #define MH_LAUNCH_TALL_BITS(BITS, MT)                                                                                 \
-    hipLaunchKernelGGL((gptq_gemm_tall_kernel<BITS, MT, 4>), dim3(p.tiles_n, p.split_k, p.row_blocks),               \
+    hipLaunchKernelGGL((gptq_gemm_tall_kernel<BITS, MT, 4>), dim3(p.whole_tiles + split_tiles * p.split_k),          \
                        dim3(tall_k_shares(MT) * 128), 0,                                                              \
                        stream, (const half_t*)x, (const uint32_t*)qweight, (const uint32_t*)qzeros,                  \
-                       (const half_t*)scales, (half_t*)out, partial, M, N, K, group_size, p.rounds_per_block,        \
-                       p.split_k, bias, epilogue)
+                       (const half_t*)scales, (half_t*)out, partial, M, N, K, group_size, p.tiles_n, p.whole_tiles,  \
+                       split_tiles, p.rounds_per_block, bias, epilogue)
 #define MH_LAUNCH_TALL(MT)                                                                                            \
     if (bits == 4)                                                                                                    \
         MH_LAUNCH_TALL_BITS(4, MT);                                                                                   \
@@ -722,7 +814,15 @@ int gptq_gemm_tall_launch(hipStream_t stream, const void* x, const int32_t* qwei
 #undef MH_LAUNCH_TALL
 #undef MH_LAUNCH_TALL_BITS
     MH_CHECK_LAUNCH();
-    if (p.split_k > 1) {
+    if (p.tail()) {
+        if (p.mt == 16)
+            hipLaunchKernelGGL(tall_finish_kernel<256>, dim3(split_tiles * 32), dim3(256), 0, stream, partial, (half_t*)out,
+                               M, N, p.tiles_n, p.whole_tiles, split_tiles, p.split_k, bias, epilogue);
+        else
+            hipLaunchKernelGGL(tall_finish_kernel<128>, dim3(split_tiles * 16), dim3(256), 0, stream, partial, (half_t*)out,
+                               M, N, p.tiles_n, p.whole_tiles, split_tiles, p.split_k, bias, epilogue);
+        MH_CHECK_LAUNCH();
+    } else if (p.split_k > 1) {
         SmallFuse fuse;
         fuse.bias = bias;
         launch_splitk_finalize(stream, partial, out, M, N, p.split_k, kEpilogueNone, fuse);
