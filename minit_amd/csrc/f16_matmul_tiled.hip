@@ -4,14 +4,15 @@
 //
 // A workgroup of four waves owns BM x 128 outputs and walks K in rounds of 64.  A stage (BM + 128 rows of
 // 128 bytes) travels global -> registers -> LDS: two rounds of loads are in flight in registers, two stages
-// lie in LDS (64 KiB at BM = 128: two workgroups per CU), one barrier per round.  Through registers and not by
+// lie in LDS (64 KiB at BM = 128: two workgroups per CU), one barrier per round.  (STAGES = 1: one stage and two
+// barriers, four workgroups per CU.)  Through registers and not by
 // LDS-destination loads because a row starts on any 2-byte boundary when K is odd -- p v over a prompt of 1499
 // tokens -- and those loads want dword addresses; a 16-byte vector load takes any.
 // The K % 64 remainder is the first round: its chunks are loaded from inside the row and shifted down by
 // whole elements, so that what lies past the end of a row is zero in both operands whatever memory holds.
-// What bounds it: q k^T of a prompt its result (32 x [1500, 1500, 128] 52 us for 144 MB of scores, 76 us for the
-// 268 MB at 2048, the part's pure write rate is 7 TB/s; without the streaming hint on the stores 55 and 107), p v
-// the read of p (32 x [1500, 128, 1500] 43 us), a product of many rows and columns the operands on their way into LDS
+// What bounds it: q k^T of a prompt its result (32 x [1500, 1500, 128] 46 us for 144 MB of scores, the part's
+// pure write rate is 7 TB/s; without the streaming hint on the stores half as long again at 2048), p v the read of p
+// (32 x [1500, 128, 1500] 47 us, with rows on 128-byte lines, K = 1536, 41), a product of many rows and columns the operands on their way into LDS
 // (2048 x 4096 x 4096 87 us, 790 TFLOP/s).  K not a multiple of 32 took one thread per output before: 27.6 ms
 // for that p v.
 // The weight fragment is the first MFMA operand: a lane ends with four consecutive n of one row, the tile
@@ -37,16 +38,16 @@ __device__ __forceinline__ uint4_t drop_elements(uint4_t v, int n) {
     return uint4_t{(unsigned)new_lo, (unsigned)(new_lo >> 32), (unsigned)new_hi, (unsigned)(new_hi >> 32)};
 }
 
-template <int BM>
-__global__ __launch_bounds__(kTiledThreads, 2) void f16_matmul_nk_tiled_kernel(
+template <int BM, int STAGES>
+__global__ __launch_bounds__(kTiledThreads, STAGES == 1 ? 4 : 2) void f16_matmul_nk_tiled_kernel(
     const half_t* __restrict__ a, const half_t* __restrict__ b, half_t* __restrict__ out, int M, int N, int K,
     int tiles_m, int tiles_n) {
-    constexpr int WN = BM == 128 ? 2 : 4;      // waves along n
-    constexpr int MT = BM == 32 ? 2 : 4;       // 16-row tiles of a per wave
+    constexpr int WN = BM > 64 ? 2 : 4;        // waves along n
+    constexpr int MT = BM / 16 / (4 / WN);     // 16-row tiles of a per wave
     constexpr int NT = kTiledBN / WN / 16;     // 16-column tiles per wave
     constexpr int AC = BM / 32, BC = 4;        // 16-byte chunks of a stage per thread
     constexpr int kStage = (BM + kTiledBN) * 128;
-    constexpr int kLds = 2 * kStage > BM * kTiledPitch ? 2 * kStage : BM * kTiledPitch;
+    constexpr int kLds = STAGES * kStage > BM * kTiledPitch ? STAGES * kStage : BM * kTiledPitch;
     __shared__ __attribute__((aligned(1024))) char smem[kLds];
 
     // Consecutive workgroups go to different XCDs: give each a run of tiles in (matrix, row, column) order, so
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(kTiledThreads, 2) void f16_matmul_nk_tiled_kernel(
         for (int i = 0; i < AC; ++i) ra[0][i] = drop_elements(ra[0][i], drop);
 #pragma unroll
         for (int i = 0; i < BC; ++i) rb[0][i] = drop_elements(rb[0][i], drop);
-        store(0, 1);
+        store(0, STAGES - 1);
     }
     if (rounds) {
         load(0, 0);
@@ -132,9 +133,25 @@ __global__ __launch_bounds__(kTiledThreads, 2) void f16_matmul_nk_tiled_kernel(
     }
     if (rest) {
         __syncthreads();
-        compute(1);
+        compute(STAGES - 1);
+        if (STAGES == 1) __syncthreads();
     }
-    if (rounds) {
+    if constexpr (STAGES == 1) {
+        for (int r = 0; r < rounds; r += 2) {
+            store(0, 0);
+            load(0, r + 2);
+            __syncthreads();
+            compute(0);
+            if (r + 1 >= rounds) break;
+            __syncthreads();
+            store(1, 0);
+            load(1, r + 3);
+            __syncthreads();
+            compute(0);
+            if (r + 2 >= rounds) break;
+            __syncthreads();
+        }
+    } else if (rounds) {
         store(0, 0);
         load(0, 2);
         __syncthreads();
@@ -204,18 +221,48 @@ bool f16_matmul_tiled_preferred(int M, int N, int K) {
     return (N <= 256 && K <= 4096) || tiles_n * ((M + 127) / 128) >= 2 * cus || (M <= 128 && tiles_n * 4 >= 3 * cus);
 }
 
+// Height of the tiles.  A CU takes about a microsecond for a stage of 256 rows whether one workgroup asks or two, so
+// the time goes with the staged rows of the CU that has most: ceil(tiles / CUs) * (BM + 128).  Measured in
+// us, 128 / 64 / 32 rows: 16 x [479, 128, 479] 11.2 / 8.4 / 6.7 (the rule's 32), 8 x [1245, 128, 1245] 22.8 / 16.5 / 20.5
+// (64), 8 x [300, 128, 300] 6.6 / 5.1 / 4.4 (32), 16 x [2000, 128, 2000] 35.6 / 43.7 / 57.8 (128), 32 x [1500, 128, 1500]
+// 53.3 / 54.0 / 78.5, with 96 rows 47.1 (96).
+// Two rounds of K and less (q k^T) are all beginnings and ends: tiles of 64 rows with one stage in LDS, four
+// workgroups per CU (32 x [1500, 1500, 128] 49.5 -> 45.8, 8 x [300, 300, 128] 6.0 -> 4.3).
+struct TiledPlan {
+    int bm, stages;
+};
+static TiledPlan plan_tiled(int batch, int M, int N, int K) {
+    if (K <= 2 * kTiledBK && M > 32) return {64, 1};
+    const size_t cus = compute_units(), columns = (size_t)batch * ((N + kTiledBN - 1) / kTiledBN);
+    TiledPlan best = {32, 2};
+    size_t least = 0;
+    for (int bm = M <= 32 ? 32 : M <= 64 ? 64 : M <= 96 ? 96 : 128; bm >= 32; bm -= 32) {
+        const size_t cost = (columns * ((M + bm - 1) / bm) + cus - 1) / cus * (bm + 128);
+        if (least == 0 || cost < least) {
+            least = cost;
+            best.bm = bm;
+        }
+    }
+    return best;
+}
+
 int f16_matmul_tiled_launch(hipStream_t stream, const void* a, const void* b, void* out, int batch, int M, int N, int K) {
-    const int bm = M <= 32 ? 32 : M <= 64 ? 64 : 128;
-    const int tiles_m = (M + bm - 1) / bm, tiles_n = (N + kTiledBN - 1) / kTiledBN;
+    const TiledPlan p = plan_tiled(batch, M, N, K);
+    const int bm = p.bm, tiles_m = (M + bm - 1) / bm, tiles_n = (N + kTiledBN - 1) / kTiledBN;
     const size_t tiles = (size_t)tiles_m * tiles_n * batch;
     MH_REQUIRE(tiles <= 0x7fffffffu, "dense fp16 product: %zu output tiles are too many for one launch", tiles);
-#define MH_TILED(BM)                                                                                               \
-    hipLaunchKernelGGL(f16_matmul_nk_tiled_kernel<BM>, dim3((unsigned)tiles), dim3(kTiledThreads), 0, stream,       \
+#define MH_TILED(BM, STAGES)                                                                                       \
+    hipLaunchKernelGGL((f16_matmul_nk_tiled_kernel<BM, STAGES>), dim3((unsigned)tiles), dim3(kTiledThreads), 0, stream, \
                        (const half_t*)a, (const half_t*)b, (half_t*)out, M, N, K, tiles_m, tiles_n)
-    switch (bm) {
-        case 32: MH_TILED(32); break;
-        case 64: MH_TILED(64); break;
-        default: MH_TILED(128); break;
+    if (p.stages == 1) {
+        MH_TILED(64, 1);
+    } else {
+        switch (bm) {
+            case 32: MH_TILED(32, 2); break;
+            case 64: MH_TILED(64, 2); break;
+            case 96: MH_TILED(96, 2); break;
+            default: MH_TILED(128, 2); break;
+        }
     }
 #undef MH_TILED
     MH_CHECK_LAUNCH();

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("batch,m,n,k", [
     (1, 1, 1, 8), (2, 5, 7, 9), (3, 33, 129, 63),          # shorter than a round: the remainder alone
     (2, 32, 128, 65), (2, 31, 130, 71), (1, 64, 127, 127),  # one round and 1, 7, 63 elements
-    (2, 65, 129, 128), (3, 128, 256, 192), (1, 129, 5, 193),  # 128-row tiles, two and three rounds, odd rows
+    (2, 65, 129, 128), (3, 128, 256, 192), (1, 129, 5, 193), (32, 1500, 100, 130), (2, 96, 130, 200), (3, 97, 129, 129),  # 128-row tiles, two and three rounds, odd rows
     (2, 200, 300, 1001), (4, 257, 128, 1500), (2, 130, 128, 4096),  # the p v of a prompt
     (1, 2100, 4200, 256), (1, 100, 24600, 512)])            # two tiles per CU; one block of rows
 def test_tiled_dense_product(hip, batch, m, n, k):
