@@ -254,9 +254,10 @@ __global__ __launch_bounds__(kRowThreads) void softmax_rows_kernel(
     for (int c = 0; c < CHUNKS; ++c) {
         const int v = c * LANES + lane, at = column(v);
         if (v < nvec) {
+            // a piece that was not read is 0 * inv and not 0: a row whose sum is NaN is NaN throughout
             if (CAUSAL && at > limit) {
-                stream_store_any(dst + at, make_uint4(0u, 0u, 0u, 0u));
-                continue;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) vals[c][i] = 0.f;
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) vals[c][i] = sizeof(T) == 2 ? vals[c][i] * inv : vals[c][i] / sum;

@@ -27,3 +27,19 @@ def test_ragged_rows(hip, heads, s, offset):
         # one fp16 step: the fp32 exponential and sum are three orders below it
         assert (np.abs(got.astype(np.float64) - ref) <= np.spacing(ref.astype(np.float16)).astype(np.float64)).all()
     assert (causal[:, np.arange(t)[None, :] - offset > np.arange(s)[:, None]] == 0).all()
+
+
+@pytest.mark.parametrize("s,t", [(40, 40), (150, 150), (600, 1500), (256, 2048), (64, 5001)])
+def test_causal_rows_without_a_sum(hip, s, t):
+    """NaN, +inf or nothing but -inf among the visible columns: the whole row is NaN, its masked end included."""
+    from minit_amd.hip.tensor import HIPTensor
+    x = np.random.default_rng(t).normal(size=(s, t)).astype(np.float16)
+    offset = t - s
+    x[1, 0], x[2, offset], x[4, :offset + 5] = np.nan, np.inf, -np.inf
+    x[6, offset + 7:] = np.nan   # masked: counts nowhere
+    d, out = HIPTensor.from_numpy(x), HIPTensor.allocate(x.shape, "float16")
+    hip.call("mh_softmax_causal", None, d.data_ptr, out.data_ptr, 1, s, t, offset, 1.0, 0)
+    got = out.numpy()
+    none = np.isin(np.arange(s), (1, 2, 4))
+    assert np.isnan(got[none]).all()
+    assert np.isfinite(got[~none]).all() and (got[6, offset + 7:] == 0).all()
