@@ -283,28 +283,6 @@ struct AttnWave {
             for (int dt = 0; dt < 8; ++dt) vf[dt][ks] = at(v, dt * 16 * kVTile + ks * 32, lane_v);
     }
 
-    // The same with an address per lane, which the compiler mixes into the chunk's arithmetic: K as soon as its
-    // registers are free, V behind Q K^T.  Four waves of a block (one per SIMD) are 3 to 7 % faster with it
-    // (8 rows x 8 heads x 2112 16.6 us against 17.8 with the form above), eight waves 4 % slower
-    // (32 x 8 x 2048 40.7 against 39.0).  Rows and tiles are clamped to the cache.
-    __device__ __forceinline__ void load_chunk_by_lane(const half_t* kbase, const half_t* vbase, int c0, int max_seq,
-                                                       int i16, int kq) {
-#pragma unroll
-        for (int pt = 0; pt < 4; ++pt) {
-            const int row = min(c0 + pt * 16 + i16, max_seq - 1);
-            const half_t* kp = kbase + (size_t)row * D + kq * 8;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) kf[pt][s] = *reinterpret_cast<const uint4*>(kp + s * 32);
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int p0 = min(c0 + ks * 32 + kq * 8, max_seq - 8);
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt)
-                vf[dt][ks] = *reinterpret_cast<const uint4*>(vbase + vt_offset(dt * 16 + i16, p0));
-        }
-    }
-
     // The loaded chunk of positions c0 .. c0 + 63, of which those below t1 (at least one) count;
     // p_s: the wave's own P tile in LDS.
     __device__ __forceinline__ void step(half_t* p_s, int c0, int t1, float scale, int i16, int kq) {
@@ -461,22 +439,18 @@ __device__ __forceinline__ void attn_fold_records(half_t* out, int d, int count,
     attn_store(out, a, ll);
 }
 
+// A block per (row, KV head) pair.
 template <int G, int D, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
-    const int32_t* __restrict__ positions, half_t* __restrict__ out, float* partial, unsigned* counters,
-    int kvh, int max_seq, float scale, int splits) {
-    const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = WAVES > 4 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
+    const int32_t* __restrict__ positions, half_t* __restrict__ out, int kvh, int max_seq, float scale) {
+    const int g = blockIdx.y, b = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i16 = lane & 15, kq = lane >> 4;
-    // Chunks of 64 positions (one tile of the V cache) are dealt round robin, first over the
-    // blocks of a (row, KV head) pair and then over their waves: chunk c belongs to block
-    // c % splits, wave (c / splits) % WAVES.  The deal does not depend on the length, so a
-    // wave requests its first chunk before the position has arrived, and no wave holds more
-    // than one chunk over the others.
-    const int stride = splits * WAVES * 64;
-    const int c_first = (split + wave * splits) * 64;
+    // Chunks of 64 positions (one tile of the V cache) are dealt round robin to the waves, whatever the length:
+    // a wave requests its first chunk before the position has arrived.
+    constexpr int stride = WAVES * 64;
+    const int c_first = wave * 64;
     const int t1 = min(max(positions[b], 0), max_seq - 1) + 1;  // the new token has been appended
 
     __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * kAttnPitch];
@@ -489,12 +463,8 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
     w.load_q(q + pair * G * D, i16, kq);
     w.reset();
     auto load = [&](int c0) {
-        if constexpr (WAVES > 4) {
-            const size_t at = (size_t)min(c0, max_seq - 64) * D;   // a chunk past the cache is not used: any will do
-            w.load_chunk(kbase + at, vbase + at, i16, kq);
-        } else {
-            w.load_chunk_by_lane(kbase, vbase, c0, max_seq, i16, kq);
-        }
+        const size_t at = (size_t)min(c0, max_seq - 64) * D;   // a chunk past the cache is not used: any will do
+        w.load_chunk(kbase + at, vbase + at, i16, kq);
     };
     load(c_first);
     // Two waves share a SIMD when a block has eight, and the older one wins every arbitration: the
@@ -503,9 +473,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
     const int n_chunks = t1 > c_first ? (t1 - c_first + stride - 1) / stride : 0;
     int chunk_no = 0;
     for (int c0 = c_first; c0 < t1;) {
-        if constexpr (WAVES > 4) {
-            set_priority_by_progress(chunk_no++, n_chunks);
-        }
+        set_priority_by_progress(chunk_no++, n_chunks);
         w.step(p_s[wave], c0, t1, scale, i16, kq);
         c0 += stride;
         if (c0 < t1) load(c0);
@@ -519,21 +487,232 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
     if (tid < merge.kItems) {
         float mm, ll;
         const float4_t a = merge.fold(h, d, mm, ll);
-        if (splits == 1) {
-            attn_store(out + (head0 + h) * D + d, a, ll);
-        } else {
-            float* pp = partial + ((head0 + h) * splits + split) * kAttnRecord;
-            store_agent4(pp + d, a);
-            if (d == 0) store_agent4(pp + D, float4_t{mm, ll, 0.f, 0.f});
+        attn_store(out + (head0 + h) * D + d, a, ll);
+    }
+}
+
+// A pair over `splits` blocks of four waves.  The body stands on its own and not on AttnWave: the same walk written
+// over that struct compiles to loads of V held back into the softmax and takes 19.6 us against 18.3 in the decode
+// loop at batch 8 (asked for ahead of the softmax by a scheduling barrier: 20.0).
+template <int G, int D>
+__global__ __launch_bounds__(256) void attn_decode_split_kernel(
+    const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
+    const int32_t* __restrict__ positions, half_t* __restrict__ out, float* partial, unsigned* counters,
+    int kvh, int max_seq, float scale, int splits) {
+    static_assert(D == 128 && G <= 16, "head size 128, at most 16 query heads per KV head");
+    constexpr int WAVES = 4, PP = kAttnPitch;
+    const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i16 = lane & 15, kq = lane >> 4;
+    // Chunks of 64 positions (one tile of the V cache) are dealt round robin, first over the
+    // blocks of a (row, KV head) pair and then over their waves: chunk c belongs to block
+    // c % splits, wave (c / splits) % WAVES.  The deal does not depend on the length, so a
+    // wave requests its first chunk before the position has arrived, and no wave holds more
+    // than one chunk over the others.
+    const int stride = splits * WAVES * 64;
+    const int c_first = (split + wave * splits) * 64;
+    const int t1 = min(max(positions[b], 0), max_seq - 1) + 1;  // the new token has been appended
+
+    __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * PP];
+    __shared__ float m_s[WAVES][16], l_s[WAVES][16];
+    __shared__ float acc_s[WAVES][G][D];
+
+    // A operand of S = Q K^T: row = head i16, k = dims s*32 + kq*8 .. +8
+    uint4 qf[4];
+    {
+        const half_t* qp = q + (((size_t)b * kvh + g) * G + min(i16, G - 1)) * D + kq * 8;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            qf[s] = *reinterpret_cast<const uint4*>(qp + s * 32);
+            if (i16 >= G) qf[s] = make_uint4(0, 0, 0, 0);
         }
     }
-    if (splits == 1) return;
+    const half_t* kbase = k_cache + ((size_t)b * kvh + g) * max_seq * D;
+    const half_t* vbase = vt_cache + ((size_t)b * kvh + g) * D * max_seq;
+
+    // rows of every accumulator tile held by this lane: heads kq*4 + r
+    float m_run[4], l_run[4];
+    float4_t acc[8];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        m_run[r] = -INFINITY;
+        l_run[r] = 0.f;
+    }
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) acc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    // all loads of a chunk are issued before the first use (refilling K after Q K^T and V
+    // after P V for the wave's next chunk, so that loads stay in flight under the arithmetic,
+    // measured no faster at batch 1 and 32 and slower at 8).  Rows and tiles are clamped to
+    // the cache, not to the length: what lies past the end is masked below.
+    uint4 kf[4][4], vf[8][2];
+    auto load_chunk = [&](int c0) {
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt) {
+            const int row = min(c0 + pt * 16 + i16, max_seq - 1);
+            const half_t* kp = kbase + (size_t)row * D + kq * 8;
+#pragma unroll
+            for (int s = 0; s < 4; ++s) kf[pt][s] = *reinterpret_cast<const uint4*>(kp + s * 32);
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int p0 = min(c0 + ks * 32 + kq * 8, max_seq - 8);
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+                vf[dt][ks] = *reinterpret_cast<const uint4*>(vbase + vt_offset(dt * 16 + i16, p0));
+        }
+    };
+    load_chunk(c_first);
+    for (int c0 = c_first; c0 < t1;) {
+        // S tile pt: rows = heads kq*4 + r, column = position c0 + pt*16 + i16
+        float4_t sc[4];
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt) {
+            sc[pt] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                sc[pt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, qf[s]),
+                                                                __builtin_bit_cast(half8_t, kf[pt][s]), sc[pt], 0, 0, 0);
+        }
+        float alpha[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int pt = 0; pt < 4; ++pt) {
+                const bool valid = c0 + pt * 16 + i16 < t1;
+                sc[pt][r] = valid ? sc[pt][r] * scale : -INFINITY;
+                mx = fmaxf(mx, sc[pt][r]);
+            }
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+            const float m_new = fmaxf(m_run[r], mx);  // finite: every chunk holds a valid position
+            alpha[r] = expf(m_run[r] - m_new);         // exp(-inf) = 0 on the first chunk
+            float sum = 0.f;
+#pragma unroll
+            for (int pt = 0; pt < 4; ++pt) {
+                const float pv = expf(sc[pt][r] - m_new);  // exp(-inf) = 0 for masked positions
+                sum += pv;
+                p_s[wave][(kq * 4 + r) * PP + pt * 16 + i16] = (half_t)pv;
+            }
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off, 64);
+            l_run[r] = l_run[r] * alpha[r] + sum;
+            m_run[r] = m_new;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // A operand of O += P V: row = head i16, k = positions ks*32 + kq*8 .. +8 of the chunk
+        uint4 pa[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+            pa[ks] = *reinterpret_cast<const uint4*>(&p_s[wave][i16 * PP + ks * 32 + kq * 8]);
+        if (c0 + 64 > t1) {
+            // positions past the end carry weight 0 but whatever the cache holds there
+            // (possibly not finite): clear them
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const int p0 = c0 + ks * 32 + kq * 8;
+#pragma unroll
+                for (int dt = 0; dt < 8; ++dt) {
+                    half8_t v = __builtin_bit_cast(half8_t, vf[dt][ks]);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (p0 + e >= t1) v[e] = (half_t)0.f;
+                    vf[dt][ks] = __builtin_bit_cast(uint4, v);
+                }
+            }
+        }
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[dt][r] *= alpha[r];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, pa[ks]),
+                                                                 __builtin_bit_cast(half8_t, vf[dt][ks]), acc[dt], 0, 0, 0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();  // p_s is rewritten by the next chunk
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        c0 += stride;
+        if (c0 < t1) load_chunk(c0);
+    }
+
+    // acc[dt][r] is head kq*4 + r, dim dt*16 + i16
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int h = kq * 4 + r;
+        if (h < G) {
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) acc_s[wave][h][dt * 16 + i16] = acc[dt][r];
+            if (i16 == 0) {
+                m_s[wave][h] = m_run[r];
+                l_s[wave][h] = l_run[r];
+            }
+        }
+    }
+    __syncthreads();
+
+    // merge the waves: thread -> (head, four dims)
+    constexpr int REC = kAttnRecord, ITEMS = G * D / 4;  // <= 256
+    const size_t head0 = ((size_t)b * kvh + g) * G;
+    const int h = tid / (D / 4), d = tid % (D / 4) * 4;
+    if (tid < ITEMS) {
+        float mm = m_s[0][h];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) mm = fmaxf(mm, m_s[w][h]);
+        float ll = 0.f;
+        float4_t a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const float f = (m_s[w][h] == -INFINITY) ? 0.f : expf(m_s[w][h] - mm);
+            ll += l_s[w][h] * f;
+            a += *reinterpret_cast<const float4_t*>(&acc_s[w][h][d]) * f;
+        }
+        float* pp = partial + ((head0 + h) * splits + split) * REC;
+        store_agent4(pp + d, a);
+        if (d == 0) store_agent4(pp + D, float4_t{mm, ll, 0.f, 0.f});
+    }
 
     __shared__ int is_last;
-    if (!arrive_and_check_last(counters + pair, (unsigned)splits, &is_last)) return;
-    if (tid < merge.kItems) {
-        const float* pp = partial + (head0 + h) * splits * kAttnRecord;
-        attn_fold_records<16>(out + (head0 + h) * D + d, d, splits, [&](int i) { return pp + (size_t)i * kAttnRecord; });
+    if (!arrive_and_check_last(counters + (size_t)b * kvh + g, (unsigned)splits, &is_last)) return;
+    // Last block: merge the splits.  Every thread folds the splits of its four
+    // output elements with the running-maximum recurrence, reading each split's
+    // maximum, sum and partial values itself: the loads of up to 16 splits are
+    // independent and in flight together, so the merge costs one memory round
+    // trip.
+    constexpr int BATCH = 16;
+    if (tid < ITEMS) {
+        const float* pp = partial + (head0 + h) * splits * REC;
+        float mm = -INFINITY, ll = 0.f;
+        float4_t a = {0.f, 0.f, 0.f, 0.f};
+        for (int sp0 = 0; sp0 < splits; sp0 += BATCH) {
+            float ms[BATCH], ls[BATCH];
+            float4_t as[BATCH];
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+                const float* ps = pp + (size_t)min(sp0 + u, splits - 1) * REC;
+                as[u] = load_agent4(ps + d);
+                ms[u] = load_agent(ps + D);
+                ls[u] = load_agent(ps + D + 1);
+            }
+            wait_agent_loads(as);
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) {
+                if (sp0 + u < splits && ms[u] != -INFINITY) {
+                    const float m_new = fmaxf(mm, ms[u]);
+                    const float f_old = expf(mm - m_new);  // exp(-inf) = 0 for the first split folded in
+                    const float f = expf(ms[u] - m_new);
+                    ll = ll * f_old + ls[u] * f;
+                    a = a * f_old + as[u] * f;
+                    mm = m_new;
+                }
+            }
+        }
+        const half4_t o = {(half_t)(a[0] / ll), (half_t)(a[1] / ll), (half_t)(a[2] / ll), (half_t)(a[3] / ll)};
+        *reinterpret_cast<half4_t*>(out + (head0 + h) * D + d) = o;
     }
 }
 
@@ -752,9 +931,9 @@ static void launch_attn_raw(hipStream_t st, const half_t* q, const half_t* k_cac
                            vt_cache, positions, out, partial, counters, batch, n_kv_heads, max_seq, scale);
     else if (splits == 1)
         hipLaunchKernelGGL((attn_decode_kernel<G, 128, 8>), dim3(1, n_kv_heads, batch), dim3(512), 0, st, q, k_cache,
-                           vt_cache, positions, out, partial, counters, n_kv_heads, max_seq, scale, 1);
+                           vt_cache, positions, out, n_kv_heads, max_seq, scale);
     else
-        hipLaunchKernelGGL((attn_decode_kernel<G, 128, 4>), dim3(splits, n_kv_heads, batch), dim3(256), 0, st, q,
+        hipLaunchKernelGGL((attn_decode_split_kernel<G, 128>), dim3(splits, n_kv_heads, batch), dim3(256), 0, st, q,
                            k_cache, vt_cache, positions, out, partial, counters, n_kv_heads, max_seq, scale, splits);
 }
 
