@@ -319,6 +319,9 @@ int mh_gather_columns(mh_stream_t stream, const void* x, const int32_t* index, v
  *                       fp32 inside, one rounding; D == 128, QH / KVH in {1, 2, 4, 8};
  *                       positions[b] is the index of the newest cache entry; cache
  *                       entries past it are never part of the result, whatever they hold.
+ *                       A row's bits follow from its own data, the batch and the cache's
+ *                       size: not from the other rows' lengths, nor from what room the
+ *                       workspace has beyond the least it needs.
  *                       The workspace is zero-filled once by the caller and left with its
  *                       counters at zero; where the counters end depends on batch and
  *                       KVH, so a workspace that moves to a call with other sizes is

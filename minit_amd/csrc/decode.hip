@@ -14,6 +14,7 @@
 //     host, minit/chat/sample.py:11-14).
 #include "gptq_common.h"
 
+#include <algorithm>
 #include <cstring>
 #include <new>
 #include <vector>
@@ -230,278 +231,94 @@ __global__ __launch_bounds__(1024) void argmax_advance_kernel(const half_t* __re
 // alternate chunks and are merged through LDS; splits are merged by the last
 // block to arrive.
 
-constexpr int kAttnPitch = 72;   // halfs per row of the P tile in LDS (64 + padding)
-
-// What one wave holds of the G heads of a (row, KV head) pair, and its walk over 64-position chunks.
-template <int G, int D>
-struct AttnWave {
-    static_assert(D == 128 && G <= 16, "head size 128, at most 16 query heads per KV head");
-    uint4 qf[4];
-    uint4 kf[4][4], vf[8][2];
-    // rows of every accumulator tile held by this lane: heads kq*4 + r; acc[dt][r] is dim dt*16 + i16
-    float m_run[4], l_run[4];
-    float4_t acc[8];
-
-    __device__ __forceinline__ void reset() {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            m_run[r] = -INFINITY;
-            l_run[r] = 0.f;
-        }
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) acc[dt] = float4_t{0.f, 0.f, 0.f, 0.f};
-    }
-
-    // A operand of S = Q K^T: row = head i16, k = dims s*32 + kq*8 .. +8 (q: the pair's G heads)
-    __device__ __forceinline__ void load_q(const half_t* q, int i16, int kq) {
-        const half_t* qp = q + (size_t)min(i16, G - 1) * D + kq * 8;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            qf[s] = *reinterpret_cast<const uint4*>(qp + s * 32);
-            if (i16 >= G) qf[s] = make_uint4(0, 0, 0, 0);
-        }
-    }
-
-    // all loads of a chunk are issued before the first use (refilling K after Q K^T and V
-    // after P V for the wave's next chunk, so that loads stay in flight under the arithmetic,
-    // measured no faster at batch 1 and 32 and slower at 8).  k, v: the chunk's 64 rows of K and
-    // its tile of V, the same address for the whole wave; what lies past a row's end is masked in
-    // step().
-    __device__ __forceinline__ void load_chunk(const half_t* k, const half_t* v, int i16, int kq) {
-        const unsigned lane_k = (i16 * D + kq * 8) * sizeof(half_t), lane_v = (i16 * kVTile + kq * 8) * sizeof(half_t);
-        auto at = [](const half_t* base, int halfs, unsigned lane) {
-            return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base + halfs) + lane);
-        };
-#pragma unroll
-        for (int pt = 0; pt < 4; ++pt)
-#pragma unroll
-            for (int s = 0; s < 4; ++s) kf[pt][s] = at(k, pt * 16 * D + s * 32, lane_k);
-        __builtin_amdgcn_sched_barrier(0);   // K first: Q K^T starts while V is on its way
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt) vf[dt][ks] = at(v, dt * 16 * kVTile + ks * 32, lane_v);
-    }
-
-    // The loaded chunk of positions c0 .. c0 + 63, of which those below t1 (at least one) count;
-    // p_s: the wave's own P tile in LDS.
-    __device__ __forceinline__ void step(half_t* p_s, int c0, int t1, float scale, int i16, int kq) {
-        // S tile pt: rows = heads kq*4 + r, column = position c0 + pt*16 + i16
-        float4_t sc[4];
-#pragma unroll
-        for (int pt = 0; pt < 4; ++pt) {
-            sc[pt] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-                sc[pt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, qf[s]),
-                                                                __builtin_bit_cast(half8_t, kf[pt][s]), sc[pt], 0, 0, 0);
-        }
-        float alpha[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            float mx = -INFINITY;
-#pragma unroll
-            for (int pt = 0; pt < 4; ++pt) {
-                const bool valid = c0 + pt * 16 + i16 < t1;
-                sc[pt][r] = valid ? sc[pt][r] * scale : -INFINITY;
-                mx = fmaxf(mx, sc[pt][r]);
-            }
-#pragma unroll
-            for (int off = 1; off < 16; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-            const float m_new = fmaxf(m_run[r], mx);  // finite: every chunk holds a valid position
-            alpha[r] = expf(m_run[r] - m_new);         // exp(-inf) = 0 on the first chunk
-            float sum = 0.f;
-#pragma unroll
-            for (int pt = 0; pt < 4; ++pt) {
-                const float pv = expf(sc[pt][r] - m_new);  // exp(-inf) = 0 for masked positions
-                sum += pv;
-                p_s[(kq * 4 + r) * kAttnPitch + pt * 16 + i16] = (half_t)pv;
-            }
-#pragma unroll
-            for (int off = 1; off < 16; off <<= 1) sum += __shfl_xor(sum, off, 64);
-            l_run[r] = l_run[r] * alpha[r] + sum;
-            m_run[r] = m_new;
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // A operand of O += P V: row = head i16, k = positions ks*32 + kq*8 .. +8 of the chunk
-        uint4 pa[2];
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-            pa[ks] = *reinterpret_cast<const uint4*>(&p_s[i16 * kAttnPitch + ks * 32 + kq * 8]);
-        if (c0 + 64 > t1) {
-            // positions past the end carry weight 0 but whatever the cache holds there
-            // (possibly not finite): clear them
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const int p0 = c0 + ks * 32 + kq * 8;
-#pragma unroll
-                for (int dt = 0; dt < 8; ++dt) {
-                    half8_t v = __builtin_bit_cast(half8_t, vf[dt][ks]);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (p0 + e >= t1) v[e] = (half_t)0.f;
-                    vf[dt][ks] = __builtin_bit_cast(uint4, v);
-                }
-            }
-        }
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[dt][r] *= alpha[r];
-#pragma unroll
-            for (int ks = 0; ks < 2; ++ks)
-                acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, pa[ks]),
-                                                                 __builtin_bit_cast(half8_t, vf[dt][ks]), acc[dt], 0, 0, 0);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();  // p_s is rewritten by the next chunk
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-};
-
 constexpr int kAttnRecord = 128 + 4;   // floats of one head's record in the workspace: acc[D], m, l, two unused
 
-// The waves of a block meet: their sums (zero chunks: maximum -inf) added into one, per head and four dims.
-template <int G, int D, int WAVES>
-struct AttnMerge {
-    static constexpr int kItems = G * D / 4;   // threads that merge: (head, four dims) each
-    float m[WAVES][16], l[WAVES][16];
-    float acc[WAVES][G][D];
-
-    __device__ __forceinline__ void put(const AttnWave<G, D>& w, int wave, int i16, int kq) {
+// Maximum, sum and accumulators of `WAVES` parts of a head added up, in the order of the waves: m(w), l(w) and
+// acc(w) are those of wave w (zero chunks: maximum -inf).
+template <int WAVES, typename M, typename L, typename A>
+__device__ __forceinline__ float4_t attn_fold_waves(M m, L l, A acc, float& ll, float& mm) {
+    mm = m(0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int h = kq * 4 + r;
-            if (h < G) {
+    for (int w = 1; w < WAVES; ++w) mm = fmaxf(mm, m(w));
+    ll = 0.f;
+    float4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int dt = 0; dt < 8; ++dt) acc[wave][h][dt * 16 + i16] = w.acc[dt][r];
-                if (i16 == 0) {
-                    m[wave][h] = w.m_run[r];
-                    l[wave][h] = w.l_run[r];
-                }
-            }
-        }
+    for (int w = 0; w < WAVES; ++w) {
+        const float f = (m(w) == -INFINITY) ? 0.f : expf(m(w) - mm);
+        ll += l(w) * f;
+        a += acc(w) * f;
     }
-    __device__ __forceinline__ float4_t fold(int h, int d, float& mm, float& ll) const {
-        mm = m[0][h];
-#pragma unroll
-        for (int w = 1; w < WAVES; ++w) mm = fmaxf(mm, m[w][h]);
-        ll = 0.f;
-        float4_t a = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const float f = (m[w][h] == -INFINITY) ? 0.f : expf(m[w][h] - mm);
-            ll += l[w][h] * f;
-            a += *reinterpret_cast<const float4_t*>(&acc[w][h][d]) * f;
-        }
-        return a;
-    }
-};
+    return a;
+}
 
 __device__ __forceinline__ void attn_store(half_t* out, float4_t a, float ll) {
     const half4_t o = {(half_t)(a[0] / ll), (half_t)(a[1] / ll), (half_t)(a[2] / ll), (half_t)(a[3] / ll)};
     *reinterpret_cast<half4_t*>(out) = o;
 }
 
-// Last block of a pair: every thread folds the records of its four output elements with the
-// running-maximum recurrence, reading each record's maximum, sum and partial values itself: the loads
-// of up to BATCH records are independent and in flight together, so the merge costs one memory round
-// trip.  record(i) is the address of record i of `count`.
-template <int BATCH, typename Record>
-__device__ __forceinline__ void attn_fold_records(half_t* out, int d, int count, Record record) {
-    float mm = -INFINITY, ll = 0.f;
-    float4_t a = {0.f, 0.f, 0.f, 0.f};
-    for (int sp0 = 0; sp0 < count; sp0 += BATCH) {
-        float ms[BATCH], ls[BATCH];
-        float4_t as[BATCH];
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const float* ps = record(min(sp0 + u, count - 1));
-            as[u] = load_agent4(ps + d);
-            ms[u] = load_agent(ps + 128);
-            ls[u] = load_agent(ps + 128 + 1);
-        }
-        wait_agent_loads(as);
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            if (sp0 + u < count && ms[u] != -INFINITY) {
-                const float m_new = fmaxf(mm, ms[u]);
-                const float f_old = expf(mm - m_new);  // exp(-inf) = 0 for the first record folded in
-                const float f = expf(ms[u] - m_new);
-                ll = ll * f_old + ls[u] * f;
-                a = a * f_old + as[u] * f;
-                mm = m_new;
-            }
-        }
-    }
-    attn_store(out, a, ll);
+// Rows of different lengths, up to a (row, KV head) pair per CU.  A pair is kAttnPairWaves streams of chunks, and they need
+// not run in one block: in the order of their rows' lengths they are dealt to the blocks there and back again (to block 0,
+// 1, 2 ..., the next ones ... 2, 1, 0), one per wave, so that all blocks hold about the same number of chunks.
+// Which chunks make up a stream, and the order in which a pair's streams are added, stay those of a block per
+// pair, whatever the other rows' lengths: so does every bit of the result.
+// Bound by the caches' bytes while all CUs have work: a block per pair leaves the chip to the longest rows at the end, and
+// CUs idle where there are fewer pairs.  Lengths from an eighth of the cache to all of it / from half / all equal,
+// us, a block per pair and this: 32 rows x 8 heads x 8192 138 / 152 / 177 and 121 / 152 / 179, 22 x 8 x 10624
+// 159 / 165 / 171 and 114 / 144 / 164, 20 x 8 x 3072 47 / 49 / 49 and 35 / 42 / 47, 24 x 8 x 2048 35 / 36 / 36 and 28 / 35
+// / 35; with 300 tokens in each row of 32 x 8 x 8192 11.1 and 11.1, with 100 6.7 and 6.7.
+// The hand-over and the waves that walk a long stream alone at the end cost about what three tenths of the longest
+// row's walk take (22 x 8 x 10624 with all rows full 171 us in blocks and 175 dealt): below that the pairs keep their
+// blocks.  (More pairs than CUs, several streams per wave: 64 x 8 x 4096 140 / 151 / 180 and 139 / 173 / 176, so they
+// keep their blocks too.)
+struct AttnDeal {
+    int len, rank;         // of the lane's row (batch <= 64), its place in the order of the lengths
+    int blocks, streams;   // blocks of the deal, streams per block
+    bool pays;             // the same in every wave of the launch
+};
+constexpr int kAttnPairWaves = 8;   // waves of a block that holds a pair by itself
+
+// A deal has no more blocks than CUs, all with the same number of streams but for the last places.
+__host__ __device__ __forceinline__ int attn_deal_streams(int pairs, int cus) { return (pairs * kAttnPairWaves + cus - 1) / cus; }
+__host__ __device__ __forceinline__ int attn_deal_blocks(int pairs, int cus) {
+    const int streams = attn_deal_streams(pairs, cus);
+    return (pairs * kAttnPairWaves + streams - 1) / streams;
 }
 
-// A block per (row, KV head) pair.
-template <int G, int D, int WAVES>
+__device__ __forceinline__ AttnDeal attn_deal(const int32_t* positions, int batch, int kvh, int max_seq, int cus, int lane) {
+    AttnDeal a;
+    a.len = lane < batch ? min(max(positions[lane], 0), max_seq - 1) + 1 : 0;
+    a.pays = false;
+    const int chunks = (a.len + 63) / 64;
+    if (__ballot(chunks >= 16) == 0) return a;   // short rows: nothing to win
+    int longest = chunks, total = chunks;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        longest = max(longest, __shfl_xor(longest, off, 64));
+        total += __shfl_xor(total, off, 64);
+    }
+    longest = __builtin_amdgcn_readfirstlane(longest);
+    const int pairs = batch * kvh, share = (int)((long long)__builtin_amdgcn_readfirstlane(total) * kvh / cus);
+    a.pays = 10 * (longest - share) >= 3 * longest + 48;
+    if (!a.pays) return a;
+    a.rank = 0;
+    for (int r = 0; r < batch; ++r) {
+        const int other = __builtin_amdgcn_readlane(a.len, r);
+        a.rank += other < a.len || (other == a.len && r < lane);
+    }
+    a.streams = attn_deal_streams(pairs, cus);
+    a.blocks = attn_deal_blocks(pairs, cus);
+    return a;
+}
+
+// DEAL: a block per share of the deal where that pays, and else per pair (splits is 1).
+template <int G, int D, int WAVES, bool DEAL>
 __global__ __launch_bounds__(WAVES * 64) void attn_decode_kernel(
     const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
-    const int32_t* __restrict__ positions, half_t* __restrict__ out, int kvh, int max_seq, float scale) {
-    const int g = blockIdx.y, b = blockIdx.z;
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i16 = lane & 15, kq = lane >> 4;
-    // Chunks of 64 positions (one tile of the V cache) are dealt round robin to the waves, whatever the length:
-    // a wave requests its first chunk before the position has arrived.
-    constexpr int stride = WAVES * 64;
-    const int c_first = wave * 64;
-    const int t1 = min(max(positions[b], 0), max_seq - 1) + 1;  // the new token has been appended
-
-    __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * kAttnPitch];
-    __shared__ __attribute__((aligned(16))) AttnMerge<G, D, WAVES> merge;
-
-    const size_t pair = (size_t)b * kvh + g;
-    const half_t* kbase = k_cache + pair * max_seq * D;
-    const half_t* vbase = vt_cache + pair * D * max_seq;
-    AttnWave<G, D> w;
-    w.load_q(q + pair * G * D, i16, kq);
-    w.reset();
-    auto load = [&](int c0) {
-        const size_t at = (size_t)min(c0, max_seq - 64) * D;   // a chunk past the cache is not used: any will do
-        w.load_chunk(kbase + at, vbase + at, i16, kq);
-    };
-    load(c_first);
-    // Two waves share a SIMD when a block has eight, and the older one wins every arbitration: the
-    // priority of a wave falls with the share of its chunks it has behind it, so that the four
-    // younger waves are not left to walk their last chunks alone.
-    const int n_chunks = t1 > c_first ? (t1 - c_first + stride - 1) / stride : 0;
-    int chunk_no = 0;
-    for (int c0 = c_first; c0 < t1;) {
-        set_priority_by_progress(chunk_no++, n_chunks);
-        w.step(p_s[wave], c0, t1, scale, i16, kq);
-        c0 += stride;
-        if (c0 < t1) load(c0);
-    }
-    merge.put(w, wave, i16, kq);
-    __syncthreads();
-
-    // merge the waves: thread -> (head, four dims)
-    const size_t head0 = pair * G;
-    const int h = tid / (D / 4), d = tid % (D / 4) * 4;
-    if (tid < merge.kItems) {
-        float mm, ll;
-        const float4_t a = merge.fold(h, d, mm, ll);
-        attn_store(out + (head0 + h) * D + d, a, ll);
-    }
-}
-
-// A pair over `splits` blocks of four waves.  The body stands on its own and not on AttnWave: the same walk written
-// over that struct compiles to loads of V held back into the softmax and takes 19.6 us against 18.3 in the decode
-// loop at batch 8 (asked for ahead of the softmax by a scheduling barrier: 20.0).
-template <int G, int D>
-__global__ __launch_bounds__(256) void attn_decode_split_kernel(
-    const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
     const int32_t* __restrict__ positions, half_t* __restrict__ out, float* partial, unsigned* counters,
-    int kvh, int max_seq, float scale, int splits) {
+    int batch, int kvh, int max_seq, float scale, int splits, int cus) {
     static_assert(D == 128 && G <= 16, "head size 128, at most 16 query heads per KV head");
-    constexpr int WAVES = 4, PP = kAttnPitch;
-    const int split = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+    constexpr int PP = 72;  // halfs per row of the P tile in LDS (64 + padding)
+    const int split = DEAL ? 0 : blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int i16 = lane & 15, kq = lane >> 4;
     // Chunks of 64 positions (one tile of the V cache) are dealt round robin, first over the
@@ -510,25 +327,49 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
     // wave requests its first chunk before the position has arrived, and no wave holds more
     // than one chunk over the others.
     const int stride = splits * WAVES * 64;
-    const int c_first = (split + wave * splits) * 64;
-    const int t1 = min(max(positions[b], 0), max_seq - 1) + 1;  // the new token has been appended
+    int pair, c_first, t1;
+    bool dealt = false;
+    if constexpr (DEAL) {
+        const int uwave = __builtin_amdgcn_readfirstlane(wave), block = blockIdx.x;
+        const AttnDeal deal = attn_deal(positions, batch, kvh, max_seq, cus, lane);
+        dealt = deal.pays;
+        int row, stream = uwave;
+        if (dealt) {
+            const int at = uwave * deal.blocks + ((uwave & 1) ? deal.blocks - 1 - block : block);
+            if (block >= deal.blocks || uwave >= deal.streams || at >= batch * kvh * WAVES) return;
+            const int place = at / WAVES, rank = place / kvh;
+            row = (int)__builtin_ctzll(__ballot(lane < batch && deal.rank == rank));
+            pair = row * kvh + place - rank * kvh;
+            stream = at - place * WAVES;
+        } else {
+            pair = block;
+            if (pair >= batch * kvh) return;
+            row = pair / kvh;
+        }
+        c_first = stream * 64;
+        t1 = __builtin_amdgcn_readlane(deal.len, row);
+    } else {
+        pair = (int)(blockIdx.z * kvh + blockIdx.y);
+        c_first = (split + wave * splits) * 64;
+        t1 = min(max(positions[blockIdx.z], 0), max_seq - 1) + 1;  // the new token has been appended
+    }
 
     __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * PP];
     __shared__ float m_s[WAVES][16], l_s[WAVES][16];
-    __shared__ float acc_s[WAVES][G][D];
+    __shared__ __attribute__((aligned(16))) float acc_s[WAVES][G][D];
 
     // A operand of S = Q K^T: row = head i16, k = dims s*32 + kq*8 .. +8
     uint4 qf[4];
     {
-        const half_t* qp = q + (((size_t)b * kvh + g) * G + min(i16, G - 1)) * D + kq * 8;
+        const half_t* qp = q + ((size_t)pair * G + min(i16, G - 1)) * D + kq * 8;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             qf[s] = *reinterpret_cast<const uint4*>(qp + s * 32);
             if (i16 >= G) qf[s] = make_uint4(0, 0, 0, 0);
         }
     }
-    const half_t* kbase = k_cache + ((size_t)b * kvh + g) * max_seq * D;
-    const half_t* vbase = vt_cache + ((size_t)b * kvh + g) * D * max_seq;
+    const half_t* kbase = k_cache + (size_t)pair * max_seq * D;
+    const half_t* vbase = vt_cache + (size_t)pair * D * max_seq;
 
     // rows of every accumulator tile held by this lane: heads kq*4 + r
     float m_run[4], l_run[4];
@@ -554,6 +395,8 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
 #pragma unroll
             for (int s = 0; s < 4; ++s) kf[pt][s] = *reinterpret_cast<const uint4*>(kp + s * 32);
         }
+        // (K ahead of V here, or the dealt launch is 3 to 7 % slower; the other instantiations keep that order unasked)
+        if constexpr (DEAL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             const int p0 = min(c0 + ks * 32 + kq * 8, max_seq - 8);
@@ -563,7 +406,15 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
         }
     };
     load_chunk(c_first);
+    // Two waves share a SIMD when a block has eight, and the older one wins every arbitration: the
+    // priority of a wave falls with the share of its chunks it has behind it, so that the four
+    // younger waves are not left to walk their last chunks alone.
+    const int n_chunks = t1 > c_first ? (t1 - c_first + stride - 1) / stride : 0;
+    int chunk_no = 0;
     for (int c0 = c_first; c0 < t1;) {
+        if constexpr (WAVES > 4) {
+            set_priority_by_progress(chunk_no++, n_chunks);
+        }
         // S tile pt: rows = heads kq*4 + r, column = position c0 + pt*16 + i16
         float4_t sc[4];
 #pragma unroll
@@ -653,31 +504,64 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
             }
         }
     }
+    if (DEAL && dealt) {
+        // The pair's streams end in different blocks: each leaves a record per head, the last to arrive adds them up.
+        // A wave by itself: no barrier, its own part of the LDS, and its stores acknowledged before it is counted.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        float* records = partial + (size_t)pair * WAVES * G * kAttnRecord;
+        float* mine = records + c_first / 64 * G * kAttnRecord;
+        for (int i = lane; i < G * D / 4; i += 64) {
+            const int h = i / (D / 4), d = i % (D / 4) * 4;
+            store_agent4(mine + h * kAttnRecord + d, *reinterpret_cast<const float4_t*>(&acc_s[wave][h][d]));
+        }
+        if (lane < G) store_agent4(mine + lane * kAttnRecord + D, float4_t{m_s[wave][lane], l_s[wave][lane], 0.f, 0.f});
+        __builtin_amdgcn_s_waitcnt(0);
+        unsigned before = 0;
+        if (lane == 0) before = __hip_atomic_fetch_add(counters + pair, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__builtin_amdgcn_readfirstlane(before) != WAVES - 1) return;
+        if (lane == 0) __hip_atomic_store(counters + pair, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int i = lane; i < G * D / 4; i += 64) {
+            const int h = i / (D / 4), d = i % (D / 4) * 4;
+            float ms[WAVES], ls[WAVES], mm, ll;
+            float4_t as[WAVES];
+#pragma unroll
+            for (int u = 0; u < WAVES; ++u) {
+                const float* r = records + (u * G + h) * kAttnRecord;
+                as[u] = load_agent4(r + d);
+                ms[u] = load_agent(r + D);
+                ls[u] = load_agent(r + D + 1);
+            }
+            wait_agent_loads(as);
+            const float4_t a = attn_fold_waves<WAVES>([&](int u) { return ms[u]; }, [&](int u) { return ls[u]; },
+                                                      [&](int u) { return as[u]; }, ll, mm);
+            attn_store(out + (size_t)pair * G * D + i * 4, a, ll);
+        }
+        return;
+    }
     __syncthreads();
 
     // merge the waves: thread -> (head, four dims)
     constexpr int REC = kAttnRecord, ITEMS = G * D / 4;  // <= 256
-    const size_t head0 = ((size_t)b * kvh + g) * G;
+    const size_t head0 = (size_t)pair * G;
     const int h = tid / (D / 4), d = tid % (D / 4) * 4;
     if (tid < ITEMS) {
-        float mm = m_s[0][h];
-#pragma unroll
-        for (int w = 1; w < WAVES; ++w) mm = fmaxf(mm, m_s[w][h]);
-        float ll = 0.f;
-        float4_t a = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const float f = (m_s[w][h] == -INFINITY) ? 0.f : expf(m_s[w][h] - mm);
-            ll += l_s[w][h] * f;
-            a += *reinterpret_cast<const float4_t*>(&acc_s[w][h][d]) * f;
+        float mm, ll;
+        const float4_t a = attn_fold_waves<WAVES>([&](int u) { return m_s[u][h]; }, [&](int u) { return l_s[u][h]; },
+                                                  [&](int u) { return *reinterpret_cast<const float4_t*>(&acc_s[u][h][d]); }, ll, mm);
+        if (DEAL || splits == 1) {
+            attn_store(out + (head0 + h) * D + d, a, ll);
+        } else {
+            float* pp = partial + ((head0 + h) * splits + split) * REC;
+            store_agent4(pp + d, a);
+            if (d == 0) store_agent4(pp + D, float4_t{mm, ll, 0.f, 0.f});
         }
-        float* pp = partial + ((head0 + h) * splits + split) * REC;
-        store_agent4(pp + d, a);
-        if (d == 0) store_agent4(pp + D, float4_t{mm, ll, 0.f, 0.f});
     }
+    if (DEAL || splits == 1) return;
 
     __shared__ int is_last;
-    if (!arrive_and_check_last(counters + (size_t)b * kvh + g, (unsigned)splits, &is_last)) return;
+    if (!arrive_and_check_last(counters + pair, (unsigned)splits, &is_last)) return;
     // Last block: merge the splits.  Every thread folds the splits of its four
     // output elements with the running-maximum recurrence, reading each split's
     // maximum, sum and partial values itself: the loads of up to 16 splits are
@@ -711,121 +595,7 @@ __global__ __launch_bounds__(256) void attn_decode_split_kernel(
                 }
             }
         }
-        const half4_t o = {(half_t)(a[0] / ll), (half_t)(a[1] / ll), (half_t)(a[2] / ll), (half_t)(a[3] / ll)};
-        *reinterpret_cast<half4_t*>(out + (head0 + h) * D + d) = o;
-    }
-}
-
-// The same for rows of different lengths: the chunks of all pairs stand in one line (pair after pair),
-// and every block takes an equal piece of it, whatever pairs it holds.
-// Bound by the caches' bytes; a block per (row, KV head) pair leaves the chip to the longest rows at the
-// end.  32 rows of a 8192-entry cache, lengths from an eighth of it to all: 150 -> 131 us (5.2 TB/s; 180 us =
-// 6.0 TB/s with all rows full).  What a block needs to know, it works out from the lengths by itself: every
-// wave holds them one row per lane and adds them up across the lanes.  A pair that one block holds whole is
-// finished there; of a pair that several share, each leaves a record and the last to arrive adds them up.
-// At the end of a pair a wave requests its first chunk of the next one before the waves meet.
-template <int G, int D, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, 2) void attn_decode_balanced_kernel(
-    const half_t* __restrict__ q, const half_t* __restrict__ k_cache, const half_t* __restrict__ vt_cache,
-    const int32_t* __restrict__ positions, half_t* __restrict__ out, float* partial, unsigned* counters, int batch,
-    int kvh, int max_seq, float scale) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i16 = lane & 15, kq = lane >> 4;
-    __shared__ __attribute__((aligned(16))) half_t p_s[WAVES][16 * kAttnPitch];
-    __shared__ __attribute__((aligned(16))) AttnMerge<G, D, WAVES> merge;
-    __shared__ int is_last;
-
-    // lane r: row r (batch <= 64): its length, and where its chunks end in the line
-    const int len = lane < batch ? min(max(positions[lane], 0), max_seq - 1) + 1 : 0;
-    const int mine = (len + 63) / 64 * kvh;
-    int upto = mine;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int v = __shfl_up(upto, off, 64);
-        if (lane >= off) upto += v;
-    }
-    const int total = __builtin_amdgcn_readlane(upto, 63);
-    // a block takes one chunk per wave or more: where the rows are short, blocks are left without work
-    const int blocks = min((int)gridDim.x, (total + WAVES - 1) / WAVES);
-    if ((int)blockIdx.x >= blocks) return;
-    auto first_of = [&](int block) { return (int)((long long)total * block / blocks); };
-    auto block_of = [&](int chunk) { return (int)((((long long)chunk + 1) * blocks - 1) / total); };
-    const int begin = first_of(blockIdx.x), end = first_of(blockIdx.x + 1);
-
-    // piece of a pair in the block's part of the line
-    struct Piece {
-        int pair, start, stop, t1;   // pair, the line's chunks start .. stop of it, its length
-    };
-    auto piece_at = [&](int chunk) {
-        Piece p;
-        const int b = __popcll(__ballot(upto <= chunk));
-        const int n = __builtin_amdgcn_readlane(mine, b) / kvh;
-        const int row0 = __builtin_amdgcn_readlane(upto, b) - n * kvh;
-        const int g = (chunk - row0) / n;
-        p.pair = b * kvh + g;
-        p.start = row0 + g * n;
-        p.stop = p.start + n;
-        p.t1 = __builtin_amdgcn_readlane(len, b);
-        return p;
-    };
-    AttnWave<G, D> w;
-    // chunk c of the line belongs to wave (c - begin) % WAVES: over the whole block no wave holds more
-    // than one chunk over the others
-    int c = begin + wave;
-    Piece p = piece_at(begin);
-    auto request = [&] {   // the wave's next chunk, if it lies in piece p
-        if (c >= min(end, p.stop)) return;
-        const size_t at = ((size_t)p.pair * max_seq + (size_t)(c - p.start) * 64) * D;
-        w.load_chunk(k_cache + at, vt_cache + at, i16, kq);
-    };
-    w.load_q(q + (size_t)p.pair * G * D, i16, kq);
-    request();
-    w.reset();
-    const int h = tid / (D / 4), d = tid % (D / 4) * 4;
-    const int n_chunks = (end - begin - wave + WAVES - 1) / WAVES;
-    int chunk_no = 0;
-    for (;;) {
-        const int stop = min(end, p.stop);
-        if (c < stop) {
-            if constexpr (WAVES > 4) set_priority_by_progress(chunk_no++, n_chunks);
-            w.step(p_s[wave], (c - p.start) * 64, p.t1, scale, i16, kq);
-            c += WAVES;
-        }
-        const Piece now = p;
-        if (c >= stop && stop < end) {
-            // what the next pair needs is requested before this one's sums meet
-            p = piece_at(stop);
-            w.load_q(q + (size_t)p.pair * G * D, i16, kq);
-        }
-        request();
-        if (c < stop) continue;
-        merge.put(w, wave, i16, kq);
-        w.reset();
-        __syncthreads();
-        const int first = block_of(now.start), last = block_of(now.stop - 1);
-        half_t* op = out + ((size_t)now.pair * G + h) * D + d;
-        if (tid < G * D / 4) {
-            float mm, ll;
-            const float4_t a = merge.fold(h, d, mm, ll);
-            if (first == last) {
-                attn_store(op, a, ll);
-            } else {
-                // two records per block: of the pair it begins with, and of the one it ends in
-                float* pp = partial + (((size_t)blockIdx.x * 2 + (now.start > begin)) * G + h) * kAttnRecord;
-                store_agent4(pp + d, a);
-                if (d == 0) store_agent4(pp + D, float4_t{mm, ll, 0.f, 0.f});
-            }
-        }
-        if (first != last && arrive_and_check_last(counters + now.pair, (unsigned)(last - first + 1), &is_last) &&
-            tid < G * D / 4) {
-            const int slot = now.start > first_of(first);
-            // (four records at a time: the next pair's chunk is in registers already)
-            attn_fold_records<4>(op, d, last - first + 1, [&](int i) {
-                return partial + (((size_t)(first + i) * 2 + (i == 0 ? slot : 0)) * G + h) * kAttnRecord;
-            });
-        }
-        if (stop >= end) break;
-        __syncthreads();   // the sums' LDS is written again
+        attn_store(out + (head0 + h) * D + d, a, ll);
     }
 }
 
@@ -886,32 +656,21 @@ static int attn_splits(int n_kv_heads, int max_seq, int batch) {
 }
 static int attn_splits(const Llama& m, int batch) { return attn_splits(m.cfg.n_kv_heads, m.cfg.max_seq, batch); }
 
-// Whether the blocks share the chunks of all rows evenly (attn_decode_balanced_kernel) instead of taking one
-// row's each.  The lengths are on the device, so the line is drawn by what the cache could hold, in chunks
-// per block.  The walk costs 3 to 6 us more than a block of its own (lengths read first, sums meeting
-// across blocks), and wins back what the longest row keeps the other blocks waiting.  Measured with lengths
-// from an eighth of the cache to all of it / from half / all equal, this kernel against the even deal, us:
-// 48 rows x 4 heads x 4096 (48 chunks) 52 / 60 / 76 against 67 / 69 / 75; 32 x 8 x 8192 (128) 131 / 147 / 181
-// against 150 / 162 / 180; below it 32 x 8 x 2048 (32) 38 / 48 / 51 against 39 / 44 / 49.  Where the even deal
-// has to meet across blocks as well (splits > 1) the line is lower: 8 x 8 x 8192 (32) 35 / 46 / 53 against
-// 43 / 50 / 55, 16 x 8 x 2048 (16) 21 / 29 / 32 against 25 / 28 / 30; below it 8 x 8 x 2112 (8) 19 / 21 / 20
-// against 19 / 20 / 21, 4 x 8 x 2048 (4) 18 / 18 / 15 against 10 / 12 / 13.
-static bool attn_balanced(int n_kv_heads, int max_seq, int batch) {
+// Whether the streams of rows of different lengths may be dealt to the blocks (attn_deal): a block per pair otherwise, no
+// more pairs than CUs, and a cache that can hold rows for which it pays (32 rows x 8 heads of 1 to 1024 entries
+// 20.6 us with a block per pair and 22.3 dealt, of 1 to 2048 35.3 and 34.6).
+constexpr int kAttnDealChunks = 32;
+static bool attn_dealt(int n_kv_heads, int max_seq, int batch) {
     if (batch < 2 || batch > 64) return false;   // a lane per row holds its length
-    const long long chunks = (long long)batch * n_kv_heads * (max_seq / kVTile);
-    return chunks >= (long long)compute_units() * (attn_splits(n_kv_heads, max_seq, batch) > 1 ? 16 : 48);
+    return attn_splits(n_kv_heads, max_seq, batch) == 1 && batch * n_kv_heads <= compute_units() &&
+           max_seq / kVTile >= kAttnDealChunks;
 }
-static size_t attn_record_bytes(int batch, int n_q_heads, int n_kv_heads, int max_seq, bool balanced) {
-    const size_t heads = balanced ? (size_t)2 * compute_units() * (n_q_heads / n_kv_heads)
-                                  : (size_t)batch * n_q_heads * attn_splits(n_kv_heads, max_seq, batch);
+static size_t attn_record_bytes(int batch, int n_q_heads, int n_kv_heads, int max_seq, bool dealt) {
+    const size_t heads = (size_t)batch * n_q_heads * (dealt ? kAttnPairWaves : attn_splits(n_kv_heads, max_seq, batch));
     return align_up(heads * kAttnRecord * sizeof(float));
 }
-// Records of whichever kernel the shape runs; never less than the even deal needs.
 static size_t attn_record_bytes(int batch, int n_q_heads, int n_kv_heads, int max_seq) {
-    const size_t even = attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq, false);
-    if (!attn_balanced(n_kv_heads, max_seq, batch)) return even;
-    const size_t balanced = attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq, true);
-    return balanced > even ? balanced : even;
+    return attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq, attn_dealt(n_kv_heads, max_seq, batch));
 }
 
 // Workspace of a stand-alone attention call: arrival counters (one per row and KV
@@ -924,17 +683,19 @@ static size_t attn_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int
 template <int G>
 static void launch_attn_raw(hipStream_t st, const half_t* q, const half_t* k_cache, const half_t* vt_cache,
                             const int32_t* positions, half_t* out, float* partial, unsigned* counters, int batch,
-                            int n_kv_heads, int max_seq, int splits, bool balanced) {
+                            int n_kv_heads, int max_seq, int splits, bool dealt) {
     const float scale = 1.0f / sqrtf(128.f);
-    if (balanced)
-        hipLaunchKernelGGL((attn_decode_balanced_kernel<G, 128, 8>), dim3(compute_units()), dim3(512), 0, st, q, k_cache,
-                           vt_cache, positions, out, partial, counters, batch, n_kv_heads, max_seq, scale);
+    const int pairs = batch * n_kv_heads, cus = compute_units(), threads = kAttnPairWaves * 64;
+    if (dealt)
+        hipLaunchKernelGGL((attn_decode_kernel<G, 128, kAttnPairWaves, true>), dim3(std::max(pairs, attn_deal_blocks(pairs, cus))),
+                           dim3(threads), 0, st, q, k_cache, vt_cache, positions, out, partial, counters, batch, n_kv_heads,
+                           max_seq, scale, 1, cus);
     else if (splits == 1)
-        hipLaunchKernelGGL((attn_decode_kernel<G, 128, 8>), dim3(1, n_kv_heads, batch), dim3(512), 0, st, q, k_cache,
-                           vt_cache, positions, out, n_kv_heads, max_seq, scale);
+        hipLaunchKernelGGL((attn_decode_kernel<G, 128, kAttnPairWaves, false>), dim3(1, n_kv_heads, batch), dim3(threads), 0, st,
+                           q, k_cache, vt_cache, positions, out, partial, counters, batch, n_kv_heads, max_seq, scale, 1, cus);
     else
-        hipLaunchKernelGGL((attn_decode_split_kernel<G, 128>), dim3(splits, n_kv_heads, batch), dim3(256), 0, st, q,
-                           k_cache, vt_cache, positions, out, partial, counters, n_kv_heads, max_seq, scale, splits);
+        hipLaunchKernelGGL((attn_decode_kernel<G, 128, 4, false>), dim3(splits, n_kv_heads, batch), dim3(256), 0, st, q,
+                           k_cache, vt_cache, positions, out, partial, counters, batch, n_kv_heads, max_seq, scale, splits, cus);
 }
 
 static Scratch carve(const Llama& m, int batch, char* base) {
@@ -988,7 +749,7 @@ static void launch_attn(hipStream_t st, const Llama& m, const Scratch& s, const 
     const mh_llama_config& c = m.cfg;
     launch_attn_raw<G>(st, s.q, (const half_t*)L.k_cache, (const half_t*)L.v_cache, positions, s.attn, s.attn_partial,
                        s.attn_counters, batch, c.n_kv_heads, c.max_seq, splits,
-                       attn_balanced(c.n_kv_heads, c.max_seq, batch));
+                       attn_dealt(c.n_kv_heads, c.max_seq, batch));
 }
 
 }  // namespace mh
@@ -1016,10 +777,10 @@ int mh_attn_decode(mh_stream_t stream, const void* q, const void* k_cache, const
     MH_REQUIRE(max_seq >= kVTile && max_seq % kVTile == 0, "mh_attn_decode: max_seq must be a multiple of 64, got %d", max_seq);
     MH_REQUIRE(((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)vt_cache | (uintptr_t)out) % 16 == 0,
                "mh_attn_decode: operands must be 16-byte aligned");
-    // a workspace that holds the even deal's records alone gets the even deal
+    // a workspace without room for a record per stream gets a block per pair, with the same results
     const size_t need = attn_counter_bytes(batch, n_kv_heads) + attn_record_bytes(batch, n_q_heads, n_kv_heads, max_seq, false);
-    const bool balanced = attn_balanced(n_kv_heads, max_seq, batch) &&
-                          workspace_bytes >= attn_workspace_bytes(batch, n_q_heads, n_kv_heads, max_seq);
+    const bool dealt = attn_dealt(n_kv_heads, max_seq, batch) &&
+                       workspace_bytes >= attn_workspace_bytes(batch, n_q_heads, n_kv_heads, max_seq);
     if (workspace == nullptr || workspace_bytes < need)
         return fail(MH_ERR_WORKSPACE, "mh_attn_decode: workspace of %zu bytes required, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
@@ -1030,7 +791,7 @@ int mh_attn_decode(mh_stream_t stream, const void* q, const void* k_cache, const
     hipStream_t st = as_stream(stream);
 #define MH_ATTN(G)                                                                                                 \
     launch_attn_raw<G>(st, (const half_t*)q, (const half_t*)k_cache, (const half_t*)vt_cache, positions, (half_t*)out, \
-                       partial, counters, batch, n_kv_heads, max_seq, splits, balanced)
+                       partial, counters, batch, n_kv_heads, max_seq, splits, dealt)
     switch (g) {
         case 1: MH_ATTN(1); break;
         case 2: MH_ATTN(2); break;

@@ -1,4 +1,5 @@
-"""Decode attention whose blocks share the chunks of all rows evenly, against float64."""
+"""Decode attention over rows of different lengths, against float64, and bit for bit whatever the neighbours' lengths:
+several blocks per (row, KV head) pair, a block per pair, and pairs whose streams are dealt to the blocks by length."""
 import numpy as np
 import pytest
 import torch
@@ -19,8 +20,8 @@ def _reference(q, k, vt, positions, kvh):
     return out
 
 
-# (rows, KV heads, query heads per KV head, cache, lengths): pairs that blocks share, pairs within one block,
-# one chunk, the cache's ends and positions outside it, the most rows a wave holds
+# (rows, KV heads, query heads per KV head, cache, lengths): pairs over several blocks, a dealt launch (48 x 4 pairs), more
+# pairs than CUs, one chunk, the cache's ends and positions outside it, the most rows a wave holds
 CASES = [
     (2, 16, 1, 16384, [0, 16383]),
     (2, 16, 2, 16384, [-7, 20000]),
@@ -69,3 +70,50 @@ def test_balanced_attention(hip, rows, kvh, g, seq, positions):
         # weights rounded to fp16 (2^-12 relative on average) and the fp16 result: 2.7e-4 measured, as by the even deal
         rel = ((outs[0].double() - want).norm() / want.norm()).item()
         assert rel <= 1e-3, rel
+
+
+def _normal(gen, *shape):
+    return torch.empty(shape, dtype=torch.float16, device="cuda").normal_(generator=gen)
+
+
+# Pairs that fill the CUs, leave the last places of the deal empty (13 x 10, 17 x 8: six and five streams per block), one
+# KV head, two rows, 64 rows; the rows that are looked at stand first, in the middle and last
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,kvh,g,seq", [(32, 8, 8, 2048), (17, 8, 4, 4096), (13, 10, 2, 3072), (2, 128, 1, 2048),
+                                            (64, 4, 8, 2048), (8, 8, 8, 8192), (40, 8, 1, 2048)])
+def test_bits_do_not_depend_on_the_neighbours(hip, rows, kvh, g, seq):
+    """A row's result is the same whether its neighbours are as long, far shorter or of all lengths, and whatever room
+    the workspace has."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + seq)
+    q, k, vt = _normal(gen, rows, kvh * g, D), _normal(gen, rows, kvh, seq, D), _normal(gen, rows, kvh, seq // 64, D, 64)
+    mixed = np.random.default_rng(rows).integers(seq // 8, seq, rows)
+    mixed[0], mixed[-1] = seq - 1, 70
+    shape = (rows, kvh * g, kvh, D, seq)
+    full = hip.call("mh_attn_decode_workspace_bytes", *shape)
+    splits = max(1, min((seq // 64 + 3) // 4, 256 // (rows * kvh), 64))
+    align = lambda n: (n + 255) // 256 * 256
+    least = align(rows * kvh * 4) + align(rows * kvh * g * splits * (D + 4) * 4)
+
+    def run(positions, nbytes):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device="cuda")
+        pos = torch.tensor(positions, dtype=torch.int32, device="cuda")
+        out = torch.full((rows, kvh * g, D), float("nan"), dtype=torch.float16, device="cuda")
+        torch.cuda.synchronize()
+        for _ in range(2):   # the counters are left as they were found
+            hip.call("mh_attn_decode", None, q.data_ptr(), k.data_ptr(), vt.data_ptr(), pos.data_ptr(), out.data_ptr(), *shape,
+                     ws.data_ptr(), nbytes)
+        torch.cuda.synchronize()
+        assert int(ws[:rows * kvh * 4].count_nonzero()) == 0
+        return out
+
+    got = run(mixed, full)
+    want = _reference(q, k, vt, mixed, kvh)
+    rel = ((got.double() - want).norm() / want.norm()).item()
+    assert rel <= 1e-3, rel   # as above
+    assert torch.equal(got, run(mixed, least))
+    for row in (0, rows // 2, rows - 1):
+        for neighbours in (int(mixed[row]), 63):
+            positions = np.full(rows, neighbours)
+            positions[row] = mixed[row]
+            assert torch.equal(got[row], run(positions, full)[row]), (row, neighbours)
