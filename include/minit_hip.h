@@ -146,15 +146,16 @@ int mh_gptq_linear(mh_stream_t stream, const void* x, const int32_t* qweight, co
  * workspace: code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc.  The first call on a device looks up the address of the
  * built-in buffer (hipGetSymbolAddress), which a stream capture must not record:
- * make that call outside any capture (a call under capture before it fails with
- * MH_ERR_INVALID and records nothing); every later call may be captured.  No counterpart in the reference (its fused product
+ * make that call outside any capture (a call under capture before it that needs the
+ * buffer fails with MH_ERR_INVALID and records nothing); every later call may be captured.  No counterpart in the reference (its fused product
  * accumulates with atomics into a zeroed output and needs no scratch,
  * examples/qwen1_5_int8.py:198,263).  Same arguments and results as
  * mh_gptq_matmul without the workspace pair: the split-K counters and partial
  * sums live in a buffer of MH_GPTQ_STATIC_SCRATCH_BYTES that the library holds
  * in device memory on every GPU it runs on until the process ends.  The call
- * allocates and frees nothing.  A shape whose mh_gptq_workspace_bytes exceeds
- * that size is rejected with MH_ERR_WORKSPACE.  Every call on a GPU uses that
+ * allocates and frees nothing.  A shape whose partial sums exceed that size is
+ * rejected with MH_ERR_WORKSPACE, unless they only serve the last pass over more
+ * tiles than CUs (M > 64, which runs in whole tiles then: sums in another order).  Every call on a GPU uses that
  * GPU's one buffer (of the device that is current at the call): calls that
  * overlap on one GPU -- different streams, or threads -- race on it and give
  * wrong sums; calls ordered on one stream are safe. */

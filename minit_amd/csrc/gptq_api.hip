@@ -12,6 +12,7 @@ int gptq_gemv_launch(hipStream_t stream, const void* x, const int32_t* qweight, 
                      void* workspace, size_t workspace_bytes);
 bool gemm_supported(int M, int N, int K, int group_size, int bits);
 size_t gemm_workspace_bytes(int M, int N, int K, int group_size, int bits);
+size_t gemm_least_workspace_bytes(int M, int N, int K, int group_size, int bits);
 bool gemm_silu_pairs_supported(int M, int N, int K, int group_size, int bits);
 bool gemm_tall_silu_pairs_supported(int M, int N, int K, int group_size, int bits);
 int gptq_gemm_launch(hipStream_t stream, const void* x, const int32_t* qweight, const int32_t* qzeros,
@@ -80,8 +81,9 @@ __global__ void static_scratch_clear_kernel(uint4* p, int n16) {
 }
 
 // The current device's copy of `scratch` (looked up on first use on that device).  The lookup loads
-// the code object's symbol table: not something to do while `stream` is being captured.
-static int static_scratch_pointer(hipStream_t stream, void** out) {
+// the code object's symbol table: not something to do while `stream` is being captured; a caller that can do
+// without the buffer (optional) gets none then.
+static int static_scratch_pointer(hipStream_t stream, bool optional, void** out) {
     int dev = 0;
     MH_CHECK_HIP(hipGetDevice(&dev));
     MH_REQUIRE(dev >= 0 && dev < kStaticMaxDevices, "mh_gptq_matmul_static: device index %d out of range", dev);
@@ -93,6 +95,7 @@ static int static_scratch_pointer(hipStream_t stream, void** out) {
         if (stream != nullptr && hipStreamIsCapturing(stream, &capturing) == hipSuccess &&
             capturing != hipStreamCaptureStatusNone) {
             pthread_mutex_unlock(&g_static_lock);
+            if (optional) return MH_OK;
             return fail(MH_ERR_INVALID, "mh_gptq_matmul_static: the first call on a device must be made outside a "
                                         "stream capture (it looks up the built-in buffer's address)");
         }
@@ -113,22 +116,35 @@ extern "C" {
 
 size_t mh_gptq_static_scratch_bytes(void) { return kStaticScratchBytes; }
 
+// As mh_gptq_workspace_bytes, without what a kernel only takes if it finds it.
+static size_t least_workspace_bytes(int M, int N, int K, int group_size, int bits) {
+    size_t a = 0, b = 0;
+    if (gemv_supported(M, N, K, group_size, bits)) a = gemv_workspace_bytes(M, N, K, group_size, bits);
+    if (gemm_supported(M, N, K, group_size, bits)) b = gemm_least_workspace_bytes(M, N, K, group_size, bits);
+    return a > b ? a : b;
+}
+
 int mh_gptq_matmul_static(mh_stream_t stream, const void* x, const int32_t* qweight, const int32_t* qzeros,
                           const void* scales, const int32_t* g_idx, void* out, int M, int N, int K,
                           int group_size, int bits) {
     int rc = check_gptq_args("mh_gptq_matmul_static", x, qweight, qzeros, scales, out, M, N, K, group_size, bits);
     if (rc) return rc;
     if (M == 0) return MH_OK;
+    // (a last pass in K ranges takes the room it finds: what counts against the buffer is what the product cannot
+    // do without)
     const size_t need = g_idx == nullptr ? mh_gptq_workspace_bytes(M, N, K, group_size, bits) : 0;
-    if (need > kStaticScratchBytes)
+    const size_t least = need > 0 ? least_workspace_bytes(M, N, K, group_size, bits) : 0;
+    if (least > kStaticScratchBytes)
         return fail(MH_ERR_WORKSPACE,
                     "mh_gptq_matmul_static: M=%d N=%d K=%d needs %zu bytes of split-K scratch, the built-in buffer "
                     "holds %zu; use mh_gptq_matmul with a caller-owned workspace",
-                    M, N, K, need, kStaticScratchBytes);
+                    M, N, K, least, kStaticScratchBytes);
     void* ws = nullptr;
-    if (need != 0) {
-        rc = static_scratch_pointer(as_stream(stream), &ws);
+    if (need != 0 && (least != 0 || need <= kStaticScratchBytes)) {
+        rc = static_scratch_pointer(as_stream(stream), least == 0, &ws);
         if (rc) return rc;
+    }
+    if (ws != nullptr) {
         // the arrival counters must start at zero; the buffer keeps whatever the previous call (or a call
         // that was interrupted) left, so clear them with a kernel (no memset node, safe under graph capture)
         const int n16 = (int)(kTileCounterBytes / 16);

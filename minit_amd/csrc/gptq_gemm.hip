@@ -852,6 +852,7 @@ int gptq_gemm_wide_launch(hipStream_t stream, const void* x, const int32_t* qwei
 // gptq_gemm_tall.hip: blocks of 128 rows, weights dequantised in registers, K sliced over the waves
 bool gemm_tall_preferred(int M, int N, int K, int group_size, int bits, int epilogue);
 size_t gemm_tall_workspace_bytes(int M, int N, int K, int bits);
+size_t gemm_tall_least_workspace_bytes(int M, int N, int K, int bits);
 bool gemm_tall_silu_pairs_supported(int M, int N, int K, int group_size, int bits);
 int gptq_gemm_tall_launch(hipStream_t stream, const void* x, const int32_t* qweight, const int32_t* qzeros,
                           const void* scales, void* out, int M, int N, int K, int group_size, int bits, void* workspace,
@@ -1081,6 +1082,13 @@ size_t gemm_workspace_bytes(int M, int N, int K, int group_size, int bits) {
     const size_t cols = M <= kSmallMaxM ? gemm_cols_workspace_bytes(M, N, K) : 0;
     const size_t fused = small > cols ? small : cols;
     return fused > tall ? fused : tall;
+}
+
+// The part of gemm_workspace_bytes() that a plain product is refused without.
+size_t gemm_least_workspace_bytes(int M, int N, int K, int group_size, int bits) {
+    if (M > kSmallMaxM && gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone))
+        return gemm_tall_least_workspace_bytes(M, N, K, bits);
+    return gemm_workspace_bytes(M, N, K, group_size, bits);
 }
 
 template <int BITS, int MT>

@@ -774,6 +774,10 @@ static size_t tall_plan_bytes(const TallPlan& p, int M, int N) {
 }
 
 size_t gemm_tall_workspace_bytes(int M, int N, int K, int bits) { return tall_plan_bytes(plan_tall(M, N, K, bits), M, N); }
+// What a launch cannot do without: the sums of a last pass in ranges are optional (whole tiles need no room).
+size_t gemm_tall_least_workspace_bytes(int M, int N, int K, int bits) {
+    return tall_plan_bytes(plan_tall(M, N, K, bits, false), M, N);
+}
 
 // kEpilogueSiluPairs in the kernel's own store: an unsplit plan, whole blocks of 128 + 128 columns.
 bool gemm_tall_silu_pairs_supported(int M, int N, int K, int group_size, int bits) {

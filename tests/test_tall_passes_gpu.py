@@ -67,3 +67,23 @@ def test_last_pass_in_ranges(hip, m, k, n, bits):
             pairs = out.double().reshape(m, n // 256, 2, 128)   # 128 gate and 128 up columns per block
             gate, up = pairs[:, :, 0], pairs[:, :, 1]
             close(act, (gate * torch.sigmoid(gate) * up).reshape(m, n // 2), "silu")
+
+
+@pytest.mark.parametrize("m,k,n", [(1537, 5120, 5120), (800, 4096, 28672), (1000, 2688, 5120)])
+def test_static_entry_serves_prompts(hip, m, k, n):
+    """The ranges' sums against the built-in buffer of the entry that takes no workspace: more than it holds (the first two:
+    whole tiles, the bits of a call without a workspace) or less (the third: the bits of a call with one)."""
+    weight, g = _weights(k, n, 128, 4, m)
+    x = torch.empty((m, k), dtype=torch.float16, device="cuda").normal_(generator=g)
+    args = (m, n, k, 128, 4)
+    need, limit = hip.call("mh_gptq_workspace_bytes", *args), hip.call("mh_gptq_static_scratch_bytes")
+    assert (need <= limit) == (m == 1000)
+    room = need if need <= limit else 0
+    ws = torch.zeros(max(room, 256), dtype=torch.uint8, device="cuda")
+    got, want = (torch.full((m, n), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    operands = (x.data_ptr(), *(t.data_ptr() for t in weight), None)
+    hip.call("mh_gptq_matmul_static", None, *operands, got.data_ptr(), *args)
+    hip.call("mh_gptq_matmul", None, *operands, want.data_ptr(), *args, ws.data_ptr(), room)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and bool(torch.isfinite(got).all())
