@@ -684,6 +684,9 @@ __global__ void gather_columns_kernel(const T* __restrict__ x, const int32_t* __
 // the columns from there, eight per thread and store; bound by the rows' bytes: 1000 x 13696 57 -> 10.2 us, 1000 x
 // 5120 15.5 -> 4.8, 4096 x 8192 123 -> 22 (6.1 TB/s).  (Parked rows at 16 x 5120 took 0.6 us longer than the
 // plain kernel on operands that come from HBM; two or four rows behind one read of the index measured the same.)
+// A workgroup per row is too much for many narrow rows, and a launch has room for 2^24 of them (2^32 threads): those stay
+// with the plain kernel (us, plain / here: 65536 x 256 41.9 / 38.1, x 128 16.2 / 30.6, x 64 9.7 / 30.4, a million
+// rows of 8 10.9 / 428; 16384 x 384 13.0 / 10.3, x 256 9.4 / 9.9; 4096 rows of any width 4 / 4).
 __global__ __launch_bounds__(256) void gather_columns_few_kernel(const uint16_t* __restrict__ x, const int4* __restrict__ index,
                                                                  uint2* __restrict__ out, int cols) {
     const int p = blockIdx.x * 256 + threadIdx.x;
@@ -838,7 +841,8 @@ int mh_gather_columns(mh_stream_t stream, const void* x, const int32_t* index, v
     MH_REQUIRE(x && index && out, "mh_gather_columns: null pointer");
     MH_REQUIRE(x != out, "mh_gather_columns: not in place");
     MH_REQUIRE(cols <= 0x7fffffffu, "mh_gather_columns: too many columns");
-    if ((dtype == MH_F16 || dtype == MH_BF16) && cols % 8 == 0 && cols * 2 <= kGatherLds && rows <= 0x7fffffffu &&
+    if ((dtype == MH_F16 || dtype == MH_BF16) && cols % 8 == 0 && cols * 2 <= kGatherLds && (cols >= 384 || rows <= 4096) &&
+        rows < ((size_t)1 << 24) &&
         ((uintptr_t)x | (uintptr_t)index | (uintptr_t)out) % 16 == 0) {
         if (rows * cols < ((size_t)1 << 20) && rows <= 65535)   // 128 x 5120 3.7 us against 4.0, 100 x 28672 12.4 / 9.1
             hipLaunchKernelGGL(gather_columns_few_kernel, dim3((unsigned)((cols / 4 + 255) / 256), (unsigned)rows), dim3(256), 0,
