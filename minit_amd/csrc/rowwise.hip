@@ -592,10 +592,11 @@ template <typename T, bool CAUSAL>
 static int softmax_t(hipStream_t st, const void* in, void* out, size_t a, size_t b, size_t c, size_t s,
                      size_t offset, float scale) {
     const bool aligned = rows_vector_path(in, out, b, c, sizeof(T));
-    // rows of any length and alignment that a group of threads can hold
-    const bool ragged = !aligned && c == 1 && sizeof(T) == 2 && b >= kRowVec && rows_fit_registers(b);
+    const int lanes = rows_lanes(b, 3072);
+    // rows of any length and alignment that a group of threads can hold, as many as a launch has threads for (2^32)
+    const bool ragged = !aligned && c == 1 && sizeof(T) == 2 && b >= kRowVec && rows_fit_registers(b) &&
+                        rows_grid(a, lanes) < (1u << 24);
     if (aligned || ragged) {
-        const int lanes = rows_lanes(b, 3072);
 #define MH_SOFTMAX_ROWS(LANES, CHUNKS)                                                                                \
     if (ragged)                                                                                                       \
         hipLaunchKernelGGL((softmax_rows_kernel<T, CAUSAL, true, LANES, CHUNKS>), dim3(rows_grid(a, LANES)),            \
