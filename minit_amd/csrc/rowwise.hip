@@ -561,12 +561,18 @@ static unsigned rows_grid(size_t a, int lanes) {
     const size_t per = kRowThreads / lanes;
     return (unsigned)((a + per - 1) / per);
 }
+// Whether one launch has threads for all rows (2^32, beyond which the grid wraps): `wide` of the workgroups of
+// kWideThreads threads per row, else groups of `lanes`.
+static bool rows_fit_launch(size_t a, int lanes, bool wide) {
+    return (wide ? a * kWideThreads : (size_t)rows_grid(a, lanes) * kRowThreads) >> 32 == 0;
+}
 
 template <typename T>
 static int rms_norm_t(hipStream_t st, const void* in, const void* weight, void* out, size_t a, size_t b,
                       size_t c, float eps) {
-    if (rows_vector_path(in, out, b, c, sizeof(T)) && (uintptr_t)weight % 16 == 0) {
-        const int lanes = rows_lanes(b, 2048);
+    const int lanes = rows_lanes(b, 2048);
+    if (rows_vector_path(in, out, b, c, sizeof(T)) && (uintptr_t)weight % 16 == 0 &&
+        rows_fit_launch(a, lanes, !rows_fit_registers(b))) {
 #define MH_RMS_ROWS(LANES, CHUNKS)                                                                                   \
     hipLaunchKernelGGL((rms_norm_rows_kernel<T, LANES, CHUNKS>), dim3(rows_grid(a, LANES)), dim3(kRowThreads), 0, st,    \
                        (const T*)in, (const T*)weight, (T*)out, a, b, eps)
@@ -592,11 +598,10 @@ template <typename T, bool CAUSAL>
 static int softmax_t(hipStream_t st, const void* in, void* out, size_t a, size_t b, size_t c, size_t s,
                      size_t offset, float scale) {
     const bool aligned = rows_vector_path(in, out, b, c, sizeof(T));
+    // rows of any length and alignment that a group of threads can hold
+    const bool ragged = !aligned && c == 1 && sizeof(T) == 2 && b >= kRowVec && rows_fit_registers(b);
     const int lanes = rows_lanes(b, 3072);
-    // rows of any length and alignment that a group of threads can hold, as many as a launch has threads for (2^32)
-    const bool ragged = !aligned && c == 1 && sizeof(T) == 2 && b >= kRowVec && rows_fit_registers(b) &&
-                        rows_grid(a, lanes) < (1u << 24);
-    if (aligned || ragged) {
+    if ((aligned || ragged) && rows_fit_launch(a, lanes, !rows_fit_registers(b))) {
 #define MH_SOFTMAX_ROWS(LANES, CHUNKS)                                                                                \
     if (ragged)                                                                                                       \
         hipLaunchKernelGGL((softmax_rows_kernel<T, CAUSAL, true, LANES, CHUNKS>), dim3(rows_grid(a, LANES)),            \
@@ -627,8 +632,8 @@ static int softmax_t(hipStream_t st, const void* in, void* out, size_t a, size_t
 
 template <typename T, bool IS_MAX, bool MEAN = false>
 static int reduce_t(hipStream_t st, const void* in, void* out, size_t a, size_t b, size_t c) {
-    if (c == 1) {
-        const int lanes = rows_lanes(b, 3072);
+    const int lanes = rows_lanes(b, 3072);
+    if (c == 1 && rows_fit_launch(a, lanes, b >= kReduceWideMin)) {
 #define MH_REDUCE_ROWS(LANES)                                                                                        \
     hipLaunchKernelGGL((reduce_rows_kernel<T, IS_MAX, MEAN, LANES>), dim3(rows_grid(a, LANES)), dim3(kRowThreads), 0, \
                        st, (const T*)in, (T*)out, a, b)
