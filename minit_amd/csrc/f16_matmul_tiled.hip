@@ -19,6 +19,8 @@
 // leaves through LDS as 16-byte row pieces.
 #include "common.h"
 
+#include <algorithm>
+
 namespace mh {
 
 constexpr int kTiledBN = 128, kTiledBK = 64, kTiledThreads = 256;
@@ -203,7 +205,13 @@ __global__ __launch_bounds__(kTiledThreads, STAGES == 1 ? 4 : 2) void f16_matmul
 
 bool f16_matmul_lds_supported(int M, int N, int K);  // f16_matmul_lds.hip
 
-bool f16_matmul_tiled_supported(int M, int N, int K) { return M > 0 && N > 0 && K >= 8; }
+// A launch holds 2^32 threads: tiles beyond that go into further launches, a row of tiles into one.
+constexpr size_t kTiledMostTiles = ((size_t)1 << 32) / kTiledThreads - 1;
+static int tiled_columns(int N) { return (int)(((long long)N + kTiledBN - 1) / kTiledBN); }
+
+bool f16_matmul_tiled_supported(int M, int N, int K) {
+    return M > 0 && N > 0 && K >= 8 && (size_t)tiled_columns(N) <= kTiledMostTiles;
+}
 
 // Of the shapes with whole 16-byte pieces the other kernels serve too (K a multiple of 32), those of more than
 // 16 rows that the LDS-streaming kernel does not take (K below 384 or no multiple of 64: 32 x [1500, 1500, 128]
@@ -217,8 +225,8 @@ bool f16_matmul_tiled_preferred(int M, int N, int K) {
     if (M <= 16 || !f16_matmul_tiled_supported(M, N, K)) return false;
     if (!f16_matmul_lds_supported(M, N, K)) return true;
     if (M <= 64) return false;
-    const size_t cus = compute_units(), tiles_n = (N + kTiledBN - 1) / kTiledBN;
-    return (N <= 256 && K <= 4096) || tiles_n * ((M + 127) / 128) >= 2 * cus || (M <= 128 && tiles_n * 4 >= 3 * cus);
+    const size_t cus = compute_units(), tiles_n = tiled_columns(N);
+    return (N <= 256 && K <= 4096) || tiles_n * (((size_t)M + 127) / 128) >= 2 * cus || (M <= 128 && tiles_n * 4 >= 3 * cus);
 }
 
 // Height of the tiles.  A CU takes about a microsecond for a stage of 256 rows whether one workgroup asks or two, so
@@ -233,11 +241,11 @@ struct TiledPlan {
 };
 static TiledPlan plan_tiled(int batch, int M, int N, int K) {
     if (K <= 2 * kTiledBK && M > 32) return {64, 1};
-    const size_t cus = compute_units(), columns = (size_t)batch * ((N + kTiledBN - 1) / kTiledBN);
+    const size_t cus = compute_units(), columns = (size_t)batch * tiled_columns(N);
     TiledPlan best = {32, 2};
     size_t least = 0;
     for (int bm = M <= 32 ? 32 : M <= 64 ? 64 : M <= 96 ? 96 : 128; bm >= 32; bm -= 32) {
-        const size_t cost = (columns * ((M + bm - 1) / bm) + cus - 1) / cus * (bm + 128);
+        const size_t cost = (columns * (((size_t)M + bm - 1) / bm) + cus - 1) / cus * (bm + 128);
         if (least == 0 || cost < least) {
             least = cost;
             best.bm = bm;
@@ -246,18 +254,17 @@ static TiledPlan plan_tiled(int batch, int M, int N, int K) {
     return best;
 }
 
-int f16_matmul_tiled_launch(hipStream_t stream, const void* a, const void* b, void* out, int batch, int M, int N, int K) {
-    const TiledPlan p = plan_tiled(batch, M, N, K);
-    const int bm = p.bm, tiles_m = (M + bm - 1) / bm, tiles_n = (N + kTiledBN - 1) / kTiledBN;
-    const size_t tiles = (size_t)tiles_m * tiles_n * batch;
-    MH_REQUIRE(tiles <= 0x7fffffffu, "dense fp16 product: %zu output tiles are too many for one launch", tiles);
-#define MH_TILED(BM, STAGES)                                                                                       \
-    hipLaunchKernelGGL((f16_matmul_nk_tiled_kernel<BM, STAGES>), dim3((unsigned)tiles), dim3(kTiledThreads), 0, stream, \
-                       (const half_t*)a, (const half_t*)b, (half_t*)out, M, N, K, tiles_m, tiles_n)
+static int tiled_launch_part(hipStream_t stream, const TiledPlan& p, const half_t* a, const half_t* b, half_t* out, int batch,
+                             int M, int N, int K) {
+    const int tiles_m = (int)(((long long)M + p.bm - 1) / p.bm), tiles_n = tiled_columns(N);
+    const unsigned tiles = (unsigned)((size_t)tiles_m * tiles_n * batch);
+#define MH_TILED(BM, STAGES)                                                                                          \
+    hipLaunchKernelGGL((f16_matmul_nk_tiled_kernel<BM, STAGES>), dim3(tiles), dim3(kTiledThreads), 0, stream, a, b, out, M, \
+                       N, K, tiles_m, tiles_n)
     if (p.stages == 1) {
         MH_TILED(64, 1);
     } else {
-        switch (bm) {
+        switch (p.bm) {
             case 32: MH_TILED(32, 2); break;
             case 64: MH_TILED(64, 2); break;
             case 96: MH_TILED(96, 2); break;
@@ -266,6 +273,24 @@ int f16_matmul_tiled_launch(hipStream_t stream, const void* a, const void* b, vo
     }
 #undef MH_TILED
     MH_CHECK_LAUNCH();
+    return MH_OK;
+}
+
+int f16_matmul_tiled_launch(hipStream_t stream, const void* a, const void* b, void* out, int batch, int M, int N, int K) {
+    const TiledPlan p = plan_tiled(batch, M, N, K);
+    const size_t tiles_n = tiled_columns(N), tiles = (((size_t)M + p.bm - 1) / p.bm) * tiles_n;
+    const half_t *pa = (const half_t*)a, *pb = (const half_t*)b;
+    half_t* po = (half_t*)out;
+    // whole matrices per launch, or row blocks of one matrix
+    const int matrices = tiles <= kTiledMostTiles ? (int)std::min((size_t)batch, kTiledMostTiles / tiles) : 1;
+    const int rows = tiles <= kTiledMostTiles ? M : (int)(kTiledMostTiles / tiles_n * p.bm);
+    for (int i = 0; i < batch; i += matrices)
+        for (long long r = 0; r < M; r += rows) {
+            const int rc = tiled_launch_part(stream, p, pa + ((size_t)i * M + r) * K, pb + (size_t)i * N * K,
+                                             po + ((size_t)i * M + r) * N, std::min(matrices, batch - i),
+                                             (int)std::min((long long)rows, M - r), N, K);
+            if (rc) return rc;
+        }
     return MH_OK;
 }
 

@@ -3,6 +3,7 @@
 matrices lie back to back (what follows a row must not leak into it), against the float64 product."""
 import numpy as np
 import pytest
+import torch
 
 from helpers import assert_fp16_close
 
@@ -30,3 +31,22 @@ def test_tiled_dense_product(hip, batch, m, n, k):
         rows = slice(1, None) if i == 1 else slice(None)
         ref = a[i, rows].astype(np.float64) @ b[i].astype(np.float64).T
         assert_fp16_close(got[i, rows], ref, what=f"matrix {i}")
+
+
+@pytest.mark.parametrize("batch,m", [(1, (1 << 30) + 70), (1500, 11200 * 64 + 3)])
+def test_more_tiles_than_a_launch_holds(hip, batch, m):
+    """2^24 tiles and a few more, of one matrix and of a batch: several launches."""
+    n, k = 1, 8
+    a = torch.empty((batch * m, k), dtype=torch.float16, device="cuda").normal_()
+    b = torch.empty((batch, n, k), dtype=torch.float16, device="cuda").normal_()
+    out = torch.full((batch * m,), float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    hip.call("mh_f16_matmul_nk_batched", None, a.data_ptr(), b.data_ptr(), out.data_ptr(), batch, m, n, k)
+    torch.cuda.synchronize()
+    assert not torch.isnan(out).any()
+    last = batch * m
+    for r in (0, 1 << 16, last // 2, last - m, last - 40000):
+        rows = torch.arange(r, min(r + 40000, last), device="cuda")
+        want = (a[rows].double() * b[rows // m, 0].double()).sum(-1)
+        # eight products in 32 bits, one fp16 rounding
+        assert ((out[rows].double() - want).abs() <= 2.0 ** -11 * want.abs() + 2.0 ** -18).all(), r
