@@ -22,9 +22,10 @@ constexpr int kDenseDepth = 8;
 // had just issued.)  Steps past the end of K re-read the last step and multiply
 // it by a zeroed a fragment.
 //
-// KS = 4: the four waves of a workgroup share one group of 16 NT columns and take a quarter of K each
+// Up to 16 rows per workgroup: what has more goes to the tiled kernel or to the one that streams the weight through
+// LDS.  KS = 4: the four waves of a workgroup share one group of 16 columns and take a quarter of K each
 // (a weight of few rows gives too few waves for the memory system otherwise); their sums meet in LDS.
-template <int MT, int NT, int KS>
+template <int KS>
 __global__ __launch_bounds__(256) void f16_matmul_nk_kernel(const half_t* __restrict__ a,
                                                             const half_t* __restrict__ b,
                                                             half_t* __restrict__ out, int M, int N, int K) {
@@ -34,43 +35,28 @@ __global__ __launch_bounds__(256) void f16_matmul_nk_kernel(const half_t* __rest
     out += (size_t)blockIdx.z * M * N;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int i16 = lane & 15, kq = lane >> 4;
-    // a wave owns NT groups of 16 output columns: above 16 rows two groups share every
-    // a fragment, which halves the a traffic per byte of b (a comes from the caches,
-    // but through the same vector memory path as b)
-    const int n0 = (KS == 1 ? blockIdx.x * 4 + wave : blockIdx.x) * (16 * NT);
-    const int m0 = blockIdx.y * (16 * MT);
+    const int n0 = (KS == 1 ? blockIdx.x * 4 + wave : blockIdx.x) * 16;
+    const int m0 = blockIdx.y * 16;
     if (n0 >= N) return;  // the whole workgroup when its waves share the columns
     const int steps = K / (32 * KS);  // of this wave
     const int k_first = KS == 1 ? 0 : wave * steps * 32;
-    const half_t* brow[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) brow[nt] = b + (size_t)min(n0 + nt * 16 + i16, N - 1) * K + kq * 8 + k_first;
-    const half_t* arow[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) arow[mt] = a + (size_t)min(m0 + mt * 16 + i16, M - 1) * K + kq * 8 + k_first;
+    const half_t* brow = b + (size_t)min(n0 + i16, N - 1) * K + kq * 8 + k_first;
+    const half_t* arow = a + (size_t)min(m0 + i16, M - 1) * K + kq * 8 + k_first;
 
-    float4_t acc[MT][NT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = float4_t{0.f, 0.f, 0.f, 0.f};
-
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
     const int last = steps - 1;
     // Workgroup i starts four i steps (128 bytes) into its K range and wraps around: started together, all
     // workgroups ask for the same bytes of rows 2 K bytes apart at once, which fall on a fraction of the
     // memory channels (3-8 % on weights of 8192 to 128256 rows).
     const int first = (int)(((uint32_t)blockIdx.x * 4u) % (uint32_t)steps);
     constexpr int D = kDenseDepth;
-    uint4_t bq[D][NT], aq[D][MT];
+    uint4_t bq[D], aq[D];
     auto load = [&](int slot, int s) {
         int at = min(s, last) + first;
         if (at >= steps) at -= steps;
         const size_t off = (size_t)at * 32;
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-            bq[slot][nt] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>(brow[nt] + off));
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) aq[slot][mt] = *reinterpret_cast<const uint4_t*>(arow[mt] + off);
+        bq[slot] = __builtin_nontemporal_load(reinterpret_cast<const uint4_t*>(brow + off));
+        aq[slot] = *reinterpret_cast<const uint4_t*>(arow + off);
     };
 #pragma unroll
     for (int d = 0; d < D; ++d) load(d, d);
@@ -78,54 +64,33 @@ __global__ __launch_bounds__(256) void f16_matmul_nk_kernel(const half_t* __rest
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             const bool live = s0 + d <= last;
-            half8_t bf[NT], af[MT];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) bf[nt] = __builtin_bit_cast(half8_t, bq[d][nt]);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                af[mt] = __builtin_bit_cast(half8_t, live ? aq[d][mt] : uint4_t{0u, 0u, 0u, 0u});
+            const half8_t bf = __builtin_bit_cast(half8_t, bq[d]);
+            const half8_t af = __builtin_bit_cast(half8_t, live ? aq[d] : uint4_t{0u, 0u, 0u, 0u});
             load(d, s0 + d + D);
             __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)  // rows of the result are m (operand A), columns are n (operand B)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[mt], bf[nt], acc[mt][nt], 0, 0, 0);
+            // rows of the result are m (operand A), columns are n (operand B)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(af, bf, acc, 0, 0, 0);
         }
     }
     if constexpr (KS > 1) {
-        __shared__ float4_t sums[KS - 1][MT * NT][64];
-        if (wave > 0) {
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) sums[wave - 1][mt * NT + nt][lane] = acc[mt][nt];
-        }
+        __shared__ float4_t sums[KS - 1][64];
+        if (wave > 0) sums[wave - 1][lane] = acc;
         __syncthreads();
         if (wave > 0) return;
 #pragma unroll
-        for (int w = 0; w < KS - 1; ++w)
+        for (int w = 0; w < KS - 1; ++w) {
+            const float4_t v = sums[w][lane];
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    const float4_t v = sums[w][mt * NT + nt][lane];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[mt][nt][r] += v[r];
-                }
+            for (int r = 0; r < 4; ++r) acc[r] += v[r];
+        }
     }
-    // acc[mt][nt][r] is row m0 + mt*16 + kq*4 + r, column n0 + nt*16 + i16
+    // acc[r] is row m0 + kq*4 + r, column n0 + i16
+    const int n = n0 + i16;
+    if (n >= N) return;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        const int n = n0 + nt * 16 + i16;
-        if (n >= N) continue;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = m0 + mt * 16 + kq * 4 + r;
-                if (m < M) out[(size_t)m * N + n] = (half_t)acc[mt][nt][r];
-            }
+    for (int r = 0; r < 4; ++r) {
+        const int m = m0 + kq * 4 + r;
+        if (m < M) out[(size_t)m * N + n] = (half_t)acc[r];
     }
 }
 
@@ -287,29 +252,21 @@ using namespace mh;
 
 // The MFMA kernels for `batch` matrices (K a multiple of 32, every matrix on a 16-byte boundary): tiles of both
 // operands in LDS for many rows, the weight streamed through LDS in whole lines where that kernel serves the
-// shape, operands straight from global memory otherwise.  Kernel and tiling depend on M, N and K only.
+// shape, operands straight from global memory otherwise (up to 16 rows).  Which kernel depends on M, N and K only; the
+// height of the tiles also on the batch, but not the order of a sum: a matrix of a batch gets the bits it gets alone.
 static int launch_dense_mfma(hipStream_t st, const void* a, const void* b, void* out, int batch, int M, int N, int K) {
     if (f16_matmul_tiled_preferred(M, N, K)) return f16_matmul_tiled_launch(st, a, b, out, batch, M, N, K);
-    if (f16_matmul_lds_supported(M, N, K) && (M + 63) / 64 <= 65535) return f16_matmul_lds_launch(st, a, b, out, batch, M, N, K);
-    const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    const int nt = mt == 1 ? 1 : 2;  // columns per wave: 16 or 32
-    dim3 grid((N + 64 * nt - 1) / (64 * nt), (M + 16 * mt - 1) / (16 * mt), batch);
+    if (f16_matmul_lds_supported(M, N, K)) return f16_matmul_lds_launch(st, a, b, out, batch, M, N, K);
+    dim3 grid((unsigned)(((long long)N + 63) / 64), (unsigned)(((long long)M + 15) / 16), batch);
     MH_REQUIRE(grid.y <= 65535, "dense fp16 product: M=%d is too large for one launch", M);
-    const bool share_k = dense_share_k(grid.x * grid.y, K);
-    if (share_k) grid.x = (N + 16 * nt - 1) / (16 * nt);
-#define MH_DENSE(MT, NT)                                                                                            \
-    if (share_k)                                                                                                    \
-        hipLaunchKernelGGL((f16_matmul_nk_kernel<MT, NT, 4>), grid, dim3(256), 0, st, (const half_t*)a,            \
-                           (const half_t*)b, (half_t*)out, M, N, K);                                                \
-    else                                                                                                            \
-        hipLaunchKernelGGL((f16_matmul_nk_kernel<MT, NT, 1>), grid, dim3(256), 0, st, (const half_t*)a,            \
-                           (const half_t*)b, (half_t*)out, M, N, K)
-    switch (mt) {
-        case 1: MH_DENSE(1, 1); break;
-        case 2: MH_DENSE(2, 2); break;
-        default: MH_DENSE(4, 2); break;
+    if (dense_share_k(grid.x * grid.y, K)) {
+        grid.x = (unsigned)(((long long)N + 15) / 16);
+        hipLaunchKernelGGL(f16_matmul_nk_kernel<4>, grid, dim3(256), 0, st, (const half_t*)a, (const half_t*)b, (half_t*)out,
+                           M, N, K);
+    } else {
+        hipLaunchKernelGGL(f16_matmul_nk_kernel<1>, grid, dim3(256), 0, st, (const half_t*)a, (const half_t*)b, (half_t*)out,
+                           M, N, K);
     }
-#undef MH_DENSE
     MH_CHECK_LAUNCH();
     return MH_OK;
 }
