@@ -213,6 +213,9 @@ int mh_f16_matmul_nk_batched(mh_stream_t stream, const void* a, const void* b, v
 int mh_i8_gemm(mh_stream_t stream, const int8_t* a, const int8_t* w,
                const float* a_scale, const float* w_scale, void* out_f16,
                int32_t* acc_i32, int M, int N, int K);
+/* rows << 16 | columns of the output tiles that mh_i8_gemm works in for a shape (16 to 64 of either where the
+ * waves of a workgroup share the tile and split K, 128 x 256 otherwise); 0 for a shape it refuses. */
+int mh_i8_gemm_tile(int M, int N, int K);
 /* out[n, k] = in[k, n]: one-time layout conversion for weights stored [K, N]. */
 int mh_i8_transpose(mh_stream_t stream, const int8_t* in, int8_t* out, int rows, int cols);
 

@@ -513,6 +513,7 @@ int i8_gemm_dma_launch(hipStream_t stream, const int8_t* a, const int8_t* w, con
                        const float* w_scale, void* out_f16, int32_t* acc_i32, int M, int N, int K);
 // i8_gemm_rows.hip: small tiles, K split over the waves of a workgroup
 bool i8_gemm_rows_preferred(int M, int N, int K);
+int i8_gemm_rows_tile(int M, int N, int K);
 int i8_gemm_rows_launch(hipStream_t stream, const int8_t* a, const int8_t* w, const float* a_scale,
                         const float* w_scale, void* out_f16, int32_t* acc_i32, int M, int N, int K);
 
@@ -573,6 +574,11 @@ int mh_i8_gemm(mh_stream_t stream, const int8_t* a, const int8_t* w, const float
 #undef MH_I8_LAUNCH
     MH_CHECK_LAUNCH();
     return MH_OK;
+}
+
+int mh_i8_gemm_tile(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || K % kI8BK != 0) return 0;
+    return i8_gemm_rows_preferred(M, N, K) ? i8_gemm_rows_tile(M, N, K) : kI8BM << 16 | kI8BN;
 }
 
 int mh_i8_transpose(mh_stream_t stream, const int8_t* in, int8_t* out, int rows, int cols) {

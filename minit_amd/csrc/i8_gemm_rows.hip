@@ -9,10 +9,11 @@
 // sixteen lines per load, four lanes of each).  Integer sums are exact in any order: the results are those of the
 // other kernels bit for bit.
 // What bounds it: the operand bytes of the tiles on their way into a CU, 58 to 66 bytes per ns whatever the tile,
-// then the weight's bytes from HBM at 5.4 to 5.8 TB/s, on top of 2.7 us of launch, first load and reduction
-// (us, against the 128 x 256 tiles: 32 x 11008 x 4096 12.6 / 27.4, 1 x 11008 x 4096 11.0 / 26.3,
-// 64 x 4096 x 4096 7.5 / 26.4, 32 x 1024 x 14336 9.9 / 78.8, 256 x 4096 x 4096 12.1 / 28.1, 512 x 4096 x 4096
-// 18.5 / 27.5; with 64 x 64 tiles 1024 x 4096 x 4096 33.5 / 28.0).
+// then the weight's bytes at 5.4 to 5.8 TB/s from HBM, on top of 2.7 us of launch, first load and reduction.  Us, here /
+// on the 128 x 256 tiles, with the weight in the last-level cache (one weight, call after call) and from HBM (a gigabyte
+// of weights in turn): 32 x 11008 x 4096 9.7 / 21.7 and 12.5 / 27.6, 1 x 11008 x 4096 9.1 / 21.2 and 11.4 / 26.0,
+// 64 x 4096 x 4096 6.0 / 21.0 and 7.7 / 27.4, 32 x 1024 x 14336 6.2 / 61.5 and 10.6 / 82.4, 256 x 4096 x 4096 10.5 / 21.7
+// and 12.8 / 29.3, 512 x 4096 x 4096 16.9 / 22.3 and 19.2 / 28.7.
 #include "common.h"
 
 #include <cmath>
@@ -200,56 +201,87 @@ __global__ __launch_bounds__(KW * 64) void i8_gemm_rows_kernel(
 
 // ---- which tile, and whether to take this kernel at all ------------------------------------------------------
 
+// A tile of mt x nt times 16 and the waves of its workgroup; the four numbers are rows_time()'s.
 struct RowsTile {
-    int mt, nt;
+    int mt, nt, waves;
+    double fixed, larger, smaller, pass;
 };
-constexpr RowsTile kRowsTiles[] = {{1, 1}, {2, 1}, {2, 2}, {1, 4}, {2, 4}, {4, 4}};
+constexpr RowsTile kRowsTiles[] = {
+    {1, 1, 8, 4.88, 0.155, 0.365, 0.44}, {2, 1, 4, 4.96, 0.254, 0.292, 0.29}, {2, 2, 4, 4.12, 0.422, 0.655, 0.45},
+    {1, 4, 4, 4.28, 0.573, 0.570, 0.00}, {2, 4, 8, 2.48, 0.594, 0.517, 1.87}, {4, 4, 4, 3.13, 0.787, 0.401, 1.26},
+};
 
-// Expected time (ns) of a product on tiles of mt x nt times 16: the bytes of the fullest CU at 62 bytes per ns, the
-// weight's bytes at 5.5 TB/s, a quarter of the smaller of the two on top of the larger, 2.7 us around them.  Over the
-// shapes that were measured (1 to 1024 rows, 1024 to 28672 columns, K 1024 to 14336) it is within 15 % and names the
-// fastest tile or one within 8 % of it.
-static double rows_cost(const RowsTile& t, int M, int N, int K) {
-    const double cus = compute_units();
-    const double rows = t.mt * 16, columns = t.nt * 16;
-    const double tiles = ceil(M / rows) * ceil(N / columns);
-    const double cu = ceil(tiles / cus) * ((M < rows ? M : rows) + columns) * K / 62.0;
-    const double hbm = (double)N * K / 5500.0;
-    return 2700.0 + (cu > hbm ? cu + 0.25 * hbm : hbm + 0.25 * cu);
+static size_t rows_tiles(const RowsTile& t, int M, int N) {
+    return (((size_t)M + t.mt * 16 - 1) / (t.mt * 16)) * (((size_t)N + t.nt * 16 - 1) / (t.nt * 16));
 }
 
-// The 128 x 256 tiles: 6.1 ns per k and round of one tile on every CU, measured at K 4096 (one round 26 to 34 us,
-// two 63 to 75, three 83 to 106) and 14336 (79 to 94 us), 9.9 on the 64-k stages of other K (24 x 5000 x 4160
-// 44.9 us, 33 x 3000 x 7232 74.9), and the weight's bytes as above.
-static double tiled_cost(int M, int N, int K) {
-    const double tiles = (double)((M + 127) / 128) * ((N + 255) / 256);
-    return 3000.0 + ceil(tiles / compute_units()) * (K % 128 == 0 ? 6.1 : 9.9) * K + 0.25 * ((double)N * K / 5500.0);
+// Us that the operand bytes take: of the fullest CU at 62 bytes per ns, and of the weight at 5.5 TB/s.
+struct RowsBytes {
+    double cu, weight, passes;
+};
+static RowsBytes rows_bytes(const RowsTile& t, int M, int N, int K) {
+    const double passes = ceil((double)rows_tiles(t, M, N) / compute_units()), rows = t.mt * 16;
+    return {passes * ((M < rows ? M : rows) + t.nt * 16) * K / 62e3, (double)N * K / 5.5e6, passes};
 }
 
-static const RowsTile* rows_best(int M, int N, int K) {
+// The tile: the larger of the two and a quarter of the smaller.  Over the shapes that were measured (1 to 1024 rows, 1024 to
+// 28672 columns, K 1024 to 14336) that names the fastest tile or one within 8 % of it.
+static const RowsTile& rows_best(int M, int N, int K) {
     const RowsTile* best = nullptr;
-    double cost = tiled_cost(M, N, K);
+    double least = 0;
     for (const RowsTile& t : kRowsTiles) {
-        const double c = rows_cost(t, M, N, K);
-        if (c < cost) {
-            cost = c;
+        const RowsBytes b = rows_bytes(t, M, N, K);
+        const double cost = b.cu > b.weight ? b.cu + 0.25 * b.weight : b.weight + 0.25 * b.cu;
+        if (best == nullptr || cost < least) {
+            least = cost;
             best = &t;
         }
     }
-    return best;
+    return *best;
 }
 
-// A resource covers the rows of one tile: up to 64 rows of K bytes below 2 GiB.
-bool i8_gemm_rows_preferred(int M, int N, int K) { return K < (1 << 24) && rows_best(M, N, K) != nullptr; }
+// Expected time in us, operands in the last-level cache: a fit per tile over 4800 shapes (1 to 4096 rows, 256 to 28672
+// columns, K 192 to 14336), four of five within 15 %.
+static double rows_time(const RowsTile& t, int M, int N, int K) {
+    const RowsBytes b = rows_bytes(t, M, N, K);
+    return t.fixed + t.larger * (b.cu > b.weight ? b.cu : b.weight) + t.smaller * (b.cu > b.weight ? b.weight : b.cu) +
+           t.pass * b.passes;
+}
+
+// The same for the 128 x 256 tiles of the other kernels, by the kernel that K picks there: 128-k stages loaded straight
+// into LDS, the same by registers (K 128 and 256), and 64-k stages.  `passes` of a tile on every CU.
+static double tiled_time(int M, int N, int K) {
+    const double passes = ceil((double)((((size_t)M + 127) / 128) * (((size_t)N + 255) / 256)) / compute_units());
+    const double k = passes * K / 1e3, weight = (double)N * K / 5.5e6;
+    if (K % 128 != 0) return -4.39 + 7.43 * k + 7.57 * passes + 1.02 * weight;
+    return K < 384 ? -1.41 + 1.86 * k + 7.27 * passes + 0.38 * weight : -5.06 + 4.02 * k + 9.68 * passes + 0.63 * weight;
+}
+
+// Taken where a tenth is to be won: of 4800 shapes that a plain comparison of the bytes sent here 170 were more than a tenth
+// slower than on the 128 x 256 tiles, up to 1.8 times (many rows and a short K: 752 x 4032 x 256 9.7 us against 7.1, 2113 x
+// 1352 x 1920 18.9 / 14.5).  With this line 10 of 12400 others are, and the geometric mean over all of them is 0.54 of the
+// 128 x 256 tiles' time.  A resource covers the rows of one tile, up to 64 rows of K bytes below 2 GiB, and a launch 2^32
+// threads.
+bool i8_gemm_rows_preferred(int M, int N, int K) {
+    if (K >= (1 << 24)) return false;
+    const RowsTile& t = rows_best(M, N, K);
+    return rows_tiles(t, M, N) * t.waves * 64 < ((size_t)1 << 32) && rows_time(t, M, N, K) < 0.9 * tiled_time(M, N, K);
+}
+
+int i8_gemm_rows_tile(int M, int N, int K) {
+    const RowsTile& t = rows_best(M, N, K);
+    return t.mt * 16 << 16 | t.nt * 16;
+}
 
 int i8_gemm_rows_launch(hipStream_t stream, const int8_t* a, const int8_t* w, const float* a_scale,
                         const float* w_scale, void* out_f16, int32_t* acc_i32, int M, int N, int K) {
-    const RowsTile t = *rows_best(M, N, K);
-    const int tiles_m = (M + t.mt * 16 - 1) / (t.mt * 16), tiles_n = (N + t.nt * 16 - 1) / (t.nt * 16);
+    const RowsTile& t = rows_best(M, N, K);
+    const int tiles_m = (int)(((size_t)M + t.mt * 16 - 1) / (t.mt * 16));
+    const unsigned tiles = (unsigned)rows_tiles(t, M, N);
     // LDS per workgroup 64, 72, 64, 80, 96 and 64 KiB: two of all but the fifth share a CU
 #define MH_I8_ROWS(MT, NT, KW, R)                                                                                     \
-    hipLaunchKernelGGL((i8_gemm_rows_kernel<MT, NT, KW, R>), dim3((unsigned)tiles_m * (unsigned)tiles_n),             \
-                       dim3(KW * 64), 0, stream, a, w, a_scale, w_scale, (half_t*)out_f16, acc_i32, M, N, K, tiles_m)
+    hipLaunchKernelGGL((i8_gemm_rows_kernel<MT, NT, KW, R>), dim3(tiles), dim3(KW * 64), 0, stream, a, w, a_scale,     \
+                       w_scale, (half_t*)out_f16, acc_i32, M, N, K, tiles_m)
     switch (t.mt * 8 + t.nt) {
         case 1 * 8 + 1: MH_I8_ROWS(1, 1, 8, 2); break;
         case 2 * 8 + 1: MH_I8_ROWS(2, 1, 4, 3); break;

@@ -24,16 +24,33 @@ def _run(hip, a, w, a_scale, w_scale, want_acc=True, want_out=True):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (128, 256, 64),       # exactly one tile, one k-step
+    (128, 256, 64),       # exactly one tile of 128 x 256, one k-step
     (1, 8, 64),           # far smaller than a tile
     (130, 260, 192),      # ragged M and N
-    (257, 1000, 512),     # 128-k stages, ring of four
-    (100, 300, 768),      # 128-k stages, ring of two
-    (64, 136, 384),       # 128-k stages, ring of one
-    (130, 260, 128),      # a single 128-k stage
-    (2048, 4096, 4096),   # config 2
+    (257, 1000, 512),     # 32 x 64 tiles
+    (100, 300, 768),      # 16 x 16 tiles
+    (64, 136, 384),
+    (130, 260, 128),
+    (2048, 4096, 4096),   # config 2: 128 x 256 tiles, stages loaded straight into LDS
 ])
 def test_i8_gemm_bit_exact(hip, m, n, k):
+    _check(hip, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (35, 2302, 128), (37, 2302, 256),      # one and two stages of 128 k through registers
+    (300, 4001, 320), (700, 5003, 704),    # stages of 64 k, an odd number
+    (1061, 6536, 2240),
+    (515, 5001, 384), (900, 9001, 512),    # stages loaded straight into LDS: the fewest, one more
+    (1061, 6531, 640), (900, 6531, 1152),
+])
+def test_i8_gemm_large_tiles_bit_exact(hip, m, n, k):
+    """Ragged rows and columns on the kernels of 128 x 256 tiles, for every kind of K they take."""
+    assert divmod(hip.call("mh_i8_gemm_tile", m, n, k), 1 << 16) == (128, 256)
+    _check(hip, m, n, k)
+
+
+def _check(hip, m, n, k):
     from minit_amd import synthetic
     a, w, a_scale, w_scale = synthetic.int8_operands(f"i8-{m}-{n}-{k}", m, n, k)
     out, acc = _run(hip, a, w, a_scale, w_scale)
@@ -62,8 +79,7 @@ def _sweep(count, seed):
 @pytest.mark.parametrize("m,n,k", _sweep(16, seed=77))
 def test_i8_gemm_random_shapes(hip, m, n, k):
     """Seeded sweep over ragged M and N (any value, not only multiples of the
-    tile) and over K in both kernels' ranges (64-k and 128-k stages): int32
-    accumulators and the scaled fp16 output bit for bit."""
+    tile) and over K: int32 accumulators and the scaled fp16 output bit for bit."""
     from minit_amd import synthetic
     a, w, a_scale, w_scale = synthetic.int8_operands(f"i8-sweep-{m}-{n}-{k}", m, n, k)
     out, acc = _run(hip, a, w, a_scale, w_scale)
