@@ -466,9 +466,16 @@ __global__ __launch_bounds__(tall_k_shares(MT) * 128) void gptq_gemm_tall_kernel
             if (r + decltype(slot)::value < n_rounds) round(slot, r + decltype(slot)::value);
         });
 
-    // the loads requested past the end are still in flight: their registers are dead to the compiler
-    // and their stages would land in LDS that the reduction is about to use
+    // the loads requested past the end are still in flight: their stages would land in LDS that the reduction is
+    // about to use, and their registers pass through statements behind the wait, or the compiler, to whom
+    // they are dead from the last round on, puts the reduction's addresses there ahead of it
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int slot = 0; slot < NS; ++slot) {
+#pragma unroll
+        for (int i = 0; i < WR; ++i) asm volatile("" : "+v"(rq[slot][i]));
+        asm volatile("" : "+v"(rs[slot]), "+v"(rz[slot]));
+    }
     __syncthreads();
 
     // ---- the K shares of the waves, added in a fixed order: (0 + 1) + (2 + 3)

@@ -241,9 +241,15 @@ __global__ __launch_bounds__(128 * WN, 2) void gptq_gemm_wide_kernel(
         if (i + 1 < n_stages) run_stage(std::integral_constant<int, 1>{}, i + 1);
     }
 
-    // the loads requested for stages past the end are still in flight: their registers are dead
-    // to the compiler from here on, so let them land before anything else is put there
+    // the loads requested for stages past the end are still in flight: let them land before anything else is put
+    // into their registers, which pass through statements behind the wait (the compiler, to whom they are dead from
+    // the last stage on, may put the addresses of the stores there ahead of it otherwise)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int slot = 0; slot < 2; ++slot)
+#pragma unroll
+        for (int j = 0; j < PT; ++j) asm volatile("" : "+v"(ra[slot][j]), "+v"(rq[slot][j]));
+    asm volatile("" : "+v"(raw_s), "+v"(raw_z));
 
     // ---- results: acc[r][c][e] is row wy*64 + r*16 + kq*4 + e, column (wx*CT + c)*16 + nl of the tile
 #pragma unroll
