@@ -715,6 +715,9 @@ static TallPlan plan_tall(int M, int N, int K, int bits, bool tail_allowed = tru
     long split = capped(64 / bits);
     const long relaxed = capped(32 / bits);
     if (((rounds + relaxed - 1) / relaxed) * 4 <= ((rounds + split - 1) / split) * 3) split = relaxed;
+    // (8 bit: the ranges' sums on their way through memory take two to seven rounds, so at least six are to be saved:
+    // 580 x 1024 x 2880 in two ranges of four rounds 22.5 us, 858 x 1024 x 1456 19.2; the 64-row blocks before 17.4, 17.6)
+    if (bits == 8 && rounds - (rounds + split - 1) / split < 6) split = 1;
     p.rounds_per_block = (int)((rounds + split - 1) / split);
     p.split_k = (rounds + p.rounds_per_block - 1) / p.rounds_per_block;
     p.whole_tiles = p.split_k == 1 ? p.tiles() : 0;
@@ -749,12 +752,25 @@ static bool tall_two_row_tiles_preferred(int M, int N, int K) {
 // column-owner kernels (us, this kernel / before): at 16 rows 5120 x 15360 18.9 / 21.5, 5120 x 27392 27.3 / 28.6,
 // 13696 x 5120 18.3 / 19.6, 14336 x 4096 15.7 / 23.0, 28672 x 8192 41.2 / 43.9, 8192 x 8192 17.5 / 17.7; at 32 rows
 // 20.5 / 27.5, 29.4 / 33.1, 19.6 / 22.3, 16.9 / 24.3, 43.6 / 51.2, 18.2 / 21.6, 4096 x 4096 11.8 / 12.3.  It loses where a
-// launch is all fixed costs (4096 x 4096 at 16 rows 10.5 / 9.5, 2048 x 1024 at 32 rows 8.7 / 7.3) and where there are
-// more column tiles than CUs (8192 x 57344 at 16 / 32 rows 79.8 / 73.1, 86.5 / 78.7).  Up to eight rows the gain is
-// within a few per cent either way and the other kernels' epilogues stay in one launch.
+// launch is all fixed costs (4096 x 4096 at 16 rows 10.5 / 9.5, 2048 x 1024 at 32 rows 8.7 / 7.3), where there are
+// more column tiles than CUs (8192 x 57344 at 16 / 32 rows 79.8 / 73.1, 86.5 / 78.7), and where the workgroups leave
+// a fifth of the CUs idle over a long walk: a CU takes 0.62 us per round however few others ask, the small-M kernel
+// spreads the weight over all of them (13696 x 17992, 141 workgroups of 107 rounds, at 10 rows 65.1 / 48.9; 24832 x 17128
+// at 12 rows 112 / 78).  Of 1050 shapes 128 were more than 5 % slower here without that line, 15 with it.  Up to
+// eight rows the gain is within a few per cent either way and the other kernels' epilogues stay in one launch.
 static bool tall_8bit_preferred(int M, int N, int K) {
     if (M < 9 || M > 32 || (N + kTallBN - 1) / kTallBN > compute_units()) return false;
-    return (size_t)N * K >= (M <= 16 ? (size_t)24 << 20 : (size_t)16 << 20);
+    if ((size_t)N * K < (M <= 16 ? (size_t)24 << 20 : (size_t)16 << 20)) return false;
+    const TallPlan p = plan_tall(M, N, K, 8);
+    return (long)p.tiles_n * p.split_k * 5 >= (long)compute_units() * 4 || p.rounds_per_block <= (M <= 16 ? 24 : 40);
+}
+
+// The same of more rows: fewer workgroups than two thirds of the CUs over 64 rounds and more (10496 x 19032, 149
+// workgroups, at 39 rows 66.8 us against 54.7 on the 64-row blocks; 20352 x 8864 at 151 rows 140 / 116; with 171 workgroups
+// and more, and with shorter walks, never slower by more than 3 % but for a handful of 10,000 shapes).
+static bool tall_8bit_idle(int M, int N, int K) {
+    const TallPlan p = plan_tall(M, N, K, 8);
+    return (long)p.tiles() * (p.split_all() ? p.split_k : 1) * 3 < (long)compute_units() * 2 && K / kTallRoundK >= 64;
 }
 
 // Measured on one box against what served these shapes before (the small-M kernel's 64-row blocks up to
@@ -780,7 +796,8 @@ bool gemm_tall_preferred(int M, int N, int K, int group_size, int bits, int epil
           (size_t)K * N * bits / 8 < ((size_t)1 << 31)))
         return false;
     if (tall_min_m_env() > 0) return M >= tall_min_m_env();
-    return M >= 33 || (bits == 4 ? tall_two_row_tiles_preferred(M, N, K) : tall_8bit_preferred(M, N, K));
+    if (bits == 4) return M >= 33 || tall_two_row_tiles_preferred(M, N, K);
+    return M >= 33 ? !tall_8bit_idle(M, N, K) : tall_8bit_preferred(M, N, K);
 }
 
 static size_t tall_plan_bytes(const TallPlan& p, int M, int N) {
