@@ -650,10 +650,11 @@ static bool tall_mt16_allowed() {
 
 // Tiles of BM = 16 mt rows in passes over the CUs: whole tiles for as many passes as they fill, and the tiles of the
 // last pass, if they leave CUs idle, in K ranges that fill them (us, before / with the ranges: 1000 x 13696 x 5120
-// 187 / 141, 1000 x 5120 x 5120 78 / 65, 1000 x 5120 x 27392 at 8 bit 302 / 285, 700 x 4096 x 12288 97 / 80).  cost: in
-// rounds of a 128 x 128 tile (about a microsecond).  A tile of 256 rows takes 1.74 times a tile of 128 (2048 x 8192 x
-// 57344 1666 us against 1932), the ranges' sums about eight rounds on their way through memory: with these two the
-// cheapest of the four plans came out fastest or within 3 % of it for each of 25 shapes of 130 to 2048 rows.
+// 187 / 141, 1000 x 5120 x 5120 78 / 65, 1000 x 5120 x 27392 at 8 bit 302 / 285, 700 x 4096 x 12288 97 / 80).  cost: us, fitted
+// to 1500 launches of 65 to 2048 rows, nine of ten within 8 %.  Beside its rounds (1.03 us of 128 k for a tile of 128 rows,
+// 0.87 of 64 k for one of 256) every pass pays for its ends, which is what decides at a short K: without that part
+// 512 to 1024 k went to 128-row tiles in twice the passes (1715 x 768 x 11624 53.5 -> 64.4 us, 1447 x 512 x 11088 41.2 ->
+// 50.3).  A split last pass adds the ranges' sums on their way through memory.
 static TallPlan plan_passes(int mt, int M, int N, int K, bool tail_allowed) {
     TallPlan p;
     const int cus = compute_units(), k_per_round = 32 * tall_k_shares(mt), rounds = K / k_per_round;
@@ -663,14 +664,14 @@ static TallPlan plan_passes(int mt, int M, int N, int K, bool tail_allowed) {
     p.split_k = 1;
     p.rounds_per_block = rounds;
     p.whole_tiles = p.tiles();
-    const double per_round = mt == 16 ? 1.74 / 2 : 1.0;
+    const double per_round = mt == 16 ? 0.87 : 1.03, ends = 6.5, sums = mt == 16 ? 9 : 4;
     const int rest = p.tiles() % cus, full = p.tiles() / cus;
-    p.cost = per_round * rounds * (full + (rest ? 1 : 0));
+    p.cost = (mt == 16 ? 2 : 0) + (full + (rest ? 1 : 0)) * (per_round * rounds + ends);
     if (rest && full && tail_allowed) {
         const int split = std::min(cus / rest, rounds / 4);
         if (split > 1) {
             const int per = (rounds + split - 1) / split;
-            const double cost = per_round * (full * rounds + per) + 8;
+            const double cost = p.cost - per_round * (rounds - per) + sums;
             if (cost < p.cost) {
                 p.whole_tiles = p.tiles() - rest;
                 p.rounds_per_block = per;
