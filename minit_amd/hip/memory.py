@@ -20,7 +20,8 @@ from .. import lib
 _POOL: "OrderedDict[int, List[int]]" = OrderedDict()
 _POOL_BYTES = 0
 _POOL_LIMIT = 4 << 30
-# Reentrant: a tensor may die (and release its block) while the lock is held.
+# Reentrant: a tensor may die (and release its block) while the lock is held.  Whatever allocates a container
+# may run the collector, so nothing read from the pool before such a place is relied on behind it.
 _POOL_LOCK = threading.RLock()
 
 
@@ -62,25 +63,23 @@ def allocate(size: int) -> int:
 def release(ptr: int, size: int) -> None:
     global _POOL_BYTES
     size = _round(size)
+    bucket: List[int] = []
     with _POOL_LOCK:
         if size > _POOL_LIMIT:
             lib.call("mh_free", ptr)
             return
         if _POOL_BYTES + size > _POOL_LIMIT:
             _make_room(size)
-        bucket = _POOL.get(size)
-        if bucket is None:
-            bucket = _POOL[size] = []
-        else:
-            _POOL.move_to_end(size)
-        bucket.append(ptr)
+        _POOL.setdefault(size, bucket).append(ptr)
+        _POOL.move_to_end(size)
         _POOL_BYTES += size
 
 
 def _make_room(size: int) -> None:
     global _POOL_BYTES
     while _POOL and _POOL_BYTES + size > _POOL_LIMIT:
-        oldest, bucket = next(iter(_POOL.items()))
+        oldest = next(iter(_POOL))
+        bucket = _POOL[oldest]
         if not bucket:
             del _POOL[oldest]
             continue

@@ -55,3 +55,56 @@ def test_blocks_above_the_limit_are_given_back(device):
     live, calls = device
     memory.release(memory.allocate(5 << 30), 5 << 30)
     assert not live and memory._POOL_BYTES == 0
+
+
+def test_a_tensor_dies_while_a_block_is_put_back(device, monkeypatch):
+    """The collector runs inside release(), where the list of a new size has been looked up and not yet stored."""
+    live, _ = device
+    size = 1 << 16
+    blocks = [memory.allocate(size) for _ in range(2)]
+
+    class Pool(type(memory._POOL)):
+        dying = [blocks[1]]
+
+        def _die(self):
+            while self.dying:
+                memory.release(self.dying.pop(), size)
+
+        def get(self, key, default=None):
+            value = super().get(key, default)
+            self._die()
+            return value
+
+        def setdefault(self, key, default=None):
+            self._die()
+            return super().setdefault(key, default)
+
+    monkeypatch.setattr(memory, "_POOL", Pool())
+    memory.release(blocks[0], size)
+    assert memory._POOL_BYTES == 2 * size
+    assert sorted(p for bucket in memory._POOL.values() for p in bucket) == sorted(blocks)
+
+
+def test_a_tensor_dies_while_blocks_are_given_back(device, monkeypatch):
+    """The collector runs inside hipFree's call, in eviction and in empty_cache()."""
+    live, _ = device
+    call, dying = memory.lib.call, []
+    size = 1 << 30
+    blocks = [memory.allocate(size) for _ in range(6)]
+
+    def call_and_collect(name, *args):
+        result = call(name, *args)
+        if name == "mh_free" and dying:
+            memory.release(dying.pop(), size)
+        return result
+
+    monkeypatch.setattr(memory.lib, "call", call_and_collect)
+    for block in blocks[:4]:
+        memory.release(block, size)
+    dying.append(blocks[5])
+    memory.release(blocks[4], size)   # evicts one, and another for the block that dies meanwhile
+    assert not dying and memory._POOL_BYTES == sum(live.values()) <= memory._POOL_LIMIT
+    assert sum(len(bucket) for bucket in memory._POOL.values()) == len(live) == 4
+    dying.append(memory.allocate(size))
+    memory.empty_cache()
+    assert not live and memory._POOL_BYTES == 0
