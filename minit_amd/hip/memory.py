@@ -9,7 +9,7 @@ blocks go to a small size-keyed free list so a steady-state loop does not call
 import ctypes
 import threading
 from collections import OrderedDict
-from typing import List
+from typing import Dict, List, Optional
 
 from .. import lib
 
@@ -20,27 +20,39 @@ from .. import lib
 _POOL: "OrderedDict[int, List[int]]" = OrderedDict()
 _POOL_BYTES = 0
 _POOL_LIMIT = 4 << 30
+# Blocks handed out for less than their size: pointer -> size.
+_LENT: Dict[int, int] = {}
 # Reentrant: a tensor may die (and release its block) while the lock is held.  Whatever allocates a container
 # may run the collector, so nothing read from the pool before such a place is relied on behind it.
 _POOL_LOCK = threading.RLock()
 
 
 def _round(size: int) -> int:
-    """Block size for ``size`` bytes: multiples of 256, above 1 MiB eighths of a power of two, so that lengths
-    close to each other share blocks (a prompt of another length costs a hipMalloc per block otherwise);
-    exact again above 1 GiB, where an eighth is no longer small change."""
-    if size <= 256:
-        return 256
-    if 1 << 20 < size <= 1 << 30:
-        step = 1 << ((size - 1).bit_length() - 4)
-        return (size + step - 1) // step * step
-    return (size + 255) // 256 * 256
+    """Block size for ``size`` bytes: a multiple of 256."""
+    return (size + 255) // 256 * 256 if size > 256 else 256
 
 
 def _malloc(size: int) -> int:
     ptr = ctypes.c_void_p()
     lib.call("mh_malloc", ctypes.byref(ptr), size)
     return ptr.value
+
+
+def _take_larger(size: int) -> Optional[int]:
+    """The smallest free block of up to an eighth more than ``size``: a prompt of another length finds the blocks of a
+    longer one and not a hipMalloc each.  A new block has the size that was asked for, so that weights and
+    caches take no more memory than they need."""
+    global _POOL_BYTES
+    found, most = 0, size + size // 8
+    for block in list(_POOL):
+        if size < block <= most and (not found or block < found) and _POOL[block]:
+            found = block
+    if not found:
+        return None
+    ptr = _POOL[found].pop()
+    _POOL_BYTES -= found
+    _LENT[ptr] = found
+    return ptr
 
 
 def allocate(size: int) -> int:
@@ -50,9 +62,12 @@ def allocate(size: int) -> int:
     with _POOL_LOCK:
         bucket = _POOL.get(size)
         if bucket:
-            ptr = bucket.pop()
             _POOL_BYTES -= size
-            return ptr
+            return bucket.pop()
+        if size > 1 << 20:
+            ptr = _take_larger(size)
+            if ptr is not None:
+                return ptr
     try:
         return _malloc(size)
     except lib.HipError:
@@ -63,14 +78,18 @@ def allocate(size: int) -> int:
 def release(ptr: int, size: int) -> None:
     global _POOL_BYTES
     size = _round(size)
-    bucket: List[int] = []
     with _POOL_LOCK:
-        if size > _POOL_LIMIT:
-            lib.call("mh_free", ptr)
-            return
+        if _LENT:
+            size = _LENT.pop(ptr, size)
         if _POOL_BYTES + size > _POOL_LIMIT:
+            if size > _POOL_LIMIT:
+                lib.call("mh_free", ptr)
+                return
             _make_room(size)
-        _POOL.setdefault(size, bucket).append(ptr)
+        bucket = _POOL.get(size)
+        if bucket is None:
+            bucket = _POOL.setdefault(size, [])
+        bucket.append(ptr)
         _POOL.move_to_end(size)
         _POOL_BYTES += size
 

@@ -22,6 +22,7 @@ def device(monkeypatch):
     monkeypatch.setattr(memory.lib, "call", call)
     monkeypatch.setattr(memory, "_POOL", type(memory._POOL)())
     monkeypatch.setattr(memory, "_POOL_BYTES", 0)
+    monkeypatch.setattr(memory, "_LENT", {}, raising=False)
     return live, calls
 
 
@@ -55,6 +56,37 @@ def test_blocks_above_the_limit_are_given_back(device):
     live, calls = device
     memory.release(memory.allocate(5 << 30), 5 << 30)
     assert not live and memory._POOL_BYTES == 0
+
+
+@pytest.mark.parametrize("size", [1, 300, 5120 * 13696, 5120 * 13824 // 2, (1 << 20) + 1, 200_000_001])
+def test_new_blocks_are_no_larger_than_asked_for(device, size):
+    """Weights and caches stay: 8-bit 5120 x 13696 takes its 70.1 MB and not the 75.5 of a rounder size."""
+    live, _ = device
+    memory.allocate(size)
+    assert sum(live.values()) <= max(256, size + 255)
+
+
+def test_close_sizes_share_blocks(device):
+    live, calls = device
+    large, small = 100 << 20, 90 << 20   # within an eighth
+    block = memory.allocate(large)
+    memory.release(block, large)
+    assert memory.allocate(small) == block and calls.count("mh_malloc") == 1 and memory._POOL_BYTES == 0
+    memory.release(block, small)
+    assert memory._POOL_BYTES == large == sum(live.values())   # a block keeps its size
+    other = memory.allocate(80 << 20)                          # more than an eighth less
+    assert other != block and memory.allocate(large) == block
+    memory.release(block, large)
+    memory.release(other, 80 << 20)
+    memory.empty_cache()
+    assert not live and memory._POOL_BYTES == 0
+
+
+def test_small_sizes_do_not_share(device):
+    _, calls = device
+    memory.release(memory.allocate(1 << 20), 1 << 20)
+    memory.allocate((1 << 20) - 4096)
+    assert calls.count("mh_malloc") == 2
 
 
 def test_a_tensor_dies_while_a_block_is_put_back(device, monkeypatch):
