@@ -200,6 +200,9 @@ int mh_f16_matmul_nk(mh_stream_t stream, const void* a, const void* b, void* out
  * for the whole batch (at most 65535 matrices). */
 int mh_f16_matmul_nk_batched(mh_stream_t stream, const void* a, const void* b, void* out,
                              int batch, int M, int N, int K);
+/* rows << 16 | LDS stages of the output tiles (by 128 columns) where the kernel of tiles serves a shape, operands on
+ * 16-byte boundaries; 0 where another one does. */
+int mh_f16_matmul_tile(int batch, int M, int N, int K);
 
 /* ---- W8A8 int8 GEMM --------------------------------------------------------------
  * No counterpart in the reference (its "int8" model is weight-only,

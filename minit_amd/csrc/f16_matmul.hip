@@ -245,6 +245,7 @@ int f16_matmul_lds_launch(hipStream_t stream, const void* a, const void* b, void
 // f16_matmul_tiled.hip
 bool f16_matmul_tiled_supported(int M, int N, int K);
 bool f16_matmul_tiled_preferred(int M, int N, int K);
+int f16_matmul_tiled_tile(int batch, int M, int N, int K);
 int f16_matmul_tiled_launch(hipStream_t stream, const void* a, const void* b, void* out, int batch, int M, int N, int K);
 }  // namespace mh
 
@@ -343,4 +344,9 @@ extern "C" int mh_f16_matmul_nk_batched(mh_stream_t stream, const void* a, const
     }
     // the single product's choice of kernel and tiling: a matrix of a batch gets the bits it gets alone
     return launch_dense_mfma(st, a, b, out, batch, M, N, K);
+}
+
+extern "C" int mh_f16_matmul_tile(int batch, int M, int N, int K) {
+    if (batch <= 0 || !f16_matmul_tiled_supported(M, N, K)) return 0;
+    return K % 32 != 0 || f16_matmul_tiled_preferred(M, N, K) ? f16_matmul_tiled_tile(batch, M, N, K) : 0;
 }

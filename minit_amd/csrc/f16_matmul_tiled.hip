@@ -254,6 +254,11 @@ static TiledPlan plan_tiled(int batch, int M, int N, int K) {
     return best;
 }
 
+int f16_matmul_tiled_tile(int batch, int M, int N, int K) {
+    const TiledPlan p = plan_tiled(batch, M, N, K);
+    return p.bm << 16 | p.stages;
+}
+
 static int tiled_launch_part(hipStream_t stream, const TiledPlan& p, const half_t* a, const half_t* b, half_t* out, int batch,
                              int M, int N, int K) {
     const int tiles_m = (int)(((long long)M + p.bm - 1) / p.bm), tiles_n = tiled_columns(N);

@@ -55,6 +55,7 @@ PROTOTYPES = {
     "mh_gptq_matmul_silu_pairs": (c_int, [_P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P, c_size_t]),
     "mh_f16_matmul_nk": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int]),
     "mh_f16_matmul_nk_batched": (c_int, [_P, _P, _P, _P, c_int, c_int, c_int, c_int]),
+    "mh_f16_matmul_tile": (c_int, [c_int, c_int, c_int, c_int]),
     "mh_i8_gemm": (c_int, [_P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int]),
     "mh_i8_gemm_tile": (c_int, [c_int, c_int, c_int]),
     "mh_i8_transpose": (c_int, [_P, _P, _P, c_int, c_int]),
@@ -92,7 +93,7 @@ PROTOTYPES = {
 }
 
 # functions whose return value is not a status code
-_NOT_STATUS = {"mh_abi_version", "mh_i8_gemm_tile", "mh_last_error", "mh_gptq_workspace_bytes", "mh_gptq_static_scratch_bytes", "mh_gptq_silu_pairs_workspace_bytes", "mh_llama_scratch_bytes",
+_NOT_STATUS = {"mh_abi_version", "mh_i8_gemm_tile", "mh_f16_matmul_tile", "mh_last_error", "mh_gptq_workspace_bytes", "mh_gptq_static_scratch_bytes", "mh_gptq_silu_pairs_workspace_bytes", "mh_llama_scratch_bytes",
                "mh_attn_decode_workspace_bytes"}
 
 DTYPE_CODES = {"float16": 0, "bfloat16": 1, "float32": 2}

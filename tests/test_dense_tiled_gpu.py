@@ -1,6 +1,7 @@
 """The tiled dense fp16 product (csrc/f16_matmul_tiled.hip) where it can go wrong: lengths of K around its rounds of
-64 and its 16-byte pieces, rows that start on odd 2-byte boundaries, ragged tiles of every height, batches whose
-matrices lie back to back (what follows a row must not leak into it), against the float64 product."""
+64 and its 16-byte pieces, rows that start on odd 2-byte boundaries, ragged tiles of every height (asked for and
+asserted), batches whose matrices lie back to back (what follows a row must not leak into it), against the
+float64 product; and the one thread per output below eight k."""
 import numpy as np
 import pytest
 import torch
@@ -13,10 +14,28 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("batch,m,n,k", [
     (1, 1, 1, 8), (2, 5, 7, 9), (3, 33, 129, 63),          # shorter than a round: the remainder alone
     (2, 32, 128, 65), (2, 31, 130, 71), (1, 64, 127, 127),  # one round and 1, 7, 63 elements
-    (2, 65, 129, 128), (3, 128, 256, 192), (1, 129, 5, 193), (32, 1500, 100, 130), (2, 96, 130, 200), (3, 97, 129, 129),  # 128-row tiles, two and three rounds, odd rows
+    (2, 65, 129, 128), (3, 128, 256, 192), (1, 129, 5, 193), (32, 1500, 100, 130), (2, 96, 130, 200), (3, 97, 129, 129),  # two and three rounds, odd rows
     (2, 200, 300, 1001), (4, 257, 128, 1500), (2, 130, 128, 4096),  # the p v of a prompt
     (1, 2100, 4200, 256), (1, 100, 24600, 512)])            # two tiles per CU; one block of rows
 def test_tiled_dense_product(hip, batch, m, n, k):
+    _check(hip, batch, m, n, k)
+
+
+@pytest.mark.parametrize("batch,m,n,k,tile", [
+    (2, 65, 129, 127, (64, 1)), (3, 33, 129, 63, (64, 1)),      # one stage in LDS
+    (4, 257, 128, 1500, (32, 2)), (2, 31, 130, 131, (32, 2)),
+    (8, 1245, 120, 131, (64, 2)), (1, 1250, 1500, 1001, (64, 2)),   # row blocks that end 35 and 30 rows early
+    (40, 420, 128, 333, (96, 2)), (32, 1500, 100, 130, (96, 2)),
+    (16, 1999, 100, 257, (128, 2)), (30, 1000, 128, 193, (128, 2)),
+    (1, 5, 7, 1, (0, 0)), (3, 33, 129, 7, (0, 0)),              # below eight k
+])
+def test_every_height(hip, batch, m, n, k, tile):
+    """Whole blocks of rows and a ragged one, several rounds and a remainder of K, odd rows."""
+    assert divmod(hip.call("mh_f16_matmul_tile", batch, m, n, k), 1 << 16) == tile
+    _check(hip, batch, m, n, k)
+
+
+def _check(hip, batch, m, n, k):
     from minit_amd.hip.tensor import HIPTensor
     rng = np.random.default_rng(m * 7 + k)
     a = rng.normal(0, 1, size=(batch, m, k)).astype(np.float16)

@@ -20,15 +20,16 @@ def test_gather_columns(hip, rows, cols, dtype):
     np.testing.assert_array_equal(out.numpy(), x[:, np.clip(index, 0, cols - 1)])
 
 
-@pytest.mark.parametrize("rows,cols", [(4096, 376), (4097, 376), (4100, 384), ((1 << 24) + 3, 8), (1 << 24, 384)])
+@pytest.mark.parametrize("rows,cols", [(33, 512), (7, 4104), (4096, 376), (4097, 376), (4100, 384), ((1 << 24) + 3, 8), (1 << 24, 384)])
 def test_gather_many_rows(hip, rows, cols):
-    """The widths and row counts at which the kernel changes; more rows than a launch of a workgroup each can hold."""
+    """bfloat16 on every kernel: four columns per thread, the widths and row counts at which a row parked in LDS takes
+    over from it and from one element per thread, more rows than a launch of a workgroup each can hold."""
     x = torch.randint(-2 ** 31, 2 ** 31, (rows, cols // 2), dtype=torch.int32, device="cuda").view(torch.float16)
     index = torch.randperm(cols, device="cuda").to(torch.int32)
     out = torch.zeros_like(x)
     torch.cuda.synchronize()
     hip.call("mh_gather_columns", None, x.data_ptr(), index.data_ptr(), out.data_ptr(), rows, cols, 1)
     torch.cuda.synchronize()
-    for r in range(0, rows, 1 << 20):   # bits: bfloat16 on the device, compared as integers
+    for r in range(0, rows, 1 << 20):   # the bits, compared as integers
         want = x[r:r + (1 << 20)].view(torch.int16)[:, index.long()]
         assert torch.equal(out[r:r + (1 << 20)].view(torch.int16), want), r

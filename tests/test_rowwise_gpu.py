@@ -247,7 +247,7 @@ def test_batch_matrix_multiply(hip):
 @pytest.mark.parametrize("batch,m,n,k", [(6, 5, 40, 128),      # q.k^T of a short prefill, one 16-row tile
                                          (64, 70, 70, 128),    # 64 heads, four row tiles, ragged
                                          (3, 33, 129, 64),     # two row tiles, ragged columns
-                                         (4, 7, 9, 20),        # K not a multiple of 32: the generic kernel
+                                         (4, 7, 9, 20),        # K not a multiple of 32: the tiled kernel
                                          (1, 12, 300, 96),     # a batch of one
                                          (3, 24, 100, 1024),   # 17 rows and more, K of 384 and more: the weight through LDS
                                          (2, 70, 130, 512),    # the same with two blocks of rows and two tiles of columns, both ragged
