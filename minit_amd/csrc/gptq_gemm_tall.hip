@@ -755,23 +755,29 @@ static bool tall_two_row_tiles_preferred(int M, int N, int K) {
 // 20.5 / 27.5, 29.4 / 33.1, 19.6 / 22.3, 16.9 / 24.3, 43.6 / 51.2, 18.2 / 21.6, 4096 x 4096 11.8 / 12.3.  It loses where a
 // launch is all fixed costs (4096 x 4096 at 16 rows 10.5 / 9.5, 2048 x 1024 at 32 rows 8.7 / 7.3), where there are
 // more column tiles than CUs (8192 x 57344 at 16 / 32 rows 79.8 / 73.1, 86.5 / 78.7), and where the workgroups leave
-// a fifth of the CUs idle over a long walk: a CU takes 0.62 us per round however few others ask, the small-M kernel
-// spreads the weight over all of them (13696 x 17992, 141 workgroups of 107 rounds, at 10 rows 65.1 / 48.9; 24832 x 17128
-// at 12 rows 112 / 78).  Of 1050 shapes 128 were more than 5 % slower here without that line, 15 with it.  Up to
-// eight rows the gain is within a few per cent either way and the other kernels' epilogues stay in one launch.
-static bool tall_8bit_preferred(int M, int N, int K) {
+// a quarter of the CUs idle over a long walk (of groups of 32, which the small-M kernel is slower with, three eighths): a
+// CU takes 0.62 us per round however few others ask, the small-M kernel spreads the weight over all of them (13696 x 17992,
+// 141 workgroups of 107 rounds, at 10 rows 65.1 / 48.9; 24832 x 17128 at 12 rows 112 / 78).  Of 1050 shapes 128 were
+// more than 5 % slower here without that line, 25 with it.  Up to eight rows the gain is within a few per cent either
+// way and the other kernels' epilogues stay in one launch.
+static bool tall_8bit_preferred(int M, int N, int K, int group_size) {
     if (M < 9 || M > 32 || (N + kTallBN - 1) / kTallBN > compute_units()) return false;
     if ((size_t)N * K < (M <= 16 ? (size_t)24 << 20 : (size_t)16 << 20)) return false;
     const TallPlan p = plan_tall(M, N, K, 8);
-    return (long)p.tiles_n * p.split_k * 5 >= (long)compute_units() * 4 || p.rounds_per_block <= (M <= 16 ? 24 : 40);
+    return (long)p.tiles_n * p.split_k * 8 >= (long)compute_units() * (group_size < 64 ? 5 : 6) ||
+           p.rounds_per_block <= (M <= 16 ? 24 : 40);
 }
 
-// The same of more rows: fewer workgroups than two thirds of the CUs over 64 rounds and more (10496 x 19032, 149
-// workgroups, at 39 rows 66.8 us against 54.7 on the 64-row blocks; 20352 x 8864 at 151 rows 140 / 116; with 171 workgroups
-// and more, and with shorter walks, never slower by more than 3 % but for a handful of 10,000 shapes).
-static bool tall_8bit_idle(int M, int N, int K) {
+// The same of more rows: fewer workgroups than three quarters of the CUs over 64 rounds and more, where the small-M kernel's
+// blocks of 64 rows and 256 columns are few enough to split K (10496 x 19032, 149 workgroups, at 39 rows 66.8 us against
+// 54.7 there; 20352 x 8864 at 151 rows 140 / 116).  Of 10,000 shapes 33 are on this side of the line, 31 of them 5 to 40 %
+// faster there and none slower; groups shorter than 128 and more blocks turn it round (19840 x 1416 at 1423
+// rows 142 us here and 179 there).
+static bool tall_8bit_idle(int M, int N, int K, int group_size) {
     const TallPlan p = plan_tall(M, N, K, 8);
-    return (long)p.tiles() * (p.split_all() ? p.split_k : 1) * 3 < (long)compute_units() * 2 && K / kTallRoundK >= 64;
+    const long blocks = (((long)M + 63) / 64) * (((long)N + 255) / 256);
+    return p.split_k == 1 && (long)p.tiles() * 4 < (long)compute_units() * 3 && K / kTallRoundK >= 64 && group_size >= 128 &&
+           blocks * 2 <= compute_units();
 }
 
 // Measured on one box against what served these shapes before (the small-M kernel's 64-row blocks up to
@@ -798,7 +804,7 @@ bool gemm_tall_preferred(int M, int N, int K, int group_size, int bits, int epil
         return false;
     if (tall_min_m_env() > 0) return M >= tall_min_m_env();
     if (bits == 4) return M >= 33 || tall_two_row_tiles_preferred(M, N, K);
-    return M >= 33 ? !tall_8bit_idle(M, N, K) : tall_8bit_preferred(M, N, K);
+    return M >= 33 ? !tall_8bit_idle(M, N, K, group_size) : tall_8bit_preferred(M, N, K, group_size);
 }
 
 static size_t tall_plan_bytes(const TallPlan& p, int M, int N) {
