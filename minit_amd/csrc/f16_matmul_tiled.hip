@@ -10,8 +10,8 @@
 // tokens -- and those loads want dword addresses; a 16-byte vector load takes any.
 // The K % 64 remainder is the first round: its chunks are loaded from inside the row and shifted down by
 // whole elements, so that what lies past the end of a row is zero in both operands whatever memory holds.
-// What bounds it: q k^T of a prompt its result (32 x [1500, 1500, 128] 46 us for 144 MB of scores, the part's
-// pure write rate is 7 TB/s; without the streaming hint on the stores half as long again at 2048), p v the read of p
+// What bounds it: q k^T of a prompt its 144 MB of scores (32 x [1500, 1500, 128] 46 us: a tile is one
+// chain of load, two rounds and store, four workgroups per CU overlap: 3.1 TB/s; without the streaming hint on the stores half as long again at 2048), p v the read of p
 // (32 x [1500, 128, 1500] 47 us, with rows on 128-byte lines, K = 1536, 41), a product of many rows and columns the operands on their way into LDS
 // (2048 x 4096 x 4096 87 us, 790 TFLOP/s).  K not a multiple of 32 took one thread per output before: 27.6 ms
 // for that p v.

@@ -37,7 +37,8 @@
 // halves of their accumulators, so that each ends up with its own share of the row tiles), the tile is
 // turned into row-major order in LDS and leaves as 16-byte row pieces: fp16 results (plus bias), with
 // kEpilogueSiluPairs silu(gate) * up of a tile made of 64 gate and the 64 matching up columns, or,
-// with K split over blockIdx.y, fp32 partial sums for splitk_finalize_kernel.
+// with K split, fp32 partial sums: for splitk_finalize_kernel where every tile is split (blockIdx.y), for
+// tall_finish_kernel where only the tiles of the last pass over the CUs are.
 //
 // 8-bit weights against the small-M kernel's 64-row blocks that served them before (us, now / before): 2048 x 4096 x
 // 28672 447 / 646, 2048 x 14336 x 4096 197 / 269, 1000 x 5120 x 15360 146 / 216, 128 x 4096 x 28672 36.9 / 57.0, 64 x
@@ -163,8 +164,8 @@ __device__ __forceinline__ void tall_lds_wait(half8_t* a) {
         asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a[0]), "+v"(a[1]) : "n"(NEWEST) : "memory");
 }
 
-// MT: 16-row MFMA tiles per block of rows (8: blocks of 128 rows; 4: one block of up to 64 rows; 2: up to 32
-// rows, reached only when MH_GEMM_TALL_MIN_M is lowered), the same walk with fewer MFMAs per dequantised word.
+// MT: 16-row MFMA tiles per block of rows (16: blocks of 256 rows; 8: of 128; 4: one block of up to 64 rows; 2: up to 32,
+// the shapes of tall_two_row_tiles_preferred and tall_8bit_preferred), the same walk with fewer MFMAs per dequantised word.
 // NS: rounds in flight = slots of the register ring = activation stages in LDS.  Four everywhere: eight (the
 // LDS allows them below eight row tiles) measured slower, 32 x 8192 x 57344 90.3 against 77.8 us and 64 x 8192 x
 // 10240 30.3 against 29.0 -- what holds the kernel back at few rows is its ~105 vector instructions per
@@ -784,8 +785,7 @@ static bool tall_8bit_idle(int M, int N, int K, int group_size) {
 // 191 rows, the LDS-staged kernel above; us, this kernel / before): 4096 x 28672 at 65 / 128 / 256 / 2048
 // rows 38.7 / 58.6, 41.2 / 62.3, 75.2 / 80.5, 561 / 567; 4096 x 14336: 29.1 / 33.0, 36.5 / 35.9, 40.1 /
 // 55.3, 278 / 310; 14336 x 4096: 28.3 / 33.8, 32.2 / 33.1, 43.1 / 60.0, 242 / 283; 8192 x 8192 at 512 rows
-// 72.0 / 113.5.  Never slower by more than 2 %, so every 4-bit product of more than 64 rows whose K is a
-// multiple of 128 comes here.  With four row tiles (33 to 64 rows) against the small-M kernel's single block
+// 72.0 / 113.5.  Every 4-bit product of more than 64 rows whose K is a multiple of 128 comes here.  With four row tiles (33 to 64 rows) against the small-M kernel's single block
 // of 64 rows, at 64 rows: 8192 x 10240 29.0 / 41.6, 28672 x 8192 55.7 / 62.3, 4096 x 14336 23.9 / 26.3, 8192 x
 // 57344 109 / 112; with two row tiles at 32 rows it loses on the largest shapes (8192 x 57344 77.8 / 67.9, 28672
 // x 8192 48.6 / 43.5: there the weight stream dominates and the small-M kernel's ring of eight loads per
@@ -819,7 +819,8 @@ size_t gemm_tall_least_workspace_bytes(int M, int N, int K, int bits) {
     return tall_plan_bytes(plan_tall(M, N, K, bits, false), M, N);
 }
 
-// kEpilogueSiluPairs in the kernel's own store: an unsplit plan, whole blocks of 128 + 128 columns.
+// kEpilogueSiluPairs in the kernel's own store, or in tall_finish_kernel for a last pass in K ranges: a plan that does not
+// split every tile, whole blocks of 128 + 128 columns.
 bool gemm_tall_silu_pairs_supported(int M, int N, int K, int group_size, int bits) {
     return gemm_tall_preferred(M, N, K, group_size, bits, kEpilogueNone) && N % 256 == 0 && !plan_tall(M, N, K, bits).split_all();
 }
