@@ -9,10 +9,7 @@ requires exactly one.  Implementations return a tuple of tensors.
 """
 from typing import Callable, Dict, List, Optional, Tuple, Type
 
-try:
-    from .._binding import dispatcher
-except ImportError:   # not built yet
-    dispatcher = None
+from ..lib import _binding
 from .object import FunctionSignature, Object, extract_function_signature, match_function_args
 
 DISPATCH_CACHE: Dict[Tuple[Type, ...], Callable] = {}
@@ -42,8 +39,8 @@ def _dispatch(*args: Object):
     return func(*args)
 
 
-# the same steps in native code (csrc/binding.cpp) where the package has been built
-dispatch = _dispatch if dispatcher is None else dispatcher(DISPATCH_CACHE, lookup_implementation_from_types)
+# the same steps in native code (csrc/binding.cpp); a process that has no extension module at import stays with the ones above
+dispatch = _dispatch if _binding is None else _binding.dispatcher(DISPATCH_CACHE, lookup_implementation_from_types)
 
 
 def register_dispatch(*, predicate: Optional[Callable] = None, priority: int = DEFAULT_PRIORITY):

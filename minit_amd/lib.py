@@ -8,9 +8,10 @@ There is no fallback: if the library is missing, loading raises.
 
 ``call`` is the extension module ``_binding`` (csrc/binding.cpp, built next to the
 library): it converts plain numbers and pointers itself and hands every other call to
-:func:`_call_general`, the ctypes path.
+:func:`_call_general`, the ctypes path.  Without the module that path takes every call.
 """
 import ctypes
+import importlib
 import os
 from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_size_t, c_uint32, c_uint64, c_void_p
 
@@ -102,12 +103,19 @@ _NOT_STATUS = {"mh_abi_version", "mh_i8_gemm_tile", "mh_f16_matmul_tile", "mh_la
 
 DTYPE_CODES = {"float16": 0, "bfloat16": 1, "float32": 2}
 
-try:
-    from . import _binding
-except ImportError:   # not built yet: cdll() says so
-    _binding = None
-
+_binding = None   # the extension module, once it is there
 _cdll = None
+
+
+def _load_binding() -> None:
+    global _binding
+    importlib.invalidate_caches()   # it may have been built since its folder was looked at
+    try:
+        module = importlib.import_module("._binding", __package__)
+    except ImportError:   # not built (yet)
+        return
+    module.set_hooks(_call_general, _failed)
+    _binding = module
 
 
 def cdll() -> ctypes.CDLL:
@@ -118,15 +126,16 @@ def cdll() -> ctypes.CDLL:
             raise HipError(
                 f"{LIB_PATH} is missing: build it with `python -m minit_amd.build` "
                 "(there is no CPU fallback for this path)")
-        if _binding is None:
-            raise HipError("minit_amd/_binding is missing: build it with `python -m minit_amd.build`")
         lib = ctypes.CDLL(LIB_PATH)
         for name, (restype, argtypes) in PROTOTYPES.items():
             fn = getattr(lib, name)
             fn.restype = restype
             fn.argtypes = argtypes
         _cdll = lib
-        _binding.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in PROTOTYPES})
+        if _binding is None:   # a process that has imported the package before it was built
+            _load_binding()
+        if _binding is not None:
+            _binding.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in PROTOTYPES})
     return _cdll
 
 
@@ -152,11 +161,13 @@ def _call_general(name: str, *args):
     return rc
 
 
-if _binding is not None:
-    _binding.set_hooks(_call_general, _failed)
-    call = _binding.call
-else:
-    call = _call_general
+def _call_late(name: str, *args):
+    """``call`` where the module was not there at import: other modules hold on to this function, so it looks each time."""
+    return (_call_general if _binding is None else _binding.call)(name, *args)
+
+
+_load_binding()
+call = _call_late if _binding is None else _binding.call
 
 
 def device_count() -> int:
