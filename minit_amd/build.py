@@ -14,6 +14,7 @@ import subprocess
 import sys
 import sysconfig
 from concurrent.futures import ThreadPoolExecutor
+from typing import Optional
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -99,23 +100,33 @@ def _build_locked(force: bool, verbose: bool, jobs: int) -> str:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
+    binding = _build_binding(hipcc, verbose)
+    # both or neither: the module has the library's prototypes compiled in
     os.replace(tmp, LIB_PATH)
-    _build_binding(hipcc, verbose)
+    if binding:
+        os.replace(binding, BINDING_PATH)
+    elif os.path.exists(BINDING_PATH):
+        os.remove(BINDING_PATH)
     return LIB_PATH
 
 
-def _build_binding(hipcc: str, verbose: bool) -> None:
-    """The CPython module (host code only) that ``lib.call`` goes through."""
+def _build_binding(hipcc: str, verbose: bool) -> Optional[str]:
+    """Compiles the CPython module (host code only) that ``lib.call`` goes through, to a name of its own.  None where
+    Python's headers are not installed: the calls go through ctypes then."""
+    include = sysconfig.get_paths()["include"]
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"{include}/Python.h is missing: calls into the library go through ctypes", file=sys.stderr)
+        return None
     tmp = BINDING_PATH + ".tmp"
     # host code that must not bring a HIP runtime of its own into the process: torch has one, the library links one
-    cmd = [hipcc, "-no-hip-rt", "-x", "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", sysconfig.get_paths()["include"],
+    cmd = [hipcc, "-no-hip-rt", "-x", "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", include,
            os.path.join(CSRC, "binding.cpp"), "-o", tmp]
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"building the Python binding failed:\n{proc.stdout}\n{proc.stderr}")
-    os.replace(tmp, BINDING_PATH)
+    return tmp
 
 
 if __name__ == "__main__":

@@ -72,3 +72,22 @@ def test_the_library_without_the_module(tree):
     _run(tree, "from minit_amd import build\nbuild.build(verbose=False)\n")
     os.remove(tree[0] / "minit_amd" / os.path.basename(build.BINDING_PATH))
     _run(tree, CALLS + "assert lib._binding is None\n")
+
+
+def test_a_module_that_does_not_compile_replaces_nothing(tree):
+    package = tree[0] / "minit_amd"
+    built = [package / os.path.basename(p) for p in (build.LIB_PATH, build.BINDING_PATH)]
+    for path in built:
+        path.write_bytes(b"of the build before")
+    (package / "csrc" / "binding.cpp").write_text("#error\n")
+    _run(tree, "from minit_amd import build\n"
+               "try:\n    build.build(verbose=False)\nexcept RuntimeError as e:\n    assert 'binding' in str(e)\n"
+               "else:\n    raise SystemExit('built')\n")
+    assert [p.read_bytes() for p in built] == [b"of the build before"] * 2
+
+
+def test_no_headers_of_python(tree):
+    """The library does not need them, and no module of an earlier build stays beside it."""
+    _run(tree, "from minit_amd import build\nbuild.build(verbose=False)\n"
+               "build.sysconfig.get_paths = lambda: {'include': 'none'}\nbuild.build(verbose=False)\n")
+    _run(tree, CALLS + "assert lib._binding is None\n")
