@@ -21,7 +21,8 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OBJ_DIR = os.path.join(HERE, "_build")
 LIB_PATH = os.path.join(HERE, "libminit_hip.so")
-BINDING_PATH = os.path.join(HERE, "_binding.so")
+# under the tag of the interpreter it is compiled for: others do not take it for theirs
+BINDING_PATH = os.path.join(HERE, "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 ARCH = "gfx950"
 # -packed-fp32-ops is switched off on purpose: hipcc otherwise forms packed fp32
@@ -107,6 +108,9 @@ def _build_locked(force: bool, verbose: bool, jobs: int) -> str:
         os.replace(binding, BINDING_PATH)
     elif os.path.exists(BINDING_PATH):
         os.remove(BINDING_PATH)
+    untagged = os.path.join(HERE, "_binding.so")   # the name it had before the tag
+    if os.path.exists(untagged):
+        os.remove(untagged)
     return LIB_PATH
 
 

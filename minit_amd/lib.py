@@ -11,8 +11,10 @@ library): it converts plain numbers and pointers itself and hands every other ca
 :func:`_call_general`, the ctypes path.  Without the module that path takes every call.
 """
 import ctypes
-import importlib
+import importlib.util
 import os
+import sys
+import sysconfig
 from ctypes import POINTER, c_char_p, c_double, c_float, c_int, c_size_t, c_uint32, c_uint64, c_void_p
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -103,19 +105,22 @@ _NOT_STATUS = {"mh_abi_version", "mh_i8_gemm_tile", "mh_f16_matmul_tile", "mh_la
 
 DTYPE_CODES = {"float16": 0, "bfloat16": 1, "float32": 2}
 
+# by its full name and not as any _binding: one without the interpreter's tag may be compiled for another
+_BINDING_PATH = os.path.join(_HERE, "_binding" + sysconfig.get_config_var("EXT_SUFFIX"))
 _binding = None   # the extension module, once it is there
 _cdll = None
 
 
 def _load_binding() -> None:
     global _binding
-    importlib.invalidate_caches()   # it may have been built since its folder was looked at
+    spec = importlib.util.spec_from_file_location(f"{__package__}._binding", _BINDING_PATH)
     try:
-        module = importlib.import_module("._binding", __package__)
+        module = importlib.util.module_from_spec(spec)
     except ImportError:   # not built (yet)
         return
+    spec.loader.exec_module(module)
     module.set_hooks(_call_general, _failed)
-    _binding = module
+    sys.modules[spec.name] = _binding = module
 
 
 def cdll() -> ctypes.CDLL:

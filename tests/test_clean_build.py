@@ -91,3 +91,13 @@ def test_no_headers_of_python(tree):
     _run(tree, "from minit_amd import build\nbuild.build(verbose=False)\n"
                "build.sysconfig.get_paths = lambda: {'include': 'none'}\nbuild.build(verbose=False)\n")
     _run(tree, CALLS + "assert lib._binding is None\n")
+
+
+def test_a_module_of_another_interpreter(tree):
+    """Python takes any _binding.so for a module of its own; what has no tag, or another one, is not loaded here."""
+    package = tree[0] / "minit_amd"
+    _run(tree, "from minit_amd import build\nbuild.build(verbose=False)\n")
+    built = package / os.path.basename(build.BINDING_PATH)
+    for name in ("_binding.so", "_binding.cpython-399-x86_64-linux-gnu.so"):
+        built = built.rename(package / name)
+        _run(tree, CALLS + "assert lib._binding is None\n")
