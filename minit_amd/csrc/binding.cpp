@@ -10,6 +10,7 @@
 #include <Python.h>
 
 #include <stddef.h>
+#include <string.h>
 
 #include <tuple>
 #include <type_traits>
@@ -40,6 +41,19 @@ bool convert(PyObject* o, T& v) {
     return true;
 }
 
+// ctypes' code of a type (c_int._type_ and so on).
+template <class T>
+constexpr char code() {
+    if constexpr (std::is_pointer_v<T>) return 'P';
+    else if constexpr (std::is_same_v<T, double>) return 'd';
+    else if constexpr (std::is_same_v<T, float>) return 'f';
+    else if constexpr (std::is_same_v<T, int>) return 'i';
+    else {
+        static_assert(std::is_same_v<T, unsigned long>, "a type without a code");
+        return 'L';
+    }
+}
+
 // Thunk<decltype(f)>::run: converts, calls f with the interpreter lock released, leaves the result; false, and no
 // call, where an argument is not plain.
 template <class F>
@@ -47,6 +61,7 @@ struct Thunk;
 template <class R, class... A>
 struct Thunk<R(A...)> {
     static constexpr int kCount = sizeof...(A);
+    static constexpr char kSignature[] = {code<R>(), code<A>()..., 0};
     template <size_t... I>
     static bool invoke(void* fn, PyObject* const* args, unsigned long* result, std::index_sequence<I...>) {
         [[maybe_unused]] std::tuple<A...> held;
@@ -67,12 +82,13 @@ struct Entry {
     const char* name;
     bool (*run)(void*, PyObject* const*, unsigned long*);
     int count;
+    const char* signature;   // codes of the result and the arguments
     bool status;   // the result is a status code: non-zero raises
     void* fn;      // set once the library is loaded
 };
 
-#define STATUS(f) {#f, Thunk<decltype(f)>::run, Thunk<decltype(f)>::kCount, true, nullptr}
-#define SIZE(f) {#f, Thunk<decltype(f)>::run, Thunk<decltype(f)>::kCount, false, nullptr}
+#define STATUS(f) {#f, Thunk<decltype(f)>::run, Thunk<decltype(f)>::kCount, Thunk<decltype(f)>::kSignature, true, nullptr}
+#define SIZE(f) {#f, Thunk<decltype(f)>::run, Thunk<decltype(f)>::kCount, Thunk<decltype(f)>::kSignature, false, nullptr}
 Entry g_entries[] = {
     STATUS(mh_free), STATUS(mh_memcpy), STATUS(mh_memset), STATUS(mh_stream_synchronize), STATUS(mh_device_synchronize),
     STATUS(mh_event_record), STATUS(mh_event_synchronize), STATUS(mh_copy_kernel), STATUS(mh_gptq_unpack),
@@ -122,19 +138,30 @@ PyObject* set_hooks(PyObject*, PyObject* args) {
     Py_RETURN_NONE;
 }
 
-// bind({name: address}): the entry points of a loaded library.
-PyObject* bind(PyObject*, PyObject* addresses) {
-    if (!PyDict_Check(addresses)) {
-        PyErr_SetString(PyExc_TypeError, "bind: a dict of addresses is expected");
+// bind({name: (address, signature)}): the entry points of a loaded library.  One whose signature is another than the header
+// had when this module was compiled is left to the ctypes path: the two may come from different builds.  Returns how many.
+PyObject* bind(PyObject*, PyObject* entries) {
+    if (!PyDict_Check(entries)) {
+        PyErr_SetString(PyExc_TypeError, "bind: a dict of addresses and signatures is expected");
         return nullptr;
     }
     PyObject* table = PyDict_New();
     if (table == nullptr) return nullptr;
+    long left = 0;
     for (Entry& e : g_entries) {
-        PyObject* address = PyDict_GetItemString(addresses, e.name);
-        if (address == nullptr) continue;
-        void* fn = PyLong_AsVoidPtr(address);
-        PyObject* entry = PyErr_Occurred() ? nullptr : PyLong_FromVoidPtr(&e);
+        PyObject *given = PyDict_GetItemString(entries, e.name), *address;
+        if (given == nullptr) continue;
+        const char* signature;
+        void* fn = nullptr;
+        PyObject* entry = nullptr;
+        if (PyArg_ParseTuple(given, "Os", &address, &signature)) {
+            if (strcmp(signature, e.signature) != 0) {
+                ++left;
+                continue;
+            }
+            fn = PyLong_AsVoidPtr(address);
+            entry = PyErr_Occurred() ? nullptr : PyLong_FromVoidPtr(&e);
+        }
         PyObject* name = entry != nullptr ? PyUnicode_InternFromString(e.name) : nullptr;
         const bool stored = name != nullptr && PyDict_SetItem(table, name, entry) == 0;
         Py_XDECREF(entry);
@@ -146,7 +173,7 @@ PyObject* bind(PyObject*, PyObject* addresses) {
         e.fn = fn;
     }
     Py_XSETREF(g_table, table);
-    Py_RETURN_NONE;
+    return PyLong_FromLong(left);
 }
 
 // dispatcher(cache, lookup) -> dispatch(*args): cache[tuple(arg.type() for arg in args)](*args), the
@@ -216,7 +243,7 @@ PyMethodDef g_methods[] = {
     {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(call)), METH_FASTCALL,
      "call(name, *args): an entry point of the library; a non-zero status raises HipError"},
     {"set_hooks", set_hooks, METH_VARARGS, "set_hooks(general, failed)"},
-    {"bind", bind, METH_O, "bind({name: address})"},
+    {"bind", bind, METH_O, "bind({name: (address, signature)}) -> number left out"},
     {"dispatcher", dispatcher, METH_VARARGS, "dispatcher(cache, lookup) -> dispatch"},
     {nullptr, nullptr, 0, nullptr}};
 

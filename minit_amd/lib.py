@@ -123,6 +123,15 @@ def _load_binding() -> None:
     sys.modules[spec.name] = _binding = module
 
 
+def _signature(restype, argtypes) -> str:
+    """The codes ctypes has for the types ("P" for every pointer); the module binds what it was compiled for."""
+    return "".join(t._type_ if isinstance(t._type_, str) else "P" for t in (restype, *argtypes))
+
+
+def _entries(lib: ctypes.CDLL) -> dict:
+    return {name: (ctypes.cast(getattr(lib, name), c_void_p).value, _signature(*types)) for name, types in PROTOTYPES.items()}
+
+
 def cdll() -> ctypes.CDLL:
     """Loads the shared library (once).  Raises if it has not been built."""
     global _cdll
@@ -140,7 +149,7 @@ def cdll() -> ctypes.CDLL:
         if _binding is None:   # a process that has imported the package before it was built
             _load_binding()
         if _binding is not None:
-            _binding.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in PROTOTYPES})
+            _binding.bind(_entries(lib))
     return _cdll
 
 

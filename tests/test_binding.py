@@ -65,6 +65,26 @@ def test_status_messages_are_the_callers_own():
     assert len(seen) == 4
 
 
+def test_signatures_of_another_build(monkeypatch):
+    """Where the prototypes are not the ones the module was compiled for, calls take the path that converts by the prototypes."""
+    entries = lib._entries(lib.cdll())
+    assert lib._binding.bind(entries) == 0
+    name = "mh_gptq_workspace_bytes"
+    reached = []
+    monkeypatch.setitem(lib._functions, name, lambda *args: reached.append(args))
+    lib.call(name, *SIZES)
+    assert not reached
+    try:
+        for signature in ("Liiii", "Liiiiii", "Liiiif", "iiiiii"):
+            assert lib._binding.bind({**entries, name: (entries[name][0], signature)}) == 1
+            lib.call(name, *SIZES)
+            assert reached.pop() == SIZES and not reached
+        with pytest.raises(Exception):
+            lib._binding.bind({**entries, name: entries[name][0]})
+    finally:
+        lib._binding.bind(entries)
+
+
 class _Op(Object):
     def type(self):
         return _Op
