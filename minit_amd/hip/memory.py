@@ -229,7 +229,9 @@ def workspace(nbytes: int) -> HIPMemory:
     return _WORKSPACE
 
 
-# What a product needs depends on its sizes alone (and on what the process was started with).
+# What a product needs depends on its sizes, on what the process was started with and, up to 32 rows of at most one column
+# tile per CU, on MH_GEMM_SMALL_KW, which is read at every call: there it is below 20 MB at any setting, less than
+# the shared workspace has at least.
 @lru_cache(maxsize=4096)
 def _product_bytes(m: int, n: int, k: int, group_size: int, bits: int) -> int:
     return max(lib.call("mh_gptq_workspace_bytes", m, n, k, group_size, bits), 256)
