@@ -65,6 +65,30 @@ def test_status_messages_are_the_callers_own():
     assert len(seen) == 4
 
 
+def test_a_failure_elsewhere_leaves_the_message():
+    """Between the status of a call and the question for its message, another thread fails with another message."""
+    failed, other_failed = threading.Event(), threading.Event()
+    seen = []
+
+    def first():
+        assert lib.cdll().mh_softmax_causal(None, 256, 256, 1, 2, 7, 3, 1.0, 0) != 0
+        failed.set()
+        assert other_failed.wait(30)
+        seen.append(lib.last_error())
+
+    def second():
+        assert failed.wait(30)
+        with pytest.raises(lib.HipError, match="bits must be 4 or 8"):
+            lib.call("mh_gptq_unpack", None, 256, 256, 4, 4, 0, 5)
+        other_failed.set()
+    threads = [threading.Thread(target=f) for f in (first, second)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(seen) == 1 and "t=7 must equal" in seen[0]
+
+
 def test_signatures_of_another_build(monkeypatch):
     """Where the prototypes are not the ones the module was compiled for, calls take the path that converts by the prototypes."""
     entries = lib._entries(lib.cdll())
