@@ -509,9 +509,16 @@ bool gemm_cols_preferred(int M, int N, int K, int group_size, int bits, int epil
     // 7.4 / 12.0, 6144x2048 10.0 / 12.8 (longer ones go to the 128-row-block kernel).
     // (The fewer CUs have a tile, the sooner: 16384x1472 at 7 rows 16.8 / 12.5, 22784x2432 at one row 18.6 / 15.3, 13312x2304 at 8
     // rows 15.0 / 12.6, 24064x3200 at 4 rows 20.9 / 17.6, 9216x1504 at 16 rows 13.5 / 11.6.)
+    // (Smaller groups, whose scales and zero points this kernel reads itself, leave sooner. Mean of its time over the small-M
+    // kernel's, 4 bit, 3073 to 4096 columns, K to 18432 / 20480 / 22528: groups of 128 0.82 / 0.87 / 0.91, of 64 0.88 / 0.95 / 0.98 and
+    // behind 20480 1.02 up to 3584 columns, of 32 at 3 and 4 rows 0.95 / 1.00 / 1.04, at 1 and 2 rows 0.92 / 0.96 / 1.01 and behind
+    // 20480 1.04 up to 3584 columns; at 5 to 8 rows groups of 32 0.92 to K = 12288 and 1.01 behind it up to 3584 columns, 0.97 over them.)
     if (M <= 8 && cols_narrow(N, cus)) {
-        const bool few = bits == 4 && M > 4;
-        if (N > 12 * cus) return kb <= (few ? 14336 : bits == 4 ? 22528 : 16384);
+        const bool few = bits == 4 && M > 4, wide = N > 14 * cus;
+        if (few && N > 12 * cus) return kb <= (group_size == 32 && !wide ? 12288 : 14336);
+        if (bits == 4 && N > 12 * cus)
+            return kb <= (group_size >= 128 || (wide && (group_size > 32 || M <= 2)) ? 22528 : group_size == 32 && M > 2 ? 18432 : 20480);
+        if (N > 12 * cus) return kb <= 16384;
         return kb <= (few ? 10240 : N > 8 * cus ? 14336 : 12288);
     }
     if (M <= 16 && cols_narrow(N, cus)) return K <= (bits == 4 ? 8192 : 6144);
@@ -522,11 +529,13 @@ bool gemm_cols_preferred(int M, int N, int K, int group_size, int bits, int epil
     // 4096x16384 8.4 / 10.8 and 11.1 / 12.6, 4096x24576 12.0 / 16.8 and 14.5 / 15.6, 3072x18432 10.7 / 14.7 and 10.4 / 11.6,
     // 4096x32768 15.0 / 20.2 and 15.9 / 17.0; with refills 5120x11008 11.4 / 14.2 and 10.3 / 11.9; 512x32768 7.4 / 8.4 and 6.2 / 6.4; 8-bit 2048x11008 6.9 / 7.6 and
     // 8.9 / 10.1, 2048x24576 11.5 / 12.4 and 13.3 / 14.5, 1024x32768 10.2 / 11.2 and 9.6 / 10.4, 4096x13824 14.2 / 15.6 and 13.4 / 15.3.
+    // Between two and three tiles per CU, over 16448 to 24576 columns at 1, 2 and 4 rows, groups of 128 take 0.86 of the time there at
+    // K = 3840 and 0.81 at 4096, smaller ones 1.02 (up to 1.09) and 0.96.
     if (tiles > cus && M <= 8 && epilogue == kEpilogueNone) {
         if (K < 1024) return tiles <= 2 * cus;
         if (bits == 8) return K <= 2048 && tiles <= 3 * cus;
         if (K <= 2048) return tiles <= 4 * cus;
-        return K <= 4096 && (tiles <= 2 * cus || (M <= 4 && K > 3584 && tiles <= 3 * cus));
+        return K <= 4096 && (tiles <= 2 * cus || (M <= 4 && K > (group_size >= 128 ? 3584 : 3840) && tiles <= 3 * cus));
     }
     // 28672x8192 against the small-M kernel: 26.5 / 27.5 us at M = 3, 27.0 / 27.6 at 4, equal at 6, 30.2 / 29.2 at 8
     return tiles <= cus && (kb <= 8192 || 2 * tiles > cus) && (kb <= 16384 || M <= 4);
@@ -535,11 +544,15 @@ bool gemm_cols_preferred(int M, int N, int K, int group_size, int bits, int epil
 // 17 to 32 rows, where the 128-row-block kernel's two row tiles are the other choice: short K, whose sums it adds in a
 // launch of its own. At 32 rows, us, that kernel and this: 4-bit 4096x4096 10.6 / 8.0, 4096x8192 12.9 / 10.5, 2048x6144 9.9
 // / 7.0, 5120x4096 11.2 / 10.7, 6144x4096 11.7 / 11.3, 8192x4096 12.6 / 13.3, 5120x8192 13.6 / 13.8; 8-bit 4096x4096 12.1
-// / 10.5, 5120x4096 12.5 / 13.7.
+// / 10.5, 5120x4096 12.5 / 13.7.  Over 4352 <= K <= 6144 and up to 4096 columns (4 bit) the mean of this kernel's time over that
+// one's is 0.82 below 11.5 million weights and 1.02 (groups of 32 1.04, up to 1.13) above, for groups of 128 at up to 24 rows 0.98;
+// in tiles of 32 columns groups of 32 take up to 1.09 of it for 2304 <= K <= 3328 and up to 6144 columns.
 bool gemm_cols_two_row_tiles_preferred(int M, int N, int K, int group_size, int bits) {
     if (M <= 16 || !gemm_cols_preferred(M, N, K, group_size, bits, kEpilogueNone)) return false;
-    const bool narrow = cols_narrow(N, compute_units());
-    return bits == 4 ? K <= (narrow ? 6144 : 4096) : narrow && K <= 4096;
+    const int cus = compute_units();
+    if (bits == 8) return cols_narrow(N, cus) && K <= 4096;
+    if (!cols_narrow(N, cus)) return K <= 4096 && (group_size > 32 || N > 24 * cus || K <= 2048 || K > 3328);
+    return K <= 4096 || (K <= 6144 && ((long)N * K < (11L << 20) || (group_size >= 128 && M <= 24)));
 }
 
 // Bytes of workspace a launch of this kernel needs for the shape (0: none).

@@ -48,3 +48,15 @@ def test_products(hip, m, k, n, g, bits):
     bias = np.random.default_rng(63).normal(0, 1, n).astype(np.float16)
     got = _run_with_bias(hip, onehot, qweight, qzeros, scales, bias, g, bits)[0]
     np.testing.assert_array_equal(got.view(np.uint16), (w[rows] + bias).view(np.uint16))
+
+
+@pytest.mark.parametrize("m,k,n,g,bits", [
+    # the longest K of groups of 32 and 64, and the first that leaves
+    (3, 18432, 3104, 32, 4), (4, 18688, 3104, 32, 4), (1, 20480, 3104, 32, 4), (4, 20736, 3104, 64, 4), (2, 20736, 3616, 32, 4),
+    (5, 12288, 3104, 32, 4), (8, 12544, 3104, 32, 4), (6, 12544, 3616, 32, 4), (1, 3840, 16416, 64, 4), (4, 4096, 16416, 32, 4),
+    # 17 to 32 rows: both sides of the lines
+    (20, 2048, 4128, 32, 4), (32, 2304, 6144, 32, 4), (32, 3328, 6176, 32, 4), (17, 3584, 6144, 32, 4),
+    (32, 6144, 1856, 64, 4), (17, 6144, 1888, 64, 4), (24, 6144, 2080, 128, 4), (25, 6144, 2080, 128, 4), (24, 4352, 2080, 256, 4),
+])
+def test_products_at_the_lines_of_small_groups(hip, m, k, n, g, bits):
+    test_products(hip, m, k, n, g, bits)
