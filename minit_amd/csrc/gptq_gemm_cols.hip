@@ -5,14 +5,14 @@
 // and needs 11-16 K splits per tile to fill the GPU; the partial sums then cross
 // workgroups (agent-scope stores, an arrival counter, a reload by the last
 // workgroup), three dependent memory round trips of about a microsecond each at
-// the end of a 10 us kernel.  Here K is split over the eight waves of the one
-// workgroup that owns the columns and the partial sums meet in LDS.
+// the end of a 10 us kernel.  Here K is split over the waves (eight, 16 or four:
+// plan_cols) of the one workgroup that owns the columns and the partial sums meet in LDS.
 //
 // A wave walks its own contiguous K range, so it shares nothing with the other
 // waves until the end and the K loop has no barrier.  Per step of 32 k a lane
 // (column pair nl = lane % 16, k chunk kq = lane / 16) loads 8 bytes: the packed
 // words of its two columns, which are the B operands of two
-// v_mfma_f32_16x16x32_f16.  Everything a step needs is requested 8 steps ahead
+// v_mfma_f32_16x16x32_f16 (tiles of 16 columns: one word, one of them).  Everything a step needs is requested 8 steps ahead
 // and in the order of use (activations of a 256-k stage, scale/zero words of a
 // group, packed weights), so each s_waitcnt vmcnt(n) leaves the 8 steps behind it
 // in flight: 4 KiB per wave, 32 KiB per CU.  More in flight measured slower (16
@@ -345,7 +345,7 @@ __global__ __launch_bounds__(WAVES * 64) void gptq_gemm_cols_kernel(const ColsAr
         }
     }
 
-    // ---- the eight partial sums of a column meet in LDS, in wave order
+    // ---- the waves' partial sums of a column meet in LDS, in wave order
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(WAVES * 64) void gptq_gemm_cols_kernel(const ColsAr
     half2_t* op = reinterpret_cast<half2_t*>(out + (size_t)m * N + col);
     if (epilogue == kEpilogueResidual) {
         // out is the residual stream: h += y in fp16, h * next_norm_w for the consumer,
-        // and the sum of squares of the tile's 32 new values (the row's 16 threads
+        // and the sum of squares of the tile's TILE new values (the row's TILE / 2 threads
         // are adjacent lanes of one wave)
         const half2_t h = ep_h + y;  // ep_h: this thread's two elements of the stream, read at the start
         *op = h;
@@ -477,8 +477,12 @@ int gemm_cols_tile(int N) { return cols_narrow(N, compute_units()) ? 16 : kColsT
 struct ColsPlan {
     int tile, waves, ring;
 };
-// See the head of this file; more than eight rows do not fit the LDS of 16 waves.  16 waves with 16 steps each from
-// 12 steps a wave on: 5120x4096 would leave six of them idle (6.2 against 5.6 us with eight and refills).
+// See the head of this file.  More than eight rows of 32 columns do not fit the LDS of 16 waves (168 KB); of 16 columns they
+// would (152 KB), and gain behind K = 2048 (us, eight waves with refills / 16 with one ring, 4096x4096 and 4096x1024 at 16
+// rows: 7.0 / 6.2, 6.4 / 5.6 at 4 bit, 10.0 / 8.6, 8.4 / 7.2 at 8 bit; 2048x4096 5.5 / 5.8): not built yet.
+// 16 waves with 16 steps each from 12 steps a wave on: 5120x4096 would leave six of them idle (6.2 against 5.6 us
+// with eight and refills).  (8-bit groups of 32 at five to eight rows spill ten registers there, and gain all the same: with
+// eight waves and refills 6400x4096 14.2 / 15.0, 7168x3072 13.8 / 14.6, 7168x4096 15.1 / 15.4, 8192x4096 16.0 / 15.9 at 8 rows.)
 static ColsPlan plan_cols(int M, int N, int K, int cus, bool cut) {
     const int steps = K / 32, tile = cols_narrow(N, cus) ? 16 : kColsTile;
     if (cut) return {kColsTile, cols_waves(M, true), 0};

@@ -201,9 +201,12 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_strided_kernel(
 // Over [48000, 1500] with the causal mask 232 -> 50 us (one element per thread, three walks, before).
 // CAUSAL: a piece that lies past the last visible column is not read.
 // Rows that are not whole lines are stored without the streaming hint, which sends the parts of a line to memory one by
-// one, as long as the result fits the memory-side cache of 256 MiB, where what reads it next finds it: a prompt's attention
-// (rotation, q k^T, this, p v) of 32 heads x 1500 tokens 172 -> 157 us, x 1777 231 -> 206, x 1850 (209 MiB) 235 -> 227; x 1977 (239
-// MiB) 270 -> 277, which keeps the hint.
+// one, as long as the result fits the memory-side cache of 256 MiB, where what reads it next finds it.  q k^T, this and p v, us, with
+// the hint / without, causal and plain: 32 heads x 1500 tokens 144 / 130 and 147 / 130, 24 x 2044 196 / 172 and 207 / 179, 32 x 1004 70 /
+// 67 and 68 / 63, 16 x 1004 43.0 / 42.6 and 42.5 / 38.9, 8 x 516 19.7 / 19.0 and 20.4 / 19.0, 32 x 516 33.5 / 35.1 and 33.7 / 33.9.  By
+// itself, with nothing that reads the result, the launch gets longer where the hint had kept the caches free (plain, 2047 columns, 8 /
+// 32 / 100 / 220 MiB: 6.0 / 7.0, 14.8 / 18.0, 38.1 / 39.5, 80 / 76).  A prompt's attention with rotation of 32 heads x 1850 tokens (209 MiB)
+// 235 / 227, x 1977 (239 MiB) 270 / 277: that keeps the hint.
 constexpr size_t kKeptBytes = (size_t)224 << 20;
 template <typename T, bool CAUSAL, bool RAGGED, int LANES, int CHUNKS>
 __global__ __launch_bounds__(kRowThreads) void softmax_rows_kernel(
