@@ -203,11 +203,17 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_strided_kernel(
 // Rows that are not whole lines are stored without the streaming hint, which sends the parts of a line to memory one by
 // one, as long as the result fits the memory-side cache of 256 MiB, where what reads it next finds it.  q k^T, this and p v, us, with
 // the hint / without, causal and plain: 32 heads x 1500 tokens 144 / 130 and 147 / 130, 24 x 2044 196 / 172 and 207 / 179, 32 x 1004 70 /
-// 67 and 68 / 63, 16 x 1004 43.0 / 42.6 and 42.5 / 38.9, 8 x 516 19.7 / 19.0 and 20.4 / 19.0, 32 x 516 33.5 / 35.1 and 33.7 / 33.9.  By
-// itself, with nothing that reads the result, the launch gets longer where the hint had kept the caches free (plain, 2047 columns, 8 /
-// 32 / 100 / 220 MiB: 6.0 / 7.0, 14.8 / 18.0, 38.1 / 39.5, 80 / 76).  A prompt's attention with rotation of 32 heads x 1850 tokens (209 MiB)
-// 235 / 227, x 1977 (239 MiB) 270 / 277: that keeps the hint.
+// 67 and 68 / 63, 8 x 300 14.8 / 14.0 and 14.6 / 13.8.  By itself, with nothing that reads the result, the launch gets longer where
+// the hint had kept the caches free (plain, 2047 columns, 8 / 32 / 100 / 220 MiB: 6.0 / 7.0, 14.8 / 18.0, 38.1 / 39.5, 80 / 76).  A
+// prompt's attention with rotation of 32 heads x 1850 tokens (209 MiB) 235 / 227, x 1977 (239 MiB) 270 / 277: that keeps the hint.
 constexpr size_t kKeptBytes = (size_t)224 << 20;
+// A result of 7 to 24 MiB in short rows keeps it too: that much waits in the L2s (32 MiB) for the end of the launch to be written
+// back.  The same three without the hint over with it, causal, 420 columns, 6 / 8 / 12 / 16 / 20 / 24 MiB: 0.98 / 1.03 / 1.12 / 1.08 / 1.01 /
+// 0.94; 604 columns 0.97 / 1.02 / 1.08 / 1.09 / 1.04 / 1.02, 804 0.94 / 0.97 / 1.05 / 1.04 / 1.00 / 1.00, 1004 0.91 to 1.00; of narrow rows it
+// ends where there are more than about 28,000: 196 columns (6 / 8 / 10 / 12) 1.03 / 1.07 / 1.02 / 1.00, 340 (8 / 12 / 16 / 20) 1.06 / 1.10 / 1.07 /
+// 0.95, 132 1.00 / 1.01 / 0.96 / 0.97.
+constexpr size_t kFlushedLeast = (size_t)7 << 20, kFlushedMost = (size_t)24 << 20, kFlushedRows = 28000;
+constexpr size_t kFlushedRowLeast = 300, kFlushedRowMost = 1536;   // bytes
 template <typename T, bool CAUSAL, bool RAGGED, int LANES, int CHUNKS>
 __global__ __launch_bounds__(kRowThreads) void softmax_rows_kernel(
     const T* __restrict__ in, T* __restrict__ out, size_t a, size_t b, size_t s, size_t offset, float scale) {
@@ -258,7 +264,10 @@ __global__ __launch_bounds__(kRowThreads) void softmax_rows_kernel(
     }
     sum = group_sum<LANES>(sum, smem);
     const float inv = 1.0f / sum;  // one division per row for 16-bit storage
-    const bool streamed = b * sizeof(T) % 128 == 0 || a * b * sizeof(T) > kKeptBytes;
+    const size_t row_bytes = b * sizeof(T), bytes = a * row_bytes;
+    const bool streamed = row_bytes % 128 == 0 || bytes > kKeptBytes ||
+                          (bytes > kFlushedLeast && bytes <= kFlushedMost && a <= kFlushedRows &&
+                           row_bytes > kFlushedRowLeast && row_bytes < kFlushedRowMost);
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) {
         const int v = c * LANES + lane, at = column(v);

@@ -19,3 +19,10 @@ def test_causal_rows(hip, heads, s, dtype):
         want = torch.softmax(x[h].float() + mask, -1)
         assert ((out[h].float() - want).abs() <= step * want + 2.0 ** -25).all(), h
         assert (out[h].triu(1) == 0).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("heads,s", [(20, 420), (21, 420), (35, 604), (34, 604), (82, 340), (83, 340), (12, 766), (12, 770), (180, 149), (180, 151)])
+def test_results_that_are_flushed(hip, heads, s, dtype):
+    """Both sides of the sizes, numbers of rows and row lengths that keep the hint."""
+    test_causal_rows(hip, heads, s, dtype)
